@@ -43,6 +43,9 @@ struct Geom {
   // Unit bins with two candidates per pixel and |rho0| + N < 2^20, where the fast candidate
   // index (rounding error < 0.4 bin) needs no clamp: the specialised backprojector applies.
   bool bp_two_cand = false;
+  // The fast candidate index is off by less than 0.4 bin (|rho0| + N < 2^20 bins), so it drops no
+  // ray with a nonzero length: the fast A^T and B^T apply.
+  bool index_safe = false;
   // Row-segment width (floats) the staged forward projector needs for 256 consecutive bins.
   int fps_w = 0;
   // Grouped staged forward projector: line groups (int4 entries, fpg_groups in sk_geom.hip),
@@ -60,6 +63,8 @@ struct Geom {
   // sk_geom.hip; null where the hoisted fast path does not apply), one buffer
   unsigned* d_bp_order = nullptr;
   size_t bp_order_off[3] = {0, 0, 0};
+  int* d_degen = nullptr;  // table indices of the LINE_DEGEN lines (null when there are none)
+  int n_degen = 0;
   // SIRT weights, computed on first use (SIRT.fut:22-25)
   float* d_rowinv = nullptr;  // [A][R]
   float* d_colinv = nullptr;  // [N][N]

@@ -331,6 +331,7 @@ int sk_geom_create(sk_ctx* ctx, const float* angles_host, int A, float rho0, flo
   Geom& G = g->g;
   G.A = A; G.R = R; G.N = N; G.rho0 = rho0; G.drho = drho; G.ncand = ncand;
   G.bp_two_cand = drho == 1.0f && ncand == 2 && std::fabs((double)rho0) + N < (double)(1 << 20);
+  G.index_safe = std::fabs((double)rho0) + N < (double)(1 << 20) * drho;
   G.device = c->device;
   G.n_steep = build_lines(angles_host, A, G.lines, N);
   {
@@ -348,6 +349,16 @@ int sk_geom_create(sk_ctx* ctx, const float* angles_host, int A, float rho0, flo
   hipError_t e = hipMalloc(&G.d_lines, sizeof(Line) * (size_t)A);
   if (e == hipSuccess)
     e = hipMemcpy(G.d_lines, G.lines.data(), sizeof(Line) * (size_t)A, hipMemcpyHostToDevice);
+  {
+    std::vector<int> degen;
+    for (int j = 0; j < A; j++)
+      if (G.lines[j].flags & LINE_DEGEN) degen.push_back(j);
+    G.n_degen = (int)degen.size();
+    if (e == hipSuccess && !degen.empty()) {
+      e = hipMalloc(&G.d_degen, sizeof(int) * degen.size());
+      if (e == hipSuccess) e = hipMemcpy(G.d_degen, degen.data(), sizeof(int) * degen.size(), hipMemcpyHostToDevice);
+    }
+  }
   if (e == hipSuccess && (long)A * R < (1L << 31) && A <= 65535) {
     e = hipMalloc(&G.d_inter, sizeof(float) * (size_t)A * R);
     if (e == hipSuccess) {
@@ -380,6 +391,7 @@ int sk_geom_create(sk_ctx* ctx, const float* angles_host, int A, float rho0, flo
   }
   if (e != hipSuccess) {
     if (G.d_lines) (void)hipFree(G.d_lines);
+    if (G.d_degen) (void)hipFree(G.d_degen);
     if (G.d_inter) (void)hipFree(G.d_inter);
     if (G.d_bp_order) (void)hipFree(G.d_bp_order);
     if (G.d_fpg) (void)hipFree(G.d_fpg);
@@ -398,6 +410,7 @@ void sk_geom_destroy(sk_geom* g) {
   for (auto& sg : g->g.sirt_graphs)
     if (sg.exec) (void)hipGraphExecDestroy(sg.exec);
   if (g->g.d_lines) (void)hipFree(g->g.d_lines);
+  if (g->g.d_degen) (void)hipFree(g->g.d_degen);
   if (g->g.d_inter) (void)hipFree(g->g.d_inter);
   if (g->g.d_bp_order) (void)hipFree(g->g.d_bp_order);
   if (g->g.d_fpg) (void)hipFree(g->g.d_fpg);

@@ -484,8 +484,12 @@ __device__ __forceinline__ float binade_step(float slope, int e) {
 template <bool EXACT, int MODE, int WEIGHTS, int NC, bool DR1, int PPT>
 __device__ __forceinline__ void bp_item(const BpParams& P, int tile_x, int tile_y, int bz,
                                         float2* win, BpLineLds* lsh) {
-  // Fast reference weights: slope sign hoisted per line, lbase folded into the staged value.
-  constexpr bool FASTREF = !EXACT && WEIGHTS == W_REF;
+  // Fast mode: slope sign hoisted per line, lbase folded into the staged value.  W_ADJ takes the
+  // same lengths: on a line that is not degenerate, intersect_fact of a candidate is the forward
+  // projector's length of that ray in that pixel (both are the part of the row's x-range inside
+  // the pixel over the range; neither counts a ray that only touches an edge), so only the
+  // degenerate lines, whose rays can lie on pixel edges, are weighed differently.
+  constexpr bool FASTREF = !EXACT;
   // The hoisted fast path keeps each line's window in descending bin order, so that the
   // candidate address comes from floor(-t) (one conversion) instead of ceil(t).
   constexpr bool REV = FASTREF && NC > 0;
@@ -651,7 +655,7 @@ __device__ __forceinline__ void bp_item(const BpParams& P, int tile_x, int tile_
               const float xb = xbase[q] + ev[q][k].x;
               if constexpr (KIND == 2) {
                 // degenerate line: general form with the m == 0 case, lbase already in e.y
-                const float l = cand_len<false, W_REF>(xb, slope, 1.0f, xm[q], x1[q], true);
+                const float l = cand_len<false, WEIGHTS>(xb, slope, 1.0f, xm[q], x1[q], true);
                 acc[q] = fmaf(l, ev[q][k].y, acc[q]);
               } else if (ex[q]) {
                 // min(m/d, 1) = min(m, d)/d with d = dx exact and 1/d in the staged value:
@@ -815,7 +819,7 @@ __device__ __forceinline__ void bp_item(const BpParams& P, int tile_x, int tile_
             for (int k = 0; k < KC; ++k) {
               if (NC == 0 && k >= ncand) break;
               const float l =
-                  cand_len<false, W_REF>(xbase + ev[k].x, L.slope, 1.0f, xmin, xmin1, true);
+                  cand_len<false, WEIGHTS>(xbase + ev[k].x, L.slope, 1.0f, xmin, xmin1, true);
               acc[q] = fmaf(l, ev[k].y, acc[q]);
             }
           } else {
