@@ -155,11 +155,11 @@ __global__ __launch_bounds__(FPS_RAYS, 8) void k_fpg_persist(const BatchArgs a, 
     const int4 grp = B.fp.groups[u32(g)];
     const int cpl = u32(grp.x >> 24);
     if (cpl <= 2)
-      fpg_item<FP_SIRT, 2, 2, false>(B.fp, grp, u32(wb), u32(bz), (float*)seg4);
+      fpg_item<FP_SIRT, 2, 1, false>(B.fp, grp, u32(wb), u32(bz), (float*)seg4);
     else if (cpl == 3)
-      fpg_item<FP_SIRT, 2, 3, false>(B.fp, grp, u32(wb), u32(bz), (float*)seg4);
+      fpg_item<FP_SIRT, 3, 1, false>(B.fp, grp, u32(wb), u32(bz), (float*)seg4);
     else
-      fpg_item<FP_SIRT, 2, 4, false>(B.fp, grp, u32(wb), u32(bz), (float*)seg4);
+      fpg_item<FP_SIRT, 4, 1, false>(B.fp, grp, u32(wb), u32(bz), (float*)seg4);
   }
 }
 
@@ -207,7 +207,7 @@ struct BatchPlan {
   bool dr1 = true;
 };
 
-static size_t fpg_lds(int cpl) { return sizeof(float) * 2 * (FPG_ROWS + 1) * 64 * (size_t)cpl; }
+static size_t fpg_lds(int cpl) { return sizeof(float) * fpg_lds_floats(FpgShape<1>::nbuf, 1, cpl, false); }
 
 // Pixels per lane of the persistent backprojector (16 x 16*PPT tiles): 4 by default (16x64
 // tiles: 3.11 s vs 3.23 s with 16x32 on the four large groups of the batched configuration,

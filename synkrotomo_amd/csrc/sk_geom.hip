@@ -89,8 +89,13 @@ static std::vector<int4> fpg_groups(const std::vector<Line>& lines, int n_steep,
     for (int j = frame ? n_steep : 0; j < (frame ? A : n_steep); ++j)
       if ((lines[j].cost > 0.0f) == pos) idx.push_back(j);
     std::stable_sort(idx.begin(), idx.end(), [&](int a, int b) { return lines[a].slope < lines[b].slope; });
-    for (size_t g0 = 0; g0 < idx.size(); g0 += FPG_LINES) {
-      const int n = (int)std::min<size_t>(FPG_LINES, idx.size() - g0);
+    for (size_t g0 = 0, gn; g0 < idx.size(); g0 += gn) {
+      // up to FPG_LINES lines that agree in sign and LINE_NEWTON (a workgroup's walk has both
+      // resolved at compile time)
+      const int key = lines[idx[g0]].flags & (LINE_SLOPE_POS | LINE_NEWTON);
+      for (gn = 1; gn < FPG_LINES && g0 + gn < idx.size(); ++gn)
+        if ((lines[idx[g0 + gn]].flags & (LINE_SLOPE_POS | LINE_NEWTON)) != key) break;
+      const int n = (int)gn;
       double spread = 0.0, inv = 0.0;
       for (int b = 0; b < nb; ++b) {
         const double r0 = (double)b * FPG_BINS, r1 = r0 + FPG_BINS - 1;

@@ -149,7 +149,7 @@ __device__ __forceinline__ float cand_len(float xbot, float slope, float lbase, 
 // ---------------------------------------------------------------------------- A.x item
 struct FpParams {
   const Line* lines;
-  int A, R, N, ncand;
+  int A, R, N, ncand, batch;
   float rho0, drho;
   const float* img;     // [batch][N][N]
   const float* imgT;    // transposed copy (flat lines)
@@ -158,6 +158,7 @@ struct FpParams {
   const float* rowinv;  // FP_SIRT: [A][R]
   const int4* groups;   // grouped staged variant: the geometry's line groups (else null)
   const float2* steps;  // grouped staged variant: per line, (D_e, 1/D_e) for binades e (else null)
+  int lds_cpl;          // grouped staged variant: chunks per row the workgroup's LDS holds
 };
 
 // Binades e = 0 .. FP_STEP_BINADES-1 of the forward projector's exact per-block step table.
@@ -183,7 +184,7 @@ __device__ __forceinline__ float bcast16(float v) {
 // reciprocal of |xtop - xbot| by one Newton step from rs = 1/|slope| (two FMAs) instead of
 // the quarter-rate v_rcp_f32 (error <= 1.6e-7 relative, see newton_min_slope).
 template <bool POS, bool NT = false>
-__device__ __forceinline__ float fp_row_add(float sum, float xb, float xt, float vb, float vo, float rs = 0.0f) {
+__device__ __forceinline__ float fp_row_frac(float xb, float xt, float rs = 0.0f) {
   const float fx = floorf(xb);
   const float d = POS ? xt - xb : xb - xt;
   const float r = NT ? fmaf(rs, fmaf(-d, rs, 1.0f), rs) : fast_rcp(d);
@@ -193,8 +194,11 @@ __device__ __forceinline__ float fp_row_add(float sum, float xb, float xt, float
   } else {              // (fx - xtop) / (xbot - xtop)
     fo = (fx - xt) * r;
   }
-  fo = fminf(fmaxf(fo, 0.0f), 1.0f);
-  return fmaf(fo, vo - vb, sum + vb);
+  return fminf(fmaxf(fo, 0.0f), 1.0f);
+}
+template <bool POS, bool NT = false>
+__device__ __forceinline__ float fp_row_add(float sum, float xb, float xt, float vb, float vo, float rs = 0.0f) {
+  return fmaf(fp_row_frac<POS, NT>(xb, xt, rs), vo - vb, sum + vb);
 }
 
 // Fast-mode row walk for RPT rays of one line, the slope sign a template argument.  Both
@@ -923,25 +927,49 @@ __device__ __forceinline__ int bcast16i(int v) {
   return __builtin_amdgcn_mov_dpp(v, 0x150 + K, 0xf, 0xf, true);
 }
 
+// S floats of S images side by side in LDS, and one of them.
+template <int S>
+struct Pack {
+  typedef float T __attribute__((ext_vector_type(S)));
+};
+template <>
+struct Pack<1> {
+  typedef float T;
+};
+template <int S>
+__device__ __forceinline__ float pack_at(const typename Pack<S>::T& v, int k) {
+  if constexpr (S == 1)
+    return v;
+  else
+    return v[k];
+}
+
 // The staged walk of one ray per lane over the workgroup's rows i0 .. i1 (uniform) in blocks
 // of ROWS (<= 16, a multiple of 4); the wave computes the blocks that meet its own rows i0w ..
 // i1w.  CPL: staged chunks of 64 columns per row.  seg_start(ib, tab) (uniform): the block's
 // segment start, one column left of floor(xbot) of the lowest ray of the workgroup over the
-// block's rows.  steps: the line's exact step per binade (fp_step_table), or null.
-template <bool POS, int NBUF, bool NT, int CPL, int ROWS, class SegStart>
-__device__ __forceinline__ float fps_walk(const float* src, int N, int h, int i0, int i1,
-                                          int i0w, int i1w, float slope, float icpt,
-                                          SegStart seg_start, float* seg, float rs = 0.0f,
-                                          const float2* __restrict__ steps = nullptr) {
+// block's rows.  block_step(ib, dr) (uniform): whether the wave's block at row ib takes the exact
+// step below, and then each lane's (D_e, 1/D_e).
+// The walk sums the ray over S images at once (src[k]: image k's frame): a row's position, LDS
+// address and fraction do not depend on the image, so they are formed once (7 to 10 VALU) and
+// each image adds a subtract, an add and an FMA.  Per image the operations are those of S = 1.
+template <bool POS, int NBUF, bool NT, int CPL, int ROWS, int PF, int S, class SegStart, class BlockStep>
+__device__ __forceinline__ void fps_walk(const float* const (&src)[S], int N, int h, int i0, int i1,
+                                         int i0w, int i1w, float slope, float icpt,
+                                         SegStart seg_start, BlockStep block_step, float* seg, float (&acc)[S],
+                                         float rs) {
+  using V = typename Pack<S>::T;
+  typedef __attribute__((address_space(3))) V lds_pack;
   const int tid = threadIdx.x;
   const int l16 = tid & 15;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   constexpr int RPW = ROWS / (FPS_RAYS / 64);  // staged rows per wave
-  constexpr int CS = ROWS + 1;                 // LDS stride of a staged column (floats)
-  constexpr int PF = ROWS / 2;                 // rows of LDS reads in flight ahead of the sums
+  constexpr int CS = ROWS + 1;                 // LDS stride of a staged column (packs)
+  constexpr int PB = 4 * S;                    // bytes of a pack
   constexpr int W = 64 * CPL;                  // staged columns
-  float st[RPW][CPL];
+  static_assert(ROWS % PF == 0, "PF: rows of LDS reads in flight ahead of the sums");
+  float st[RPW][CPL][S];
   // Per block, lane l16 holds row ib + l16's i*slope (tab); the block's segment starts at
   // image column sb = seg_start(ib, tab).
   auto block_rows = [&](int ib, float& tab, int& sb) {
@@ -949,42 +977,54 @@ __device__ __forceinline__ float fps_walk(const float* src, int N, int h, int i0
     sb = seg_start(ib, tab);
   };
   // Wave w stages rows RPW*w .. RPW*w + RPW-1 of the block, lane l columns s0 + l + 64m:
-  // coalesced dword loads through the row's descriptor (zero outside the image row and
-  // for rows past i1).
+  // coalesced dword loads through the row's descriptor (zero outside the image row -- an offset
+  // left of it is out of range as an unsigned number -- and for rows past i1, whose descriptor is
+  // empty).  The chunks' offsets are formed once for all rows and images (the empty asm keeps
+  // them whole: folded into the loads' immediates, a negative one would need a branch).
+  const unsigned row_bytes = (unsigned)N * 4u;
   auto load = [&](int ib, int s0) {
+    int o[CPL];
+#pragma unroll
+    for (int m = 0; m < CPL; ++m) {
+      o[m] = (s0 + 64 * m + lane) << 2;
+      asm volatile("" : "+v"(o[m]));
+    }
+    const int ir = ib + RPW * wave;
+    const unsigned r0 = (unsigned)(ir + h) * row_bytes;  // below 2^31: N <= 16384
 #pragma unroll
     for (int t = 0; t < RPW; ++t) {
-      const int i = ib + RPW * wave + t;
-      const __amdgpu_buffer_rsrc_t rr = row_rsrc(src + (size_t)(i < i1 ? i + h : 0) * N, i < i1 ? N : 0);
-      const int vo = (s0 + lane) << 2;
-      if (s0 >= 0) {  // wave-uniform: non-negative offsets, the constant parts as immediates
+#pragma unroll
+      for (int k = 0; k < S; ++k) {
+        const __amdgpu_buffer_rsrc_t rr = row_rsrc(
+            reinterpret_cast<const float*>(reinterpret_cast<const char*>(src[k]) + (r0 + t * row_bytes)),
+            ir + t < i1 ? N : 0);
 #pragma unroll
         for (int m = 0; m < CPL; ++m)
-          st[t][m] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rr, vo + 256 * m, 0, 0));
-      } else {
-        // segment starting left of the image: each load's full offset in its own register
-        // (a negative one is out of range as an unsigned offset and reads 0)
-#pragma unroll
-        for (int m = 0; m < CPL; ++m) {
-          int o = vo + 256 * m;
-          asm volatile("" : "+v"(o));
-          st[t][m] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rr, o, 0, 0));
-        }
+          st[t][m][k] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rr, o[m], 0, 0));
       }
     }
   };
   // LDS layout of a staged block: column-interleaved, column j of row slot r at j*CS + r
   // (CS = ROWS + 1 spreads consecutive columns over the banks), so a lane's pair in row K
   // is one address plus the constant offsets K and K + CS.
+  V* segv = reinterpret_cast<V*>(seg);
   auto store = [&](int buf) {
 #pragma unroll
     for (int t = 0; t < RPW; ++t) {
-      float* base = seg + (size_t)buf * W * CS + lane * CS + RPW * wave + t;
+      V* base = segv + (size_t)buf * W * CS + lane * CS + RPW * wave + t;
 #pragma unroll
-      for (int m = 0; m < CPL; ++m) base[64 * CS * m] = st[t][m];
+      for (int m = 0; m < CPL; ++m) {
+        V v;
+        if constexpr (S == 1)
+          v = st[t][m][0];
+        else
+          for (int k = 0; k < S; ++k) v[k] = st[t][m][k];
+        base[64 * CS * m] = v;
+      }
     }
   };
-  float acc = 0.0f;
+#pragma unroll
+  for (int k = 0; k < S; ++k) acc[k] = 0.0f;
   const int seg_lds = (int)(uintptr_t)(lds_float*)seg;  // LDS address of the block
   // Exact per-block step.  When every x_bot and x_top of the wave's rays over the block's rows
   // lies in one binade [2^e, 2^(e+1)), e >= 0 (tile_binade of the block's column range), all
@@ -992,81 +1032,61 @@ __device__ __forceinline__ float fps_walk(const float* src, int N, int h, int i0
   // |x_top - x_bot| is the line's constant D_e (binade_step; no rounding tie, D_e > 0).  The
   // row then needs no x_top, difference or reciprocal: with fr = fract(x_bot) (exact for
   // |x_bot| >= 1), x_top - floor(x_bot) = fr + D_e and floor(x_bot) - x_top = D_e - fr
-  // exactly, and 1/D_e is fp_row_add's reciprocal of D_e (from the table) -- so each row's
-  // fraction, and the sum, are bit for bit fp_row_add's.  The wave's x_bot extremes over the
-  // block are at its extreme rays and rows (x_bot is monotone in the intercept and the row).
-  // The block's column range from 16.16 fixed-point bounds on the scalar unit: x_bot =
-  // RN(RN(i*slope) + icpt) lies within 3e-3 of i*slope + icpt (|i| <= 4112, |icpt| < 2^14),
-  // the fixed-point products and intercepts within 2^-17*|i| + 2^-16 (< 0.04) of theirs, so
-  // the floors of the fixed-point extremes, widened by one column each way, bound every lane's
-  // and row's floor(x_bot).
-  // Walks with |intercept| >= 2^14 or images over 8192 rows (where the products could leave
-  // 32 bits) take the per-row step.
-  const float ic0 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, icpt), 0));
-  const float ic1 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, icpt), 63));
-  const float ic_lo = fminf(ic0, ic1), ic_hi = fmaxf(ic0, ic1);
-  const bool xok = steps && N <= 8192 && ic_lo > -16384.0f && ic_hi < 16384.0f;
-  const int s_fx = __builtin_amdgcn_readfirstlane(xok ? (int)rintf(slope * 65536.0f) : 0);
-  const int lo_fx = __builtin_amdgcn_readfirstlane(xok ? (int)floorf(ic_lo * 65536.0f) : 0);
-  const int hi_fx = __builtin_amdgcn_readfirstlane(xok ? (int)ceilf(ic_hi * 65536.0f) : 0);
-  auto block_step = [&](int ib, float2& dr) -> bool {
-    if (!xok) return false;
-    const int a = ib * s_fx, z = (ib + ROWS - 1) * s_fx;
-    const int x0 = ((min(a, z) + lo_fx) >> 16) - 1, x1 = ((max(a, z) + hi_fx) >> 16) + 1;
-    const int e = tile_binade(x0, x1);
-    if (e < 0 || e >= FP_STEP_BINADES) return false;
-    dr = steps[e];
-    return dr.x > 0.0f;
-  };
+  // exactly, and 1/D_e is fp_row_frac's reciprocal of D_e (from the table) -- so each row's
+  // fraction, and the sum, are bit for bit the per-row step's.
   // The LDS reads run PF rows ahead of the sums (rolling window of PF row registers).
   // xbs: the row's x_bot (per-row step) or fract(x_bot) (exact step).
-  float xbs[PF], vas[PF], vcs[PF];
+  float xbs[PF];
+  V vas[PF], vcs[PF];
   auto fetch = [&](auto ex, auto kc, float tab, int bbase) {
     constexpr int K = decltype(kc)::value;
-    constexpr int S = K % PF;
+    constexpr int Q = K % PF;
     const float xb = bcast16<K>(tab) + icpt;
-    // LDS byte address of the pair's first column in row slot 0: 4*CS*floor(xbot) + bbase
+    // LDS byte address of the pair's first column in row slot 0: PB*CS*floor(xbot) + bbase
     unsigned off;
     if constexpr (decltype(ex)::value) {
-      xbs[S] = __builtin_amdgcn_fractf(xb);
+      xbs[Q] = __builtin_amdgcn_fractf(xb);
       // floor(xbot) = xbot - fract(xbot) exactly; the address in FP32 is exact (integers
       // below 2^24)
-      off = (unsigned)(int)fmaf(xb - xbs[S], (float)(4 * CS), (float)bbase);
+      off = (unsigned)(int)fmaf(xb - xbs[Q], (float)(PB * CS), (float)bbase);
     } else {
-      xbs[S] = xb;
-      off = (unsigned)(__mul24(floor_to_int(xb), 4 * CS) + bbase);
+      xbs[Q] = xb;
+      off = (unsigned)(__mul24(floor_to_int(xb), PB * CS) + bbase);
     }
-    const lds_float* p = (const lds_float*)(uintptr_t)off;
-    vas[S] = p[K];
-    vcs[S] = p[K + CS];
+    const lds_pack* p = (const lds_pack*)(uintptr_t)off;
+    vas[Q] = p[K];
+    vcs[Q] = p[K + CS];
   };
-  auto sum_row = [&](auto ex, int S, float2 dr) {
+  auto sum_row = [&](auto ex, int q, float2 dr) {
+    float fo;
     if constexpr (decltype(ex)::value) {
-      const float fr = xbs[S], D = dr.x, rD = dr.y;
-      float fo = POS ? fmaf(fr + D, rD, -rD) : (D - fr) * rD;
+      const float fr = xbs[q], D = dr.x, rD = dr.y;
+      fo = POS ? fmaf(fr + D, rD, -rD) : (D - fr) * rD;
       fo = fminf(fmaxf(fo, 0.0f), 1.0f);
-      const float vb = POS ? vas[S] : vcs[S], vo = POS ? vcs[S] : vas[S];
-      acc = fmaf(fo, vo - vb, acc + vb);
     } else {
-      const float xb = xbs[S], xt = xb + slope;
-      acc = POS ? fp_row_add<true, NT>(acc, xb, xt, vas[S], vcs[S], rs)
-                : fp_row_add<false, NT>(acc, xb, xt, vcs[S], vas[S], rs);
+      fo = fp_row_frac<POS, NT>(xbs[q], xbs[q] + slope, rs);
+    }
+#pragma unroll
+    for (int k = 0; k < S; ++k) {
+      const float va = pack_at<S>(vas[q], k), vc = pack_at<S>(vcs[q], k);
+      const float vb = POS ? va : vc, vo = POS ? vc : va;
+      acc[k] = fmaf(fo, vo - vb, acc[k] + vb);
     }
   };
   auto step = [&](auto ex, auto kc, float tab, int bbase, float2 dr) {  // sum row K, fetch K + PF
     constexpr int K = decltype(kc)::value;
-    sum_row(ex, K, dr);
+    sum_row(ex, K % PF, dr);
     fetch(ex, std::integral_constant<int, K + PF>{}, tab, bbase);
     __builtin_amdgcn_sched_barrier(0);
   };
   auto compute = [&](auto ex, int buf, float tab, int sb, float2 dr) {
-    // LDS byte address of the pair's first column in the block's row 0: 4*CS*floor(xbot) + bbase
-    const int bbase = (buf * W * CS + (h - sb - (POS ? 0 : 1)) * CS) * 4 + seg_lds;
+    // LDS byte address of the pair's first column in the block's row 0: PB*CS*floor(xbot) + bbase
+    const int bbase = (buf * W * CS + (h - sb - (POS ? 0 : 1)) * CS) * PB + seg_lds;
     unroll_seq(std::make_integer_sequence<int, PF>{}, [&](auto kc) { fetch(ex, kc, tab, bbase); });
     __builtin_amdgcn_sched_barrier(0);
     unroll_seq(std::make_integer_sequence<int, ROWS - PF>{}, [&](auto kc) { step(ex, kc, tab, bbase, dr); });
 #pragma unroll
-    for (int S = 0; S < PF; ++S) sum_row(ex, S, dr);
+    for (int q = 0; q < PF; ++q) sum_row(ex, q, dr);
   };
   float tab, tabn;
   int sb, sbn;
@@ -1096,7 +1116,6 @@ __device__ __forceinline__ float fps_walk(const float* src, int N, int h, int i0
     tab = tabn;
     sb = sbn;
   }
-  return acc;
 }
 
 // One staged work item: bins blk*FPS_RAYS .. +FPS_RAYS-1 of line j of image bz, one ray per
@@ -1145,21 +1164,26 @@ __device__ __forceinline__ void fps_item(const FpParams& P, int j, int blk, int 
     const int sv = floor_to_int(tab + icpt_lo) + h - 1;
     return min(__builtin_amdgcn_readlane(sv, 0), __builtin_amdgcn_readlane(sv, FPS_ROWS - 1));
   };
-  float acc = 0.0f;
+  auto no_step = [](int, float2&) { return false; };
+  float acc[1] = {0.0f};
   if (i0 < i1) {
     const bool nt = L.flags & LINE_NEWTON;
     const float rs = nt ? 1.0f / fabsf(slope) : 0.0f;
+    auto walk = [&](auto pos, auto newton) {
+      fps_walk<decltype(pos)::value, NBUF, decltype(newton)::value, FPS_CPL, FPS_ROWS, FPS_ROWS / 2, 1>(
+          {src}, N, h, i0, i1, i0w, i1w, slope, icpt, seg_start, no_step, seg, acc, rs);
+    };
     if ((L.flags & LINE_SLOPE_POS) && nt)
-      acc = fps_walk<true, NBUF, true, FPS_CPL, FPS_ROWS>(src, N, h, i0, i1, i0w, i1w, slope, icpt, seg_start, seg, rs);
+      walk(std::true_type{}, std::true_type{});
     else if (L.flags & LINE_SLOPE_POS)
-      acc = fps_walk<true, NBUF, false, FPS_CPL, FPS_ROWS>(src, N, h, i0, i1, i0w, i1w, slope, icpt, seg_start, seg);
+      walk(std::true_type{}, std::false_type{});
     else if (nt)
-      acc = fps_walk<false, NBUF, true, FPS_CPL, FPS_ROWS>(src, N, h, i0, i1, i0w, i1w, slope, icpt, seg_start, seg, rs);
+      walk(std::false_type{}, std::true_type{});
     else
-      acc = fps_walk<false, NBUF, false, FPS_CPL, FPS_ROWS>(src, N, h, i0, i1, i0w, i1w, slope, icpt, seg_start, seg);
+      walk(std::false_type{}, std::false_type{});
   }
   if (r >= P.R) return;  // after the walk: every lane took part in its barriers
-  const float s = acc * L.lbase;
+  const float s = acc[0] * L.lbase;
   const size_t o = (size_t)bz * P.A * P.R + (size_t)L.orig * P.R + r;
   if constexpr (MODE == FP_PLAIN)
     P.out[o] = s;
@@ -1169,16 +1193,23 @@ __device__ __forceinline__ void fps_item(const FpParams& P, int j, int blk, int 
 
 // ------------------------------------------------------- grouped staged forward projection
 // A workgroup = FPG_BINS (64) consecutive bins of up to FPG_LINES (4) lines of one frame that
-// are adjacent in slope (the geometry's group table); wave w walks line w's 64 rays.  The
+// are adjacent in slope and agree in sign and LINE_NEWTON (the geometry's group table).  The
 // rays of such lines at the same bins cross a frame row within a few columns of each other,
 // so a block's staged segment (every column any of the 256 rays touches) is CPL = 2..4 chunks
 // of 64 columns, where 256 bins of one line need 6: the staging per ray-row drops to a third
-// or a half, and blocks of FPG_ROWS = 16 rows fit (fewer per-block steps per row).  The walk
-// and each ray's sums are fps_walk's (bitwise equal results).
+// or a half, and blocks of FPG_ROWS = 16 rows fit (fewer per-block steps per row).
+// A wave holds 16 bins of the four lines, one line per 16-lane row (the row broadcast of
+// i*slope then serves each line its own products): its 64 rays span about 30 columns instead of
+// the 64 to 91 of 64 bins of one line, so lanes seldom read different columns of one LDS bank,
+// adjacent lines' rays often read the same word, more blocks lie in one binade (the exact step)
+// and fewer rows outside the wave's own rays are walked.  Each ray's sum is fps_walk's (bitwise
+// equal results).
 constexpr int FPG_LINES = FPS_RAYS / 64;
 constexpr int FPG_BINS = 64;
+constexpr int FPG_WBINS = FPG_BINS / (FPS_RAYS / 64);  // bins per wave
 constexpr int FPG_MAXCPL = 4;
 constexpr int FPG_ROWS = 16;  // rows per staged block (8.5 KB of LDS per buffer at CPL 2)
+static_assert(FPG_WBINS == 16 && FPG_LINES == 4, "one line per 16-lane row of the wave");
 
 // A group table entry: the lines' table indices (x: first line | CPL << 24; y, z, w: the
 // others, -1 past the group's size).
@@ -1186,47 +1217,66 @@ __device__ __forceinline__ int fpg_line(const int4& g, int k) {
   return k == 0 ? (g.x & 0xffffff) : (k == 1 ? g.y : (k == 2 ? g.z : g.w));
 }
 
-// XSTEP: take the exact per-block step where the table allows (off: the per-row step only).
-template <int MODE, int NBUF, int CPL, bool XSTEP = true>
+// LDS of a grouped item: NBUF blocks of CPL chunks for S images, and with XSTEP the group's
+// exact steps (FPG_LINES x FP_STEP_BINADES).
+__host__ __device__ constexpr size_t fpg_lds_floats(int nbuf, int s, int cpl, bool xstep) {
+  return (size_t)nbuf * (FPG_ROWS + 1) * 64 * cpl * s + (xstep ? 2 * FPG_LINES * FP_STEP_BINADES : 0);
+}
+
+// How the grouped item runs for S images at once.  S = 1: two buffers and one barrier per block
+// (17 KB at CPL 2, 8 workgroups per CU), the exact step.  S = 2, 4: one buffer (17 and 35 KB at
+// CPL 2); the row's arithmetic is shared by the images, so the exact step saves little and its
+// registers are left to the images.  pf: rows of LDS reads in flight (a divisor of FPG_ROWS).
+template <int S>
+struct FpgShape {
+  static constexpr int nbuf = S == 1 ? 2 : 1;
+  static constexpr int pf = S == 4 ? 2 : 4;
+  static constexpr bool xstep = S == 1;
+};
+
+// Images bz*S .. bz*S + S-1 (an image past the last one repeats it and is not written).
+// XSTEP: take the exact per-block step where it applies (off: the per-row step only).
+template <int MODE, int CPL, int S, bool XSTEP = FpgShape<S>::xstep>
 __device__ __forceinline__ void fpg_item(const FpParams& P, const int4 grp, int blk, int bz, float* seg) {
+  constexpr int NBUF = FpgShape<S>::nbuf, ROWS = FPG_ROWS, PF = FpgShape<S>::pf;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int nl = 1 + (grp.y >= 0) + (grp.z >= 0) + (grp.w >= 0);  // lines fill slots 0 .. nl-1
-  const bool active = wave < nl;
+  const int q = lane >> 4;
+  const int jq = fpg_line(grp, q < nl ? q : 0);  // a lane without a line repeats the first one's rays
   const int N = P.N, h = N >> 1;
-  const int first = blk * FPG_BINS, r = first + lane;
-  const int last = min(first + FPG_BINS - 1, P.R - 1);
-  const Line L = P.lines[fpg_line(grp, active ? wave : 0)];
-  const float cost = L.cost, slope = L.slope;
-  const float icpt = (P.rho0 + (float)r * P.drho) / cost;  // forwardprojection.fut:33-34
-  // Lane k < 2*nl describes line k/2 at its first (k even) or last ray: the workgroup's row
-  // hull (valid rays) and the block segment starts (every lane's ray, valid or not: the
-  // intercepts are monotone in the bin, so the extremes are the block's first and last bin).
-  // Lanes past 2*nl repeat lane 0.
-  const int kk = lane < 2 * nl ? lane : 0;
-  const Line Lk = P.lines[fpg_line(grp, kk >> 1)];
+  const int first = blk * FPG_BINS, wfirst = first + FPG_WBINS * wave, r = wfirst + (lane & 15);
+  const Line L = P.lines[jq];
+  const float slope = L.slope;
+  const float icpt = (P.rho0 + (float)r * P.drho) / L.cost;  // forwardprojection.fut:33-34
+  // Lane k < 8 describes line slot k/2 at the workgroup's first (k even) or last ray, lane 8 + k
+  // at the wave's: the row hulls (valid rays).  For the block segment starts (lanes < 8) every
+  // lane's ray counts, valid or not: the intercepts are monotone in the bin, so the extremes
+  // are the block's first and last bin.  Slots past nl repeat slot 0.
+  const int kl = (lane >> 1) & 3;
+  const Line Lk = P.lines[fpg_line(grp, kl < nl ? kl : 0)];
   const float ia = (P.rho0 + (float)first * P.drho) / Lk.cost;
   const float iz = (P.rho0 + (float)(first + FPG_BINS - 1) * P.drho) / Lk.cost;
   const float sl_k = Lk.slope, ilo_k = fminf(ia, iz);
-  const int ro_k = (kk & 1) ? FPG_ROWS - 1 : 0;
-  int i0 = 0, i1 = 0, i0w = 0, i1w = 0;
+  const int ro_k = (lane & 1) ? ROWS - 1 : 0;
+  int i0, i1, i0w, i1w;
   {
+    const int f = lane < 8 ? first : wfirst, n = lane < 8 ? FPG_BINS : FPG_WBINS;
+    const int bin = min((lane & 1) ? f + n - 1 : f, P.R - 1);
     int c0, c1;
-    row_clip(sl_k, (kk & 1) ? (P.rho0 + (float)last * P.drho) / Lk.cost : ia, h, c0, c1);
+    row_clip(sl_k, (P.rho0 + (float)bin * P.drho) / Lk.cost, h, c0, c1);
     i0 = __builtin_amdgcn_readlane(c0, 0);
     i1 = __builtin_amdgcn_readlane(c1, 0);
+    i0w = __builtin_amdgcn_readlane(c0, 8);
+    i1w = __builtin_amdgcn_readlane(c1, 8);
 #pragma unroll
     for (int k = 1; k < 2 * FPG_LINES; ++k) {
       i0 = min(i0, __builtin_amdgcn_readlane(c0, k));
       i1 = max(i1, __builtin_amdgcn_readlane(c1, k));
+      i0w = min(i0w, __builtin_amdgcn_readlane(c0, 8 + k));
+      i1w = max(i1w, __builtin_amdgcn_readlane(c1, 8 + k));
     }
-    // the wave's own rows: its line's lanes (2*wave, 2*wave + 1)
-    if (active) {
-      i0w = min(__builtin_amdgcn_readlane(c0, 2 * wave), __builtin_amdgcn_readlane(c0, 2 * wave + 1));
-      i1w = max(__builtin_amdgcn_readlane(c1, 2 * wave), __builtin_amdgcn_readlane(c1, 2 * wave + 1));
-    } else {
-      i0w = i1w = i0;  // no line: stages its rows, computes nothing
-    }
+    if (wfirst >= P.R) i0w = i1w = i0;  // no valid ray: stages its rows, computes nothing
   }
   // Segment start of the block at row ib: the lowest floor(xbot) - 1 over the group's lines
   // at the block's first and last rows, xbot rounded exactly as the lanes round it.
@@ -1237,30 +1287,80 @@ __device__ __forceinline__ void fpg_item(const FpParams& P, const int4 grp, int 
     for (int k = 1; k < 2 * FPG_LINES; ++k) sb = min(sb, __builtin_amdgcn_readlane(sv, k));
     return sb;
   };
-  const float* src = ((L.flags & LINE_FLAT) ? P.imgT : P.img) + (size_t)bz * N * N;
-  const float2* lsteps =
-      XSTEP && P.steps ? P.steps + (size_t)fpg_line(grp, active ? wave : 0) * FP_STEP_BINADES : nullptr;
-  float acc = 0.0f;
-  if (i0 < i1) {
-    const bool nt = L.flags & LINE_NEWTON;
-    const float rs = nt ? 1.0f / fabsf(slope) : 0.0f;
-    if ((L.flags & LINE_SLOPE_POS) && nt)
-      acc = fps_walk<true, NBUF, true, CPL, FPG_ROWS>(src, N, h, i0, i1, i0w, i1w, slope, icpt, seg_start, seg, rs, lsteps);
-    else if (L.flags & LINE_SLOPE_POS)
-      acc = fps_walk<true, NBUF, false, CPL, FPG_ROWS>(src, N, h, i0, i1, i0w, i1w, slope, icpt, seg_start, seg, 0.0f, lsteps);
-    else if (nt)
-      acc = fps_walk<false, NBUF, true, CPL, FPG_ROWS>(src, N, h, i0, i1, i0w, i1w, slope, icpt, seg_start, seg, rs, lsteps);
-    else
-      acc = fps_walk<false, NBUF, false, CPL, FPG_ROWS>(src, N, h, i0, i1, i0w, i1w, slope, icpt, seg_start, seg, 0.0f, lsteps);
+  // Exact step: the wave's column range over a block from 16.16 fixed-point bounds on the scalar
+  // unit.  x_bot = RN(RN(i*slope) + icpt) lies within 3e-3 of i*slope + icpt (|i| <= 4112,
+  // |icpt| < 2^14), the fixed-point products and intercepts within 2^-17*|i| + 2^-16 (< 0.04) of
+  // theirs, so the extremes over the four lines' slopes and intercepts, widened by one column
+  // each way, bound every lane's and row's floor(x_bot).  Waves with an |intercept| >= 2^14 or
+  // images over 8192 rows (where the products could leave 32 bits) take the per-row step.  The
+  // group's steps sit in LDS; `usable` has bit e where every line has one (D_e > 0).
+  float2* steps = reinterpret_cast<float2*>(seg + fpg_lds_floats(NBUF, S, P.lds_cpl, false));
+  unsigned usable = 0;
+  int s_lo = 0, s_hi = 0, c_lo = 0, c_hi = 0;
+  if constexpr (XSTEP) {
+    const float2 d = P.steps[(size_t)jq * FP_STEP_BINADES + (lane & 15)];
+    if (wave == 0) steps[lane] = d;  // read after the walk's first barrier
+    const unsigned long long b = __ballot(d.x > 0.0f);
+    usable = (unsigned)(b & (b >> 16) & (b >> 32) & (b >> 48)) & 0xffffu;
+    const bool small = icpt > -16384.0f && icpt < 16384.0f;
+    if (N > 8192 || __ballot(!small)) usable = 0;
+    const float ic = small ? icpt : 0.0f;
+    const int sf = (int)rintf(slope * 65536.0f), lo = (int)floorf(ic * 65536.0f), hi = (int)ceilf(ic * 65536.0f);
+    s_lo = s_hi = __builtin_amdgcn_readlane(sf, 0);
+    c_lo = __builtin_amdgcn_readlane(lo, 0);
+    c_hi = __builtin_amdgcn_readlane(hi, 0);
+#pragma unroll
+    for (int k = 0; k < FPG_LINES; ++k) {
+      s_lo = min(s_lo, __builtin_amdgcn_readlane(sf, 16 * k));
+      s_hi = max(s_hi, __builtin_amdgcn_readlane(sf, 16 * k));
+      c_lo = min(c_lo, min(__builtin_amdgcn_readlane(lo, 16 * k), __builtin_amdgcn_readlane(lo, 16 * k + 15)));
+      c_hi = max(c_hi, max(__builtin_amdgcn_readlane(hi, 16 * k), __builtin_amdgcn_readlane(hi, 16 * k + 15)));
+    }
   }
-  if (!active || r >= P.R) return;  // after the walk: every lane took part in its barriers
-  const float s = acc * L.lbase;
-  const size_t o = (size_t)bz * P.A * P.R + (size_t)L.orig * P.R + r;
-  if constexpr (MODE == FP_PLAIN)
-    P.out[o] = s;
-  else
-    P.out[o] = P.rowinv[(size_t)L.orig * P.R + r] * (P.b[o] - s);  // SIRT.fut:33-36
+  auto block_step = [&](int ib, float2& dr) -> bool {
+    if constexpr (!XSTEP) return false;
+    const int a = min(ib * s_lo, ib * s_hi), z = min((ib + ROWS - 1) * s_lo, (ib + ROWS - 1) * s_hi);
+    const int b = max(ib * s_lo, ib * s_hi), y = max((ib + ROWS - 1) * s_lo, (ib + ROWS - 1) * s_hi);
+    const int e = tile_binade(((min(a, z) + c_lo) >> 16) - 1, ((max(b, y) + c_hi) >> 16) + 1);
+    if (e < 0 || !((usable >> e) & 1)) return false;
+    dr = steps[(q << 4) + e];
+    return true;
+  };
+  const int flags = P.lines[grp.x & 0xffffff].flags;  // sign, frame and LINE_NEWTON: the group's
+  const size_t nn = (size_t)N * N;
+  const float* src[S];
+#pragma unroll
+  for (int k = 0; k < S; ++k)
+    src[k] = ((flags & LINE_FLAT) ? P.imgT : P.img) + (size_t)(S == 1 ? bz : min(bz * S + k, P.batch - 1)) * nn;
+  float acc[S] = {};
+  if (i0 < i1) {
+    const bool nt = flags & LINE_NEWTON;
+    const float rs = nt ? 1.0f / fabsf(slope) : 0.0f;
+    auto walk = [&](auto pos, auto newton) {
+      fps_walk<decltype(pos)::value, NBUF, decltype(newton)::value, CPL, ROWS, PF, S>(
+          src, N, h, i0, i1, i0w, i1w, slope, icpt, seg_start, block_step, seg, acc, rs);
+    };
+    if ((flags & LINE_SLOPE_POS) && nt)
+      walk(std::true_type{}, std::true_type{});
+    else if (flags & LINE_SLOPE_POS)
+      walk(std::true_type{}, std::false_type{});
+    else if (nt)
+      walk(std::false_type{}, std::true_type{});
+    else
+      walk(std::false_type{}, std::false_type{});
+  }
+  if (q >= nl || r >= P.R) return;  // after the walk: every lane took part in its barriers
+  const size_t in_img = (size_t)L.orig * P.R + r;
+#pragma unroll
+  for (int k = 0; k < S; ++k) {
+    if (S > 1 && bz * S + k >= P.batch) break;
+    const float s = acc[k] * L.lbase;
+    const size_t o = (size_t)(bz * S + k) * P.A * P.R + in_img;
+    if constexpr (MODE == FP_PLAIN)
+      P.out[o] = s;
+    else
+      P.out[o] = P.rowinv[in_img] * (P.b[o] - s);  // SIRT.fut:33-36
+  }
 }
-
 
 }  // namespace sk

@@ -16,9 +16,9 @@
 //               coalesced dword loads into LDS, then every lane forms its ray's row steps
 //               from LDS.  Same per-step expressions as k_fp (bitwise equal results).
 //   k_fp_grouped A.x, grouped staged (variant 7): a workgroup = 64 consecutive bins of four
-//               lines adjacent in slope, one wave per line, so the staged segment of a
-//               block is two to four chunks of 64 columns instead of six; blocks of 16
-//               rows.  Same walk.  k_fp_grouped_res: its SIRT-residual instance.
+//               lines adjacent in slope, 16 bins of each line per wave, so the staged segment
+//               of a block is two to four chunks of 64 columns instead of six; blocks of 16
+//               rows.  Same walk, for 1, 2 or 4 images at once.
 //   k_bp  B.r   (futhark/backprojection.fut:20-93).  Pixel-parallel gather, no atomics: a
 //               block owns a 16 x 16*PPT pixel tile and walks the lines in order, staging
 //               for each block of 32 lines the tile's rho-window of the sinogram in LDS
@@ -95,32 +95,27 @@ __global__ __launch_bounds__(FPS_RAYS) void k_fp_staged(FpParams P) {
 
 // Grouped staged A.x (variant 7): grid (line groups, bin blocks of FPG_BINS, images).
 // Dynamic LDS: NBUF * (FPG_ROWS + 1) * 64 * (the geometry's largest CPL) floats.
-template <int MODE, int NBUF>
-__device__ __forceinline__ void fpg_block(const FpParams& P) {
+// Grouped staged A.x (variant 7) of S images at once: grid (line groups, bin blocks of FPG_BINS,
+// images / S).  CPLMAX: the largest chunk count of the geometry's groups.  Dynamic LDS:
+// fpg_lds_floats.
+// One image: VALU issue bounds it (13 per row and ray off the exact step, 10 on it, and 45 per
+// block and wave of staging and block bounds; 1.3 per CU-clock).  More images share a row's
+// position, address and fraction, so each adds 3 VALU and its 8 bytes of LDS reads per row and
+// ray; at S = 4 the LDS is busy 65% of the time.  64 images of 512^2, 512 angles: 3.01 ms
+// one image at a time, 2.24 ms for S = 2, 1.75 ms for S = 4.
+constexpr int fpg_waves_per_simd(int s, int cpl) { return s == 1 ? 8 : (s == 4 ? 4 : (cpl == 2 ? 8 : (cpl == 3 ? 6 : 5))); }
+
+template <int MODE, int S, int CPLMAX>
+__global__ __launch_bounds__(FPS_RAYS, fpg_waves_per_simd(S, CPLMAX)) void k_fp_grouped(FpParams P) {
   extern __shared__ float4 seg4[];
   const int4 grp = P.groups[blockIdx.x];
   const int cpl = grp.x >> 24;  // uniform
-  if (cpl <= 2)
-    fpg_item<MODE, NBUF, 2>(P, grp, blockIdx.y, blockIdx.z, (float*)seg4);
-  else if (cpl == 3)
-    fpg_item<MODE, NBUF, 3>(P, grp, blockIdx.y, blockIdx.z, (float*)seg4);
+  if (CPLMAX == 2 || cpl <= 2)
+    fpg_item<MODE, 2, S>(P, grp, blockIdx.y, blockIdx.z, (float*)seg4);
+  else if (CPLMAX == 3 || cpl == 3)
+    fpg_item<MODE, CPLMAX >= 3 ? 3 : 2, S>(P, grp, blockIdx.y, blockIdx.z, (float*)seg4);
   else
-    fpg_item<MODE, NBUF, 4>(P, grp, blockIdx.y, blockIdx.z, (float*)seg4);
-}
-
-template <int MODE, int NBUF>
-__global__ __launch_bounds__(FPS_RAYS, 8) void k_fp_grouped(FpParams P) {
-  fpg_block<MODE, NBUF>(P);
-}
-
-// The same for the SIRT residual (FP_SIRT), whose epilogue keeps two more pointers across the
-// walk: under the 8-workgroups-per-CU bound's scalar-register budget (about 80) they spilled
-// 14 scalar registers into a vector register's lanes and one vector register to scratch,
-// reloaded once per row block.  64 vector registers (still 8 waves per SIMD) without that
-// bound's scalar limit: 84 scalar registers, no spill.
-template <int NBUF>
-__global__ __launch_bounds__(FPS_RAYS) __attribute__((amdgpu_num_vgpr(64))) void k_fp_grouped_res(FpParams P) {
-  fpg_block<FP_SIRT, NBUF>(P);
+    fpg_item<MODE, CPLMAX >= 4 ? 4 : 2, S>(P, grp, blockIdx.y, blockIdx.z, (float*)seg4);
 }
 
 // Grid: (tiles across, tiles down, images).  Dynamic LDS: BP_LB * W float2.
@@ -151,8 +146,8 @@ int launch_transpose(Ctx* c, const float* in, float* out, int N, int batch, hipS
 }
 
 FpParams fp_params(const Geom* g, const FpArgs& a) {
-  return FpParams{g->d_lines, g->A, g->R, g->N, g->ncand, g->rho0, g->drho,
-                  a.img, a.imgT, a.out, a.b, a.rowinv, g->d_fpg, g->d_fp_steps};
+  return FpParams{g->d_lines, g->A, g->R, g->N, g->ncand, a.batch, g->rho0, g->drho,
+                  a.img, a.imgT, a.out, a.b, a.rowinv, g->d_fpg, g->d_fp_steps, g->fpg_cpl};
 }
 
 // fp variants: 0/1/2 = 1/2/4 rays per lane, bin blocks fastest; 3/4 = 1/2 rays per lane,
@@ -195,16 +190,39 @@ static void fp_go_staged(const Geom* g, const FpArgs& a, hipStream_t s) {
                      fp_params(g, a));
 }
 
-template <int MODE, int NBUF>
-static void fp_go_grouped(const Geom* g, const FpArgs& a, hipStream_t s) {
+template <int MODE, int S>
+static void fp_go_grouped_s(const Geom* g, const FpArgs& a, hipStream_t s) {
   const unsigned nb = (unsigned)((g->R + FPG_BINS - 1) / FPG_BINS);
-  const size_t lds = sizeof(float) * NBUF * (FPG_ROWS + 1) * 64 * (size_t)g->fpg_cpl;
-  if constexpr (MODE == FP_SIRT)
-    hipLaunchKernelGGL((k_fp_grouped_res<NBUF>), dim3(g->n_fpg, nb, a.batch), dim3(FPS_RAYS), lds, s,
-                       fp_params(g, a));
+  const size_t lds = sizeof(float) * fpg_lds_floats(FpgShape<S>::nbuf, S, g->fpg_cpl, FpgShape<S>::xstep);
+  const dim3 grid(g->n_fpg, nb, (a.batch + S - 1) / S);
+  const FpParams P = fp_params(g, a);
+  if (g->fpg_cpl == 2)
+    hipLaunchKernelGGL((k_fp_grouped<MODE, S, 2>), grid, dim3(FPS_RAYS), lds, s, P);
+  else if (g->fpg_cpl == 3)
+    hipLaunchKernelGGL((k_fp_grouped<MODE, S, 3>), grid, dim3(FPS_RAYS), lds, s, P);
   else
-    hipLaunchKernelGGL((k_fp_grouped<MODE, NBUF>), dim3(g->n_fpg, nb, a.batch), dim3(FPS_RAYS), lds, s,
-                       fp_params(g, a));
+    hipLaunchKernelGGL((k_fp_grouped<MODE, S, 4>), grid, dim3(FPS_RAYS), lds, s, P);
+}
+
+// Images per workgroup: 4 (from three images on: a fourth that repeats costs less than a second
+// pass) or 2 where that leaves at least two workgroups per CU, else 1.  Below that the chip is
+// not full and more images per workgroup only lengthen it: 256^2, 179 angles (270 workgroups an
+// image), 4 images: 36.0, 30.3 and 32.3 us for 1, 2 and 4; 8 images: 62.6, 45.2, 40.8; 128^2, 89
+// angles (69), 2 images: 13.3, 13.8; 512^2, 358 angles (1080), 3 images: 127.5, 126.1, 110.0.
+int fpg_images(const Geom* g, int batch) {
+  const long per = (long)g->n_fpg * ((g->R + FPG_BINS - 1) / FPG_BINS);
+  if (batch >= 3 && per * ((batch + 3) / 4) >= 512) return 4;
+  if (batch >= 2 && per * ((batch + 1) / 2) >= 512) return 2;
+  return 1;
+}
+
+template <int MODE>
+static void fp_go_grouped(const Geom* g, const FpArgs& a, hipStream_t s) {
+  switch (fpg_images(g, a.batch)) {
+    case 4: fp_go_grouped_s<MODE, 4>(g, a, s); break;
+    case 2: fp_go_grouped_s<MODE, 2>(g, a, s); break;
+    default: fp_go_grouped_s<MODE, 1>(g, a, s);
+  }
 }
 
 int launch_fp(Ctx* c, const Geom* g, FpMode mode, const FpArgs& a, hipStream_t s) {
@@ -212,11 +230,10 @@ int launch_fp(Ctx* c, const Geom* g, FpMode mode, const FpArgs& a, hipStream_t s
   int v = g->fp_variant >= 0 ? g->fp_variant : c->fp_variant;
   if (v == 7) {
     if (!ex && g->d_fpg && mode != FP_ONES_INV) {
-      // two buffers, one barrier per block (17 KB of LDS at CPL 2: 8 workgroups per CU)
       if (mode == FP_PLAIN)
-        fp_go_grouped<FP_PLAIN, 2>(g, a, s);
+        fp_go_grouped<FP_PLAIN>(g, a, s);
       else
-        fp_go_grouped<FP_SIRT, 2>(g, a, s);
+        fp_go_grouped<FP_SIRT>(g, a, s);
       return launched(c, "forward projection kernel");
     }
     v = 6;  // no group table for this geometry: the one-line staged kernel

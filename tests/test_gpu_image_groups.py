@@ -1,0 +1,59 @@
+"""Kernels that work on several images at once (A.x 4 or 2 images per workgroup) give each image
+the bits it gets alone: batches around the group sizes, every staged width (chunks of 64
+columns: bin widths 1, 1.3 and 2), groups of fewer than four lines and a ragged last bin block.
+The images hold both signs and, in one case, values far apart."""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+# name, N, angles, bins, first angle, bin width; enough workgroups that batches run grouped
+GEOMETRIES = [
+    ("two_chunks", 64, 701, 93, 0.0, 1.0),
+    ("three_chunks", 96, 803, 130, 0.01, 1.3),
+    ("four_chunks", 128, 901, 130, 0.4, 2.0),
+]
+
+
+def _geometry(ctx, N, A, R, start, drho):
+    ang = (start + np.arange(A) * math.pi / A).astype(np.float32)
+    return ctx.geometry(ang, -(R - 1) / 2 * drho + 0.3, drho, R, N)
+
+
+@pytest.mark.parametrize("name,N,A,R,start,drho", GEOMETRIES, ids=[g[0] for g in GEOMETRIES])
+@pytest.mark.parametrize("batch", [2, 3, 5, 8])
+def test_projection_of_a_batch_is_each_images_own(ctx, name, N, A, R, start, drho, batch):
+    geo = _geometry(ctx, N, A, R, start, drho)
+    gen = torch.Generator(device="cuda").manual_seed(batch)
+    x = torch.randn(batch, N, N, device="cuda", generator=gen)
+    x[-1] *= 1e6
+    geo.set_variants(7, 2)
+    try:
+        got = geo.fp(x)
+        geo.set_variants(0, 2)  # one ray per lane, one image per launch block
+        for k in range(batch):
+            assert torch.equal(got[k], geo.fp(x[k].contiguous())), k
+    finally:
+        geo.set_variants(-1, -1)
+
+
+@pytest.mark.parametrize("batch", [2, 3, 6])
+def test_sirt_of_a_batch_is_each_slices_own(ctx, batch):
+    name, N, A, R, start, drho = GEOMETRIES[0]
+    geo = _geometry(ctx, N, A, R, start, drho)
+    gen = torch.Generator(device="cuda").manual_seed(7)
+    b = torch.rand(batch, A, R, device="cuda", generator=gen)
+    x = torch.zeros(batch, N, N, device="cuda")
+    geo.set_variants(7, 2)
+    try:
+        geo.sirt_(x, b, 3)
+        geo.set_variants(0, 0)
+        for k in range(batch):
+            one = torch.zeros(N, N, device="cuda")
+            geo.sirt_(one, b[k].contiguous(), 3)
+            assert torch.equal(x[k], one), k
+    finally:
+        geo.set_variants(-1, -1)
