@@ -146,6 +146,23 @@ __device__ __forceinline__ float cand_len(float xbot, float slope, float lbase, 
   }
 }
 
+// S floats of S images side by side in LDS, and one of them.
+template <int S>
+struct Pack {
+  typedef float T __attribute__((ext_vector_type(S)));
+};
+template <>
+struct Pack<1> {
+  typedef float T;
+};
+template <int S>
+__device__ __forceinline__ float pack_at(const typename Pack<S>::T& v, int k) {
+  if constexpr (S == 1)
+    return v;
+  else
+    return v[k];
+}
+
 // ---------------------------------------------------------------------------- A.x item
 struct FpParams {
   const Line* lines;
@@ -384,7 +401,7 @@ __device__ __forceinline__ void fp_item(const FpParams& P, int j, int wb, int bz
 // ---------------------------------------------------------------------------- B.r item
 struct BpParams {
   const Line* lines;
-  int A, R, N, ncand, W;
+  int A, R, N, ncand, W, batch;
   int nsteep;           // lines [0, nsteep) are steep, the rest flat
   float rho0, drho;
   const float* sino;    // [batch][A][R]
@@ -485,9 +502,19 @@ __device__ __forceinline__ float binade_step(float slope, int e) {
 // reference's up to the reciprocal) but computes the candidate index with fewer roundings:
 // a pixel whose rounded index moves by one bin gains or loses only a bin at distance
 // >= sqrt(2)/2 from its centre, where the intersection length is zero.
-template <bool EXACT, int MODE, int WEIGHTS, int NC, bool DR1, int PPT>
+//
+// S > 1 (the hoisted fast path): images bz*S .. bz*S + S-1 at once (an image past the last one
+// repeats it and is not written).  A candidate's index, LDS position and length do not depend on
+// the image: each image adds one FMA per candidate.  The window then holds the intercepts
+// (BP_LB*W floats) and after them the S images' values side by side (BP_LB*W packs); per image
+// the operations are those of S = 1.
+template <bool EXACT, int MODE, int WEIGHTS, int NC, bool DR1, int PPT, int S = 1>
 __device__ __forceinline__ void bp_item(const BpParams& P, int tile_x, int tile_y, int bz,
                                         float2* win, BpLineLds* lsh) {
+  using V = typename Pack<S>::T;
+  static_assert(S == 1 || (!EXACT && NC > 0), "several images: the hoisted fast path");
+  constexpr int LB = BP_LB;  // the same for every kernel: a block's tie lines are summed at its end
+  static_assert(LB <= 64, "one lane per line of a block");
   // Fast mode: slope sign hoisted per line, lbase folded into the staged value.  W_ADJ takes the
   // same lengths: on a line that is not degenerate, intersect_fact of a candidate is the forward
   // projector's length of that ray in that pixel (both are the part of the row's x-range inside
@@ -503,15 +530,21 @@ __device__ __forceinline__ void bp_item(const BpParams& P, int tile_x, int tile_
   constexpr int TH = 16 * PPT;
   const int X0 = tile_x * BP_TW, Y0 = tile_y * TH;
   const int N = P.N, h = N >> 1;
-  const float* sb = P.sino + (size_t)bz * P.A * P.R;
+  const int img0 = bz * S;
+  const float* sb[S];
+#pragma unroll
+  for (int m = 0; m < S; ++m)
+    sb[m] = P.sino + (size_t)(S == 1 ? bz : min(img0 + m, P.batch - 1)) * P.A * P.R;
+  float* win_x = reinterpret_cast<float*>(win);                  // S > 1: intercepts
+  V* win_v = reinterpret_cast<V*>(win_x + LB * W);               // S > 1: values (LB*W*4 is a multiple of 16)
   const int X = X0 + tx;
-  float xs[PPT], ys[PPT], acc_s[PPT], acc_f[PPT];
+  float xs[PPT], ys[PPT], acc_s[PPT][S], acc_f[PPT][S];
 #pragma unroll
   for (int k = 0; k < PPT; ++k) {
     xs[k] = (float)(X - h);
     ys[k] = (float)(Y0 + ty + 16 * k - h);
-    acc_s[k] = 0.0f;
-    acc_f[k] = 0.0f;
+#pragma unroll
+    for (int m = 0; m < S; ++m) acc_s[k][m] = acc_f[k][m] = 0.0f;
   }
 
   // hoisted fast path: the tile's binade for steep lines (frame x = image column; -1 where
@@ -526,8 +559,8 @@ __device__ __forceinline__ void bp_item(const BpParams& P, int tile_x, int tile_
   const int fslots = (fband >> ((Y0 - Y64) >> 4)) & ((1 << PPT) - 1);
   const int ebin[2] = {REV ? tile_binade(X0 - h, X0 - h + BP_TW - 1) : -1, eflat};
 
-  for (int l0 = 0; l0 < P.A; l0 += BP_LB) {
-    const int nl = min(BP_LB, P.A - l0);
+  for (int l0 = 0; l0 < P.A; l0 += LB) {
+    const int nl = min(LB, P.A - l0);
     if ((int)threadIdx.x < nl) {
       const Line L = P.lines[l0 + threadIdx.x];
       const bool fl = L.flags & LINE_FLAT;
@@ -579,15 +612,27 @@ __device__ __forceinline__ void bp_item(const BpParams& P, int tile_x, int tile_
           inter = P.inter[(l0 + jj) * P.R + sp];
         else
           inter = ((float)sp * P.drho + P.rho0) / lsh[jj].cost;
-        float p;
-        if constexpr (MODE == BP_ONES_INV) {
-          p = in ? 1.0f : 0.0f;
-        } else {
-          const float v = sb[(size_t)lsh[jj].orig * P.R + (in ? sp : 0)];  // in bounds either way
-          p = in ? v : 0.0f;
+        float p[S];
+#pragma unroll
+        for (int m = 0; m < S; ++m) {
+          if constexpr (MODE == BP_ONES_INV) {
+            p[m] = in ? 1.0f : 0.0f;
+          } else {
+            const float v = sb[m][(size_t)lsh[jj].orig * P.R + (in ? sp : 0)];  // in bounds either way
+            p[m] = in ? v : 0.0f;
+          }
+          if constexpr (FASTREF) p[m] = p[m] * lsh[jj].wscale;
         }
-        if constexpr (FASTREF) p = p * lsh[jj].wscale;
-        win[jj * W + (REV ? W - 1 - k : k)] = make_float2(inter, p);
+        const int at = jj * W + (REV ? W - 1 - k : k);
+        if constexpr (S == 1) {
+          win[at] = make_float2(inter, p[0]);
+        } else {
+          win_x[at] = inter;
+          V v;
+#pragma unroll
+          for (int m = 0; m < S; ++m) v[m] = p[m];
+          win_v[at] = v;
+        }
       }
     }
     __syncthreads();
@@ -598,7 +643,7 @@ __device__ __forceinline__ void bp_item(const BpParams& P, int tile_x, int tile_
     for (int part = 0; part < 2; ++part) {
       const int j_begin = part == 0 ? 0 : nsteep, j_end = part == 0 ? nsteep : nl;
       if (j_begin >= j_end) continue;
-      float xm[PPT], ym[PPT], xh[PPT], yh[PPT], x1[PPT], acc[PPT];
+      float xm[PPT], ym[PPT], xh[PPT], yh[PPT], x1[PPT], acc[PPT][S];
 #pragma unroll
       for (int q = 0; q < PPT; ++q) {
         xm[q] = part ? ys[q] : xs[q];
@@ -606,7 +651,8 @@ __device__ __forceinline__ void bp_item(const BpParams& P, int tile_x, int tile_
         xh[q] = xm[q] + 0.5f;
         yh[q] = ym[q] + 0.5f;
         x1[q] = xm[q] + 1.0f;
-        acc[q] = part ? acc_f[q] : acc_s[q];
+#pragma unroll
+        for (int m = 0; m < S; ++m) acc[q][m] = part ? acc_f[q][m] : acc_s[q][m];
       }
       if constexpr (REV) {
         // The table keeps the lines of each part in angle order, so the lines of one slope
@@ -630,8 +676,9 @@ __device__ __forceinline__ void bp_item(const BpParams& P, int tile_x, int tile_
           // candidates: the LDS reads of all pixels are in flight together.  Bin s sits at
           // window position W-1-(s-w0); wrev[-s] is the entry of the last candidate of the
           // pixel whose first candidate is s (w0 is uniform: scalar base arithmetic).
-          const float2* wrev = win + __builtin_amdgcn_readfirstlane(jj * W + W - NC + lc.w0);
-          float2 ev[PPT][NC];
+          const int rev0 = __builtin_amdgcn_readfirstlane(jj * W + W - NC + lc.w0);
+          float ei[PPT][NC];  // the candidates' intercepts
+          V ev[PPT][NC];      // and values
           float xbase[PPT], edge[PPT];
           bool ex[PPT];  // the slot takes the exact step (constant once the loops unroll)
 #pragma unroll
@@ -640,14 +687,23 @@ __device__ __forceinline__ void bp_item(const BpParams& P, int tile_x, int tile_
             // t is within 0.4 bin of the reference's index (|rho0| + N < 2^20 for this
             // path), so its ceiling lies in [w0, w0 + W - NC]: no clamp.
             const float t = part == 0 ? fmaf(lc.si, yh[q], tb) : fmaf(lc.ci, xh[q], tb);
-            const float2* wrow = wrev + neg_ceil_to_int(t);
+            const int at = neg_ceil_to_int(t);
             xbase[q] = ym[q] * slope;  // backprojection.fut:55
             // x_top - xmin = x_bot - (xmin - d), resp. xmin + 1 - x_top = (xmin + 1 + d) -
             // x_bot, exactly: x_bot, x_top and the moved edge are multiples of u in the
             // tile's binade
             if (ex[q]) edge[q] = POS ? xm[q] - lc.dx : x1[q] + lc.dx;
 #pragma unroll
-            for (int k = 0; k < NC; ++k) ev[q][k] = wrow[NC - 1 - k];
+            for (int k = 0; k < NC; ++k) {
+              if constexpr (S == 1) {
+                const float2 e = (win + rev0 + at)[NC - 1 - k];
+                ei[q][k] = e.x;
+                ev[q][k] = e.y;
+              } else {
+                ei[q][k] = (win_x + rev0 + at)[NC - 1 - k];
+                ev[q][k] = (win_v + rev0 + at)[NC - 1 - k];
+              }
+            }
           }
           // Non-degenerate lines: max(min(a, b), 0) == med3(a, b, 0): a and b cannot both
           // be negative when the ray's x-range has positive length; m/diff is then >= 0,
@@ -656,38 +712,37 @@ __device__ __forceinline__ void bp_item(const BpParams& P, int tile_x, int tile_
           for (int q = 0; q < PPT; ++q)
 #pragma unroll
             for (int k = 0; k < NC; ++k) {
-              const float xb = xbase[q] + ev[q][k].x;
+              const float xb = xbase[q] + ei[q][k];
+              float g;  // the candidate's weight of its staged value
               if constexpr (KIND == 2) {
                 // degenerate line: general form with the m == 0 case, lbase already in e.y
-                const float l = cand_len<false, WEIGHTS>(xb, slope, 1.0f, xm[q], x1[q], true);
-                acc[q] = fmaf(l, ev[q][k].y, acc[q]);
+                g = cand_len<false, WEIGHTS>(xb, slope, 1.0f, xm[q], x1[q], true);
               } else if (ex[q]) {
                 // min(m/d, 1) = min(m, d)/d with d = dx exact and 1/d in the staged value:
                 // max(min(a, b, d), 0) is one v_min3 with the output clamp (d <= 1).  A line
                 // whose step is a rounding tie has dx = 0 and adds 0 here (tie pass below).
                 const float a = POS ? xb - edge[q] : xb - xm[q];
                 const float b = POS ? x1[q] - xb : edge[q] - xb;
-                const float g = __builtin_amdgcn_fmed3f(fminf(fminf(a, b), lc.dx), 0.0f, 1.0f);
-                acc[q] = fmaf(g, ev[q][k].y, acc[q]);
+                g = __builtin_amdgcn_fmed3f(fminf(fminf(a, b), lc.dx), 0.0f, 1.0f);
               } else {
                 const float xt = xb + slope;
                 const float d = POS ? xt - xb : xb - xt;
                 const float m = POS ? __builtin_amdgcn_fmed3f(xt - xm[q], x1[q] - xb, 0.0f)
                                     : __builtin_amdgcn_fmed3f(xb - xm[q], x1[q] - xt, 0.0f);
-                float f;
                 if constexpr (KIND == 3 || KIND == 4) {
                   // 1/d by one Newton step from 1/|slope| (d = |x_top - x_bot| is |slope| to
                   // within the rounding of x_bot): two full-rate FMAs for the quarter-rate
                   // v_rcp_f32
                   const float r = fmaf(lc.rs, fmaf(-d, lc.rs, 1.0f), lc.rs);
-                  f = fminf(fmaxf(m * r, 0.0f), 1.0f);
+                  g = fminf(fmaxf(m * r, 0.0f), 1.0f);
                 } else {
-                  f = fminf(fmaxf(m * fast_rcp(d), 0.0f), 1.0f);
+                  g = fminf(fmaxf(m * fast_rcp(d), 0.0f), 1.0f);
                 }
                 // a tie line (dx = 0) adds 0 here as well
-                if constexpr (SLOTS >= 0) f = f * lc.dx;
-                acc[q] = fmaf(f, ev[q][k].y, acc[q]);
+                if constexpr (SLOTS >= 0) g = g * lc.dx;
               }
+#pragma unroll
+              for (int m = 0; m < S; ++m) acc[q][m] = fmaf(g, pack_at<S>(ev[q][k], m), acc[q][m]);
             }
         };
         auto run = [&](auto kind, auto slots, int jb, int je) {
@@ -746,7 +801,7 @@ __device__ __forceinline__ void bp_item(const BpParams& P, int tile_x, int tile_
           // tie pass: the part's lines whose step depends on x_bot's last bit, with the
           // hardware reciprocal (their staged values carry lbase only)
           const int lane = threadIdx.x & 63;
-          const bool tie = lane >= j_begin && lane < j_end && lsh[lane < BP_LB ? lane : 0].tie;
+          const bool tie = lane >= j_begin && lane < j_end && lsh[lane < LB ? lane : 0].tie;
           unsigned long long tm = __ballot(tie);
           while (tm) {  // uniform
             const int jj = __builtin_ctzll(tm);
@@ -804,7 +859,7 @@ __device__ __forceinline__ void bp_item(const BpParams& P, int tile_x, int tile_
                 const float xt = xb + L.slope;
                 const float m = __builtin_amdgcn_fmed3f(xt - xmin, xmin1 - xb, 0.0f);
                 const float f = fminf(fmaxf(m * fast_rcp(xt - xb), 0.0f), 1.0f);
-                acc[q] = fmaf(f, ev[k].y, acc[q]);
+                acc[q][0] = fmaf(f, ev[k].y, acc[q][0]);
               }
             } else {
 #pragma unroll
@@ -814,7 +869,7 @@ __device__ __forceinline__ void bp_item(const BpParams& P, int tile_x, int tile_
                 const float xt = xb + L.slope;
                 const float m = __builtin_amdgcn_fmed3f(xb - xmin, xmin1 - xt, 0.0f);
                 const float f = fminf(fmaxf(m * fast_rcp(xb - xt), 0.0f), 1.0f);
-                acc[q] = fmaf(f, ev[k].y, acc[q]);
+                acc[q][0] = fmaf(f, ev[k].y, acc[q][0]);
               }
             }
           } else if (FASTREF) {
@@ -824,7 +879,7 @@ __device__ __forceinline__ void bp_item(const BpParams& P, int tile_x, int tile_
               if (NC == 0 && k >= ncand) break;
               const float l =
                   cand_len<false, WEIGHTS>(xbase + ev[k].x, L.slope, 1.0f, xmin, xmin1, true);
-              acc[q] = fmaf(l, ev[k].y, acc[q]);
+              acc[q][0] = fmaf(l, ev[k].y, acc[q][0]);
             }
           } else {
             // reference order: the line's candidates summed, then added to the pixel
@@ -837,16 +892,19 @@ __device__ __forceinline__ void bp_item(const BpParams& P, int tile_x, int tile_
                   cand_len<EXACT, WEIGHTS>(xbase + e.x, L.slope, L.lbase, xmin, xmin1, degen);
               inner = inner + l * e.y;
             }
-            acc[q] = acc[q] + inner;
+            acc[q][0] = acc[q][0] + inner;
           }
         }
       }
 #pragma unroll
       for (int q = 0; q < PPT; ++q) {
-        if (part)
-          acc_f[q] = acc[q];
-        else
-          acc_s[q] = acc[q];
+#pragma unroll
+        for (int m = 0; m < S; ++m) {
+          if (part)
+            acc_f[q][m] = acc[q][m];
+          else
+            acc_s[q][m] = acc[q][m];
+        }
       }
     }
     __syncthreads();
@@ -858,30 +916,36 @@ __device__ __forceinline__ void bp_item(const BpParams& P, int tile_x, int tile_
     // scatter with stride N.
     constexpr int TS = 17;  // LDS row stride of the staged tile (floats)
     float* st = reinterpret_cast<float*>(win);
-    const bool staged = 2 * BP_LB * W >= TH * TS;  // uniform
+    const bool staged = (1 + S) * LB * W >= TH * TS;  // uniform
 #pragma unroll
-    for (int q = 0; q < PPT; ++q) {
-      const int Y = Y0 + ty + 16 * q;
-      if (X >= N || Y >= N) continue;
-      const size_t p = (size_t)bz * N * N + (size_t)Y * N + X;
-      const float v = acc_s[q] + acc_f[q];  // backprojection.fut:78
-      const float xn = P.out[p] + P.colinv[(size_t)Y * N + X] * v;
-      P.out[p] = xn;
-      if (staged)
-        st[(ty + 16 * q) * TS + tx] = xn;
-      else
-        P.outT[(size_t)bz * N * N + (size_t)X * N + Y] = xn;
-    }
-    if (staged) {
-      __syncthreads();
-      // thread -> column x = tid / 16 of the tile, rows PPT*(tid % 16) .. + PPT-1
-      const int cx = threadIdx.x >> 4, cy = (threadIdx.x & 15) * PPT;
-      const int XT = X0 + cx;
-      if (XT < N) {
+    for (int m = 0; m < S; ++m) {
+      if (S > 1 && img0 + m >= P.batch) break;  // uniform
+      if (m > 0 && staged) __syncthreads();     // the previous image's tile has been read
+      const size_t off = (size_t)(img0 + m) * N * N;
 #pragma unroll
-        for (int k = 0; k < PPT; ++k) {
-          const int YT = Y0 + cy + k;
-          if (YT < N) P.outT[(size_t)bz * N * N + (size_t)XT * N + YT] = st[(cy + k) * TS + cx];
+      for (int q = 0; q < PPT; ++q) {
+        const int Y = Y0 + ty + 16 * q;
+        if (X >= N || Y >= N) continue;
+        const size_t p = off + (size_t)Y * N + X;
+        const float v = acc_s[q][m] + acc_f[q][m];  // backprojection.fut:78
+        const float xn = P.out[p] + P.colinv[(size_t)Y * N + X] * v;
+        P.out[p] = xn;
+        if (staged)
+          st[(ty + 16 * q) * TS + tx] = xn;
+        else
+          P.outT[off + (size_t)X * N + Y] = xn;
+      }
+      if (staged) {
+        __syncthreads();
+        // thread -> column x = tid / 16 of the tile, rows PPT*(tid % 16) .. + PPT-1
+        const int cx = threadIdx.x >> 4, cy = (threadIdx.x & 15) * PPT;
+        const int XT = X0 + cx;
+        if (XT < N) {
+#pragma unroll
+          for (int k = 0; k < PPT; ++k) {
+            const int YT = Y0 + cy + k;
+            if (YT < N) P.outT[off + (size_t)XT * N + YT] = st[(cy + k) * TS + cx];
+          }
         }
       }
     }
@@ -889,15 +953,19 @@ __device__ __forceinline__ void bp_item(const BpParams& P, int tile_x, int tile_
   }
   if (X >= N) return;
 #pragma unroll
-  for (int q = 0; q < PPT; ++q) {
-    const int Y = Y0 + ty + 16 * q;
-    if (Y >= N) continue;
-    const size_t p = (size_t)bz * N * N + (size_t)Y * N + X;
-    const float v = acc_s[q] + acc_f[q];  // backprojection.fut:78
-    if constexpr (MODE == BP_PLAIN) {
-      P.out[p] = v;
-    } else {
-      P.out[p] = (v == 0.0f) ? 0.0f : 1.0f / v;
+  for (int m = 0; m < S; ++m) {
+    if (S > 1 && img0 + m >= P.batch) break;  // uniform
+#pragma unroll
+    for (int q = 0; q < PPT; ++q) {
+      const int Y = Y0 + ty + 16 * q;
+      if (Y >= N) continue;
+      const size_t p = (size_t)(img0 + m) * N * N + (size_t)Y * N + X;
+      const float v = acc_s[q][m] + acc_f[q][m];  // backprojection.fut:78
+      if constexpr (MODE == BP_PLAIN) {
+        P.out[p] = v;
+      } else {
+        P.out[p] = (v == 0.0f) ? 0.0f : 1.0f / v;
+      }
     }
   }
 }
@@ -925,23 +993,6 @@ typedef __attribute__((address_space(3))) float lds_float;
 template <int K>
 __device__ __forceinline__ int bcast16i(int v) {
   return __builtin_amdgcn_mov_dpp(v, 0x150 + K, 0xf, 0xf, true);
-}
-
-// S floats of S images side by side in LDS, and one of them.
-template <int S>
-struct Pack {
-  typedef float T __attribute__((ext_vector_type(S)));
-};
-template <>
-struct Pack<1> {
-  typedef float T;
-};
-template <int S>
-__device__ __forceinline__ float pack_at(const typename Pack<S>::T& v, int k) {
-  if constexpr (S == 1)
-    return v;
-  else
-    return v[k];
 }
 
 // The staged walk of one ray per lane over the workgroup's rows i0 .. i1 (uniform) in blocks

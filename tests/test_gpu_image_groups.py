@@ -1,6 +1,7 @@
-"""Kernels that work on several images at once (A.x 4 or 2 images per workgroup) give each image
-the bits it gets alone: batches around the group sizes, every staged width (chunks of 64
-columns: bin widths 1, 1.3 and 2), groups of fewer than four lines and a ragged last bin block.
+"""Kernels that work on several images at once (A.x 4 or 2 images per workgroup, B.r, A^T.r and the
+SIRT update 8, 4 or 2) give each image the bits it gets alone: batches around the group sizes,
+every staged width of A.x (chunks of 64 columns: bin widths 1, 1.3 and 2), groups of fewer than
+four lines, a ragged last bin block and tile row, tiles with and without the exact step.
 The images hold both signs and, in one case, values far apart."""
 import math
 
@@ -38,6 +39,36 @@ def test_projection_of_a_batch_is_each_images_own(ctx, name, N, A, R, start, drh
             assert torch.equal(got[k], geo.fp(x[k].contiguous())), k
     finally:
         geo.set_variants(-1, -1)
+
+
+# the batches run 2, 4, 4, 8 and 8 images per workgroup at 440^2 (28 x 14 tiles of 16 x 32)
+@pytest.mark.parametrize("batch", [2, 3, 6, 11, 16])
+@pytest.mark.parametrize("op", ["bp", "bp_adjoint"])
+def test_backprojection_of_a_batch_is_each_images_own(ctx, op, batch):
+    N, A, R = 440, 37, 631
+    geo = _geometry(ctx, N, A, R, 0.0, 1.0)
+    gen = torch.Generator(device="cuda").manual_seed(batch)
+    y = torch.randn(batch, A, R, device="cuda", generator=gen)
+    y[-1] *= 1e6
+    got = getattr(geo, op)(y)
+    geo.set_variants(7, 2)
+    try:
+        for k in range(batch):
+            assert torch.equal(got[k], getattr(geo, op)(y[k].contiguous())), k
+    finally:
+        geo.set_variants(-1, -1)
+
+
+def test_sirt_update_of_a_batch_is_each_slices_own(ctx):
+    N, A, R, batch = 440, 37, 631, 9
+    geo = _geometry(ctx, N, A, R, 0.0, 1.0)
+    b = torch.rand(batch, A, R, device="cuda", generator=torch.Generator(device="cuda").manual_seed(3))
+    x = torch.zeros(batch, N, N, device="cuda")
+    geo.sirt_(x, b, 3)
+    for k in range(batch):
+        one = torch.zeros(N, N, device="cuda")
+        geo.sirt_(one, b[k].contiguous(), 3)
+        assert torch.equal(x[k], one), k
 
 
 @pytest.mark.parametrize("batch", [2, 3, 6])
