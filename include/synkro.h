@@ -46,7 +46,8 @@ enum {
    * 0 (default): the per-step quotients use the hardware reciprocal (<= 2 ulp per
    *    length); pixel indices and candidate sets are unchanged. */
   SK_OPT_EXACT = 1,
-  /* Tile / rays-per-thread variant for the projector kernels (0 = autotuned default). */
+  /* Kernel variant of the projector kernels for geometries that were not tuned (0 = chosen by a
+   * rule on the sizes). */
   SK_OPT_FP_VARIANT = 2,
   SK_OPT_BP_VARIANT = 3
 };

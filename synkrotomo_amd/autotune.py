@@ -23,7 +23,7 @@ def cache_path() -> str:
 
 
 # Bumped whenever the meaning of the variant numbers changes, so old cache entries are ignored.
-VARIANT_TABLE = 5
+VARIANT_TABLE = 6
 
 
 def batch_bucket(batch: int) -> int:

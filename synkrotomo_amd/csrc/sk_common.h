@@ -40,12 +40,15 @@ struct alignas(32) Line {
 struct Geom {
   int A = 0, R = 0, N = 0, n_steep = 0, ncand = 0;
   float rho0 = 0.f, drho = 1.f;
-  // Unit bins with two candidates per pixel and |rho0| + N < 2^20, where the fast candidate
-  // index (rounding error < 0.4 bin) needs no clamp: the specialised backprojector applies.
+  // Unit bins with two candidates per pixel and |rho0| + N < 2^20: the exact backprojector's
+  // specialised loop applies.
   bool bp_two_cand = false;
   // The fast candidate index is off by less than 0.4 bin (|rho0| + N < 2^20 bins), so it drops no
   // ray with a nonzero length: the fast A^T and B^T apply.
   bool index_safe = false;
+  // Candidates per pixel (1..4) of the hoisted fast backprojector, whose fast index needs no clamp;
+  // 0 where it does not apply (index not safe, or bins narrower than 0.354: the general path).
+  int bp_nc = 0;
   // Row-segment width (floats) the staged forward projector needs for 256 consecutive bins.
   int fps_w = 0;
   // Grouped staged forward projector: line groups (int4 entries, fpg_groups in sk_geom.hip),

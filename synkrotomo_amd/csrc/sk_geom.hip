@@ -337,6 +337,7 @@ int sk_geom_create(sk_ctx* ctx, const float* angles_host, int A, float rho0, flo
   G.A = A; G.R = R; G.N = N; G.rho0 = rho0; G.drho = drho; G.ncand = ncand;
   G.bp_two_cand = drho == 1.0f && ncand == 2 && std::fabs((double)rho0) + N < (double)(1 << 20);
   G.index_safe = std::fabs((double)rho0) + N < (double)(1 << 20) * drho;
+  G.bp_nc = G.index_safe && ncand <= 4 ? ncand : 0;
   G.device = c->device;
   G.n_steep = build_lines(angles_host, A, G.lines, N);
   {
@@ -373,7 +374,7 @@ int sk_geom_create(sk_ctx* ctx, const float* angles_host, int A, float rho0, flo
     }
     if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
   }
-  if (e == hipSuccess && G.bp_two_cand && N / BP_TW < 65536) {
+  if (e == hipSuccess && G.bp_nc && N / BP_TW < 65536) {
     const std::vector<unsigned> ord = bp_tile_orders(N, G.n_steep, A, G.bp_order_off);
     e = hipMalloc(&G.d_bp_order, sizeof(unsigned) * ord.size());
     if (e == hipSuccess)

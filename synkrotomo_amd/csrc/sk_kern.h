@@ -525,6 +525,7 @@ __device__ __forceinline__ void bp_item(const BpParams& P, int tile_x, int tile_
   // candidate address comes from floor(-t) (one conversion) instead of ceil(t).
   constexpr bool REV = FASTREF && NC > 0;
   const int ncand = NC > 0 ? NC : P.ncand;
+  const bool unit = DR1 || P.drho == 1.0f;  // uniform
   const int W = P.W;
   const int tx = threadIdx.x & (BP_TW - 1), ty = threadIdx.x / BP_TW;
   constexpr int TH = 16 * PPT;
@@ -567,17 +568,17 @@ __device__ __forceinline__ void bp_item(const BpParams& P, int tile_x, int tile_
       const float cx0 = (float)((fl ? Y0 : X0) - h), cy0 = (float)((fl ? X0 : Y0) - h);
       const float cx1 = cx0 + (float)((fl ? TH : BP_TW) - 1);
       const float cy1 = cy0 + (float)((fl ? BP_TW : TH) - 1);
-      float smin = cand_s<DR1>(L, cx0, cy0, P.rho0, P.drho);
-      smin = fminf(smin, cand_s<DR1>(L, cx1, cy0, P.rho0, P.drho));
-      smin = fminf(smin, cand_s<DR1>(L, cx0, cy1, P.rho0, P.drho));
-      smin = fminf(smin, cand_s<DR1>(L, cx1, cy1, P.rho0, P.drho));
+      auto first = [&](float x, float y) {  // t / 1 = t: no division for unit bins
+        return unit ? cand_s<true>(L, x, y, P.rho0, P.drho) : cand_s<false>(L, x, y, P.rho0, P.drho);
+      };
+      const float smin = fminf(fminf(first(cx0, cy0), first(cx1, cy0)), fminf(first(cx0, cy1), first(cx1, cy1)));
       BpLineLds e;
       // The hoisted fast path starts the window one bin lower: its index may round one bin
       // below the reference's at the tile's lowest corner (the top keeps a one-bin margin).
       e.w0 = (int)smin - (REV ? 1 : 0);
       e.ci = e.si = e.cst = 0.0f;
       if constexpr (FASTREF) {
-        const float idr = DR1 ? 1.0f : 1.0f / P.drho;
+        const float idr = unit ? 1.0f : 1.0f / P.drho;
         e.ci = L.cost * idr;
         e.si = L.sint * idr;
         e.cst = -(fmaf(L.cost, L.fc, L.sint * L.fs) + P.rho0) * idr;
@@ -684,7 +685,7 @@ __device__ __forceinline__ void bp_item(const BpParams& P, int tile_x, int tile_
 #pragma unroll
           for (int q = 0; q < PPT; ++q) {
             ex[q] = KIND == 5 || KIND == 6 || (KIND != 2 && SLOTS >= 0 && ((SLOTS >> q) & 1));
-            // t is within 0.4 bin of the reference's index (|rho0| + N < 2^20 for this
+            // t is within 0.4 bin of the reference's index (|rho0| + N < 2^20 bins for this
             // path), so its ceiling lies in [w0, w0 + W - NC]: no clamp.
             const float t = part == 0 ? fmaf(lc.si, yh[q], tb) : fmaf(lc.ci, xh[q], tb);
             const int at = neg_ceil_to_int(t);

@@ -1,4 +1,5 @@
-// sk_proj.hip -- the per-call projector kernels and their C-ABI entry points.
+// sk_proj.hip -- the per-call forward projector kernels and the projectors' C-ABI entry points
+// (the backprojector kernels: sk_bp.hip).
 //
 //   k_fp  A.x   (futhark/forwardprojection.fut:21-84).  Ray-parallel: one lane per ray (or
 //               two, variant 1), a wavefront = 64 consecutive bins of one line.  All lanes
@@ -19,11 +20,6 @@
 //               lines adjacent in slope, 16 bins of each line per wave, so the staged segment
 //               of a block is two to four chunks of 64 columns instead of six; blocks of 16
 //               rows.  Same walk, for 1, 2 or 4 images at once.
-//   k_bp  B.r   (futhark/backprojection.fut:20-93).  Pixel-parallel gather, no atomics: a
-//               block owns a 16 x 16*PPT pixel tile and walks the lines in order, staging
-//               for each block of 32 lines the tile's rho-window of the sinogram in LDS
-//               together with the per-bin intercepts r/cost.
-//   k_bp_images B.r of 2, 4 or 8 images per workgroup on 16 x 32 tiles (unit bins, fast mode).
 //
 // The work items themselves live in sk_kern.h (shared with the persistent kernels).
 // With SK_OPT_EXACT the results are bitwise those of the sequential FP32 restatement of
@@ -119,42 +115,6 @@ __global__ __launch_bounds__(FPS_RAYS, fpg_waves_per_simd(S, CPLMAX)) void k_fp_
     fpg_item<MODE, CPLMAX >= 4 ? 4 : 2, S>(P, grp, blockIdx.y, blockIdx.z, (float*)seg4);
 }
 
-// Grid: (tiles across, tiles down, images).  Dynamic LDS: BP_LB * W float2.
-template <bool EXACT, int MODE, int WEIGHTS, int NC, bool DR1, int PPT>
-__global__ __launch_bounds__(256, NC > 0 ? 8 : 1) void k_bp(BpParams P) {
-  extern __shared__ float2 win[];
-  __shared__ BpLineLds lsh[BP_LB];
-  int tx = blockIdx.x, ty = blockIdx.y;
-  if (P.order) {
-    const unsigned t = P.order[blockIdx.y * gridDim.x + blockIdx.x];
-    tx = (int)(t & 0xffffu);
-    ty = (int)(t >> 16);
-  }
-  bp_item<EXACT, MODE, WEIGHTS, NC, DR1, PPT>(P, tx, ty, blockIdx.z, win, lsh);
-}
-
-// The hoisted fast path for S images at once on 16 x 32 tiles: grid (tiles across, tiles down,
-// images / S).  Dynamic LDS: BP_LB * W * (1 + S) floats.  One image issues 13 VALU per pixel and
-// line for the index, the positions and the lengths of the two candidates and 2 FMAs; S images
-// share the 13 and read 8 + 8 S bytes of LDS instead of 16 S.  64 images of 512^2, 512 angles:
-// 3.41 ms one at a time (16 x 64 tiles), 2.37, 1.61 and 1.45 ms for S = 2, 4 and 8, which is LDS
-// bandwidth next (16 x 64 tiles with S = 4 hold 127 registers and leave 3 workgroups per CU:
-// 1.69 ms; 16 x 16: 1.79).
-constexpr int BP_IMAGES_PPT = 2;
-
-template <int MODE, int WEIGHTS, int S>
-__global__ __launch_bounds__(256, S == 8 ? 3 : (S == 4 ? 6 : 8)) void k_bp_images(BpParams P) {
-  extern __shared__ float4 win4[];
-  __shared__ BpLineLds lsh[BP_LB];
-  int tx = blockIdx.x, ty = blockIdx.y;
-  if (P.order) {
-    const unsigned t = P.order[blockIdx.y * gridDim.x + blockIdx.x];
-    tx = (int)(t & 0xffffu);
-    ty = (int)(t >> 16);
-  }
-  bp_item<false, MODE, WEIGHTS, 2, true, BP_IMAGES_PPT, S>(P, tx, ty, blockIdx.z, (float2*)win4, lsh);
-}
-
 // ------------------------------------------------------------------------ launchers
 int launched(Ctx* c, const char* what) {
   hipError_t e = hipGetLastError();
@@ -178,7 +138,6 @@ FpParams fp_params(const Geom* g, const FpArgs& a) {
 int fp_rays_per_lane(int variant) {
   return (variant == 1 || variant == 4) ? 2 : (variant == 2 ? 4 : 1);
 }
-int bp_pixels_per_lane(int variant) { return variant == 1 ? 2 : (variant == 2 ? 4 : 1); }
 
 template <bool EXACT, int MODE, int WEIGHTS, bool DR1, int RPT, int ORDER = 0>
 static void fp_go(const Geom* g, const FpArgs& a, hipStream_t s) {
@@ -248,9 +207,18 @@ static void fp_go_grouped(const Geom* g, const FpArgs& a, hipStream_t s) {
   }
 }
 
+// The kernel of a geometry that was not tuned, on a context whose option is 0: the grouped one (and
+// below it what a geometry without line groups, or exact mode, falls back to).  From 128^2 to
+// 2048^2, angle counts 0.35 N to 1.6 N and bins of 0.5 to 2 it is the fastest or within 0.3 us of
+// the fastest (one ray per lane, the default before, us against grouped: 128^2 and 89 angles 13.5,
+// 13.2; 256^2 and 179 30.6, 21.1; 512^2 and 358 91, 59; 2048^2 and 1433 3662, 1750).  Smaller
+// images take a few rows only and the short per-wave kernel is as fast (64^2, 100 angles: 9.0,
+// 9.5), with a tenth of the code to fetch on a first call.
+static int fp_variant_default(const Geom* g) { return g->N < 128 ? 3 : 7; }
+
 int launch_fp(Ctx* c, const Geom* g, FpMode mode, const FpArgs& a, hipStream_t s) {
   const bool ex = c->exact != 0;
-  int v = g->fp_variant >= 0 ? g->fp_variant : c->fp_variant;
+  int v = g->fp_variant >= 0 ? g->fp_variant : (c->fp_variant ? c->fp_variant : fp_variant_default(g));
   if (v == 7) {
     if (!ex && g->d_fpg && mode != FP_ONES_INV) {
       if (mode == FP_PLAIN)
@@ -304,111 +272,6 @@ int launch_fp_bpt(Ctx* c, const Geom* g, const FpArgs& a, hipStream_t s) {
   else
     hipLaunchKernelGGL((k_fp_listed<false>), grid, dim3(FP_BLOCK), 0, s, fp_params(g, a), g->d_degen);
   return launched(c, "backprojection-transpose kernel");
-}
-
-BpParams bp_params(const Geom* g, const BpArgs& a, int ppt) {
-  const unsigned* order =
-      g->d_bp_order ? g->d_bp_order + g->bp_order_off[ppt == 1 ? 0 : (ppt == 2 ? 1 : 2)] : nullptr;
-  return BpParams{g->d_lines, g->A, g->R, g->N, g->ncand, bp_window_bins(ppt, g->drho, g->ncand), a.batch,
-                  g->n_steep, g->rho0, g->drho, a.sino, a.out, a.outT, a.colinv, g->d_inter, order};
-}
-
-template <bool EXACT, int MODE, int WEIGHTS, int NC, bool DR1, int PPT>
-static void bp_go(const Geom* g, const BpArgs& a, hipStream_t s) {
-  const BpParams P = bp_params(g, a, PPT);
-  const int TH = 16 * PPT;
-  dim3 grid((g->N + BP_TW - 1) / BP_TW, (g->N + TH - 1) / TH, a.batch);
-  const size_t lds = sizeof(float2) * BP_LB * (size_t)P.W;
-  hipLaunchKernelGGL((k_bp<EXACT, MODE, WEIGHTS, NC, DR1, PPT>), grid, dim3(256), lds, s, P);
-}
-
-template <int MODE, int WEIGHTS, int S>
-static void bp_go_images(const Geom* g, const BpArgs& a, hipStream_t s) {
-  const BpParams P = bp_params(g, a, BP_IMAGES_PPT);
-  const int TH = 16 * BP_IMAGES_PPT;
-  const dim3 grid((g->N + BP_TW - 1) / BP_TW, (g->N + TH - 1) / TH, (a.batch + S - 1) / S);
-  const size_t lds = sizeof(float) * BP_LB * (size_t)P.W * (1 + S);
-  hipLaunchKernelGGL((k_bp_images<MODE, WEIGHTS, S>), grid, dim3(256), lds, s, P);
-}
-
-template <int MODE, int WEIGHTS>
-static void bp_go_images_s(int images, const Geom* g, const BpArgs& a, hipStream_t s) {
-  if (images == 8)
-    bp_go_images<MODE, WEIGHTS, 8>(g, a, s);
-  else if (images == 4)
-    bp_go_images<MODE, WEIGHTS, 4>(g, a, s);
-  else
-    bp_go_images<MODE, WEIGHTS, 2>(g, a, s);
-}
-
-// Images per workgroup of the fast backprojector, 1 = the one-image kernels.  Below about a
-// workgroup per CU more images only lengthen each one (the walk over the lines is serial): 256^2,
-// 179 angles (128 tiles of 16 x 32), us for 1, 2 and 4 images per workgroup: 3 images 40.6, 48.4,
-// 53.9; 6 images 58.2, 52.5, 56.2; 16 images 103, 73.8, 61.3.  512^2, 358 angles (512 tiles):
-// 2 images 114, 95.7, 107; 3 images 149, 130, 110; 8 images 336, 220, 150, and 8 per workgroup
-// 140.
-int bp_images(const Geom* g, int batch) {
-  if (!g->bp_two_cand) return 1;
-  const int TH = 16 * BP_IMAGES_PPT;
-  const long tiles = (long)((g->N + BP_TW - 1) / BP_TW) * ((g->N + TH - 1) / TH);
-  if (batch >= 7 && tiles * ((batch + 7) / 8) >= 512) return 8;
-  if (batch >= 3 && tiles * ((batch + 3) / 4) >= 256) return 4;
-  if (batch >= 2 && tiles * ((batch + 1) / 2) >= 384) return 2;
-  return 1;
-}
-
-template <bool EXACT, int MODE, int WEIGHTS, int PPT>
-static void bp_go_nc(const Geom* g, const BpArgs& a, hipStream_t s) {
-  if (g->bp_two_cand)
-    bp_go<EXACT, MODE, WEIGHTS, 2, true, PPT>(g, a, s);
-  else
-    bp_go<EXACT, MODE, WEIGHTS, 0, false, PPT>(g, a, s);
-}
-
-template <bool EXACT, int MODE, int WEIGHTS>
-static void bp_go_v(int variant, const Geom* g, const BpArgs& a, hipStream_t s) {
-  if ((EXACT && WEIGHTS != W_REF) || variant == 0)
-    bp_go_nc<EXACT, MODE, WEIGHTS, 1>(g, a, s);
-  else if (variant == 1)
-    bp_go_nc<EXACT, MODE, WEIGHTS, 2>(g, a, s);
-  else
-    bp_go_nc<EXACT, MODE, WEIGHTS, 4>(g, a, s);
-}
-
-template <int MODE, int WEIGHTS>
-static void bp_go_ex(bool ex, int variant, const Geom* g, const BpArgs& a, hipStream_t s) {
-  if (ex)
-    bp_go_v<true, MODE, WEIGHTS>(variant, g, a, s);
-  else
-    bp_go_v<false, MODE, WEIGHTS>(variant, g, a, s);
-}
-
-int launch_bp(Ctx* c, const Geom* g, BpMode mode, BpWeights w, const BpArgs& a, hipStream_t s) {
-  const bool ex = c->exact != 0;
-  int v = g->bp_variant >= 0 ? g->bp_variant : c->bp_variant;
-  if (sizeof(float2) * BP_LB * (size_t)bp_window_bins(bp_pixels_per_lane(v), g->drho, g->ncand) > 60 * 1024)
-    v = 0;
-  if (sizeof(float2) * BP_LB * (size_t)bp_window_bins(1, g->drho, g->ncand) > 60 * 1024)
-    return fail(c, SK_EINVAL, "backprojection window exceeds LDS (deltarho too small)");
-  if (w == W_ADJ && mode != BP_PLAIN) return fail(c, SK_EINVAL, "adjoint weights support plain mode only");
-  const int images = ex || mode == BP_ONES_INV ? 1 : bp_images(g, a.batch);
-  if (images > 1) {
-    if (w == W_ADJ)
-      bp_go_images_s<BP_PLAIN, W_ADJ>(images, g, a, s);
-    else if (mode == BP_SIRT)
-      bp_go_images_s<BP_SIRT, W_REF>(images, g, a, s);
-    else
-      bp_go_images_s<BP_PLAIN, W_REF>(images, g, a, s);
-  } else if (w == W_REF) {
-    switch (mode) {
-      case BP_PLAIN: bp_go_ex<BP_PLAIN, W_REF>(ex, v, g, a, s); break;
-      case BP_ONES_INV: bp_go_ex<BP_ONES_INV, W_REF>(ex, 0, g, a, s); break;
-      case BP_SIRT: bp_go_ex<BP_SIRT, W_REF>(ex, v, g, a, s); break;
-    }
-  } else {
-    bp_go_ex<BP_PLAIN, W_ADJ>(ex || !g->index_safe, v, g, a, s);
-  }
-  return launched(c, "backprojection kernel");
 }
 
 }  // namespace sk
