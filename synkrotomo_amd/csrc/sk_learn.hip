@@ -16,14 +16,14 @@
 //                 derivative of the layer's output fused into the staging of its input.
 //   k_conv_in     1 or 2 -> 32 (288 MACs per pixel and input channel) on VALU with fused bias and
 //                 ReLU, in FP32 on the FP32 input (the image, or the image and the SIRT update
-//                 direction interleaved); the data gradients of both thin layers likewise.
+//                 direction interleaved); the data gradient of the last layer likewise.
 //   k_conv_out_mfma  32 -> 1: per 16x16 tile, the 9 tap products of every halo pixel in one
 //                 MFMA per 16 pixels, then a 9-term shifted sum per output, fused bias and
-//                 residual.
+//                 residual; the data gradient of the first layer likewise.
 //   k_wgrad32_mfma  weight and bias gradients of the 32 -> 32 layers on MFMA (K = pixels),
-//                 channel-major operands staged in LDS; per-block partial sums (deterministic),
-//                 then k_reduce_partials.
-//   k_wgrad       weight and bias gradients of the thin layers (1 -> 32, 32 -> 1) on VALU, the
+//                 tiles staged in LDS as they are and transposed by the reads; per-block partial
+//                 sums (deterministic), then k_reduce_partials.
+//   k_wgrad_thin  weight and bias gradients of the thin layers (1 -> 32, 32 -> 1) on VALU, the
 //                 same per-block partials.
 //   k_phantom     random-ellipse phantoms, evaluated in FP64 exactly as the numpy
 //                 generator (synkrotomo_amd/phantom.py) does.
@@ -293,155 +293,96 @@ __global__ __launch_bounds__(256) void k_conv_out_dgrad(int H, int W, long npix,
 }
 
 // dx[q][c] = sum_{t,co} w[co][t][c] g1[q - off_t][co],  g1 = dh * (h > 0)   (data gradient of
-// k_conv_in; dx FP32 [B][H][W][CIN])
+// k_conv_in; dx FP32 [B][H][W][CIN]).  As k_conv_out_mfma: per 16x16 tile and input channel c, each
+// of the 18x18 halo pixels of g1 gets U[p][t] = sum_co g1[p][co] w[co][t][c] for the 9 taps in one
+// MFMA per 16 pixels (products of BF16 values, exact in the FP32 accumulator's input), then each
+// output sums its 9 shifted taps.  Bound by the two activation streams: 8 x 512^2, 1.21 times 134 MB
+// each, 69 us = 4.7 TB/s (on VALU with one thread per pixel re-reading every neighbour's 32
+// channels: 851 us).
 template <int CIN>
-__global__ __launch_bounds__(256) void k_conv_in_dgrad(int H, int W, long npix, const __bf16* __restrict__ dh,
+__global__ __launch_bounds__(256) void k_conv_in_dgrad(int H, int W, const __bf16* __restrict__ dh,
                                                        const __bf16* __restrict__ hmask,
                                                        const __bf16* __restrict__ w,
                                                        float* __restrict__ dx) {
-  __shared__ float sw[NCH * 9 * CIN];
-  for (int i = threadIdx.x; i < NCH * 9 * CIN; i += 256) sw[i] = (float)w[i];
-  __syncthreads();
-  const long p = (long)blockIdx.x * 256 + threadIdx.x;
-  if (p >= npix) return;
-  const long b = p / ((long)H * W);
-  const int r = (int)(p - b * H * W);
-  const int py = r / W, px = r - py * W;
-  float s[CIN];
+  __shared__ float U[CO_SLOTS * 9];
+  const int tiles_x = (W + CT - 1) / CT, tiles_img = tiles_x * ((H + CT - 1) / CT);
+  const int tile = blockIdx.x % tiles_img;
+  const int tx0 = (tile % tiles_x) * CT, ty0 = (tile / tiles_x) * CT;
+  const size_t img = (size_t)(blockIdx.x / tiles_img) * H * W;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int m = lane & 15, kq = lane >> 4;
+  constexpr int NG = CO_SLOTS / 16, GPW = (NG + 3) / 4;
+  bf16x8 a[GPW];
 #pragma unroll
-  for (int c = 0; c < CIN; ++c) s[c] = 0.0f;
-  for (int t = 0; t < 9; ++t) {
-    const int yy = py - (t / 3 - 1), xx = px - (t % 3 - 1);
-    if (yy < 0 || yy >= H || xx < 0 || xx >= W) continue;
-    const size_t off = ((b * H + yy) * W + xx) * NCH;
-    for (int q = 0; q < 4; ++q) {
-      const bf16x8 gv = *(const bf16x8*)(dh + off + q * 8);
-      const bf16x8 mv = *(const bf16x8*)(hmask + off + q * 8);
+  for (int k = 0; k < GPW; ++k) {
+    const int slot = (wv + 4 * k) * 16 + m;  // A row m: halo pixel `slot`
+    const int hy = slot / (CT + 2), hx = slot - hy * (CT + 2);
+    const int gy = ty0 + hy - 1, gx = tx0 + hx - 1;
+    for (int i = 0; i < 8; ++i) a[k][i] = (__bf16)0.0f;
+    if (slot < (CT + 2) * (CT + 2) && gy >= 0 && gy < H && gx >= 0 && gx < W) {
+      const size_t off = (img + (size_t)gy * W + gx) * NCH + 8 * kq;
+      const bf16x8 g = *(const bf16x8*)(dh + off), mk = *(const bf16x8*)(hmask + off);
+#pragma unroll
       for (int i = 0; i < 8; ++i)
-        if ((float)mv[i] > 0.0f)
-#pragma unroll
-          for (int c = 0; c < CIN; ++c) s[c] = fmaf(sw[((q * 8 + i) * 9 + t) * CIN + c], (float)gv[i], s[c]);
+        if ((float)mk[i] > 0.0f) a[k][i] = g[i];
     }
   }
+  const int ty = threadIdx.x >> 4, tx = threadIdx.x & 15;
+  const int oy = ty0 + ty, ox = tx0 + tx;
 #pragma unroll
-  for (int c = 0; c < CIN; ++c) dx[p * CIN + c] = s[c];
+  for (int c = 0; c < CIN; ++c) {
+    if (c > 0) __syncthreads();  // the previous channel's sums have been read
+    // B: w[co 8kq .. 8kq+7][tap m][c] for taps 0..8, zero columns for m >= 9
+    bf16x8 wb;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) wb[i] = m < 9 ? w[((8 * kq + i) * 9 + m) * CIN + c] : (__bf16)0.0f;
+#pragma unroll
+    for (int k = 0; k < GPW; ++k) {
+      const int g = wv + 4 * k;
+      if (g >= NG) break;  // wave-uniform
+      const f32x4 u = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[k], wb, f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+      if (m < 9)
+        for (int i = 0; i < 4; ++i) U[(g * 16 + 4 * kq + i) * 9 + m] = u[i];
+    }
+    __syncthreads();
+    if (oy < H && ox < W) {
+      // tap t of output (ty, tx) comes from halo pixel (ty + 1 - (t/3 - 1), tx + 1 - (t%3 - 1))
+      float sum = 0.0f;
+#pragma unroll
+      for (int t = 0; t < 9; ++t) sum += U[((ty + 2 - t / 3) * (CT + 2) + tx + 2 - t % 3) * 9 + t];
+      dx[(img + (size_t)oy * W + ox) * CIN + c] = sum;
+    }
+  }
 }
 
 // ---------------------------------------------------------------------- weight gradients
-// dW[co][t][ci] = sum_p G[p][co] X[p + off_t][ci],  db[co] = sum_p G[p][co]
-// G: CO channels (bf16 NHWC, optionally masked by M > 0) or an FP32 image (CO == 1).
-// X: CI = 32 channels (bf16 NHWC) or CI <= 2 FP32 channels ([B][H][W][CI]).  Each block
-// accumulates over a grid-stride set of 16x16 tiles and writes CO*9*CI + CO partial sums.
-template <int CO, int CI>
-__global__ __launch_bounds__(256) void k_wgrad(int H, int W, int B, const void* __restrict__ Gp,
-                                               const __bf16* __restrict__ M,
-                                               const void* __restrict__ Xp,
-                                               float* __restrict__ partials) {
-  constexpr int NOUT = CO * 9 * CI + CO;
-  constexpr int PER = (NOUT + 255) / 256;
-  // 32-channel operands are BF16 already and stay BF16 in LDS; FP32 images stay FP32.
-  using GT = typename std::conditional<CO == 1, float, __bf16>::type;
-  using XT = typename std::conditional<CI <= 2, float, __bf16>::type;
-  __shared__ GT sg[CT * CT * CO];
-  __shared__ XT sx[(CT + 2) * (CT + 2) * CI];
-  float acc[PER];
-  for (int k = 0; k < PER; ++k) acc[k] = 0.0f;
-  const int tiles_x = (W + CT - 1) / CT, tiles_y = (H + CT - 1) / CT;
-  const long ntiles = (long)tiles_x * tiles_y * B;
-  for (long tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    const int b = (int)(tile / ((long)tiles_x * tiles_y));
-    const int tr = (int)(tile - (long)b * tiles_x * tiles_y);
-    const int ty0 = (tr / tiles_x) * CT, tx0 = (tr % tiles_x) * CT;
-    for (int e = threadIdx.x; e < CT * CT * CO; e += 256) {
-      const int pix = e / CO, co = e - pix * CO;
-      const int gy = ty0 + pix / CT, gx = tx0 + pix % CT;
-      float v = 0.0f;
-      if (gy < H && gx < W) {
-        const size_t p = ((size_t)b * H + gy) * W + gx;
-        if constexpr (CO == 1) {
-          v = ((const float*)Gp)[p];
-        } else {
-          v = (float)((const __bf16*)Gp)[p * CO + co];
-          if (M && !((float)M[p * CO + co] > 0.0f)) v = 0.0f;
-        }
-      }
-      sg[e] = (GT)v;
-    }
-    for (int e = threadIdx.x; e < (CT + 2) * (CT + 2) * CI; e += 256) {
-      const int pix = e / CI, ci = e - pix * CI;
-      const int py = pix / (CT + 2), px = pix % (CT + 2);
-      const int gy = ty0 + py - 1, gx = tx0 + px - 1;
-      float v = 0.0f;
-      if (gy >= 0 && gy < H && gx >= 0 && gx < W) {
-        const size_t p = ((size_t)b * H + gy) * W + gx;
-        if constexpr (CI <= 2)
-          v = ((const float*)Xp)[p * CI + ci];
-        else
-          v = (float)((const __bf16*)Xp)[p * CI + ci];
-      }
-      sx[e] = (XT)v;
-    }
-    __syncthreads();
-    for (int k = 0; k < PER; ++k) {
-      const int o = threadIdx.x + 256 * k;
-      if (o >= NOUT) break;
-      float s = 0.0f;
-      if (o < CO * 9 * CI) {
-        const int co = o / (9 * CI), rem = o - co * 9 * CI, t = rem / CI, ci = rem - t * CI;
-        const int ky = t / 3, kx = t % 3;
-        for (int py = 0; py < CT; ++py)
-          for (int px = 0; px < CT; ++px)
-            s = fmaf((float)sg[(py * CT + px) * CO + co],
-                     (float)sx[((py + ky) * (CT + 2) + px + kx) * CI + ci], s);
-      } else {
-        const int co = o - CO * 9 * CI;
-        for (int pix = 0; pix < CT * CT; ++pix) s += (float)sg[pix * CO + co];
-      }
-      acc[k] += s;
-    }
-    __syncthreads();
-  }
-  for (int k = 0; k < PER; ++k) {
-    const int o = threadIdx.x + 256 * k;
-    if (o < NOUT) partials[(size_t)blockIdx.x * NOUT + o] = acc[k];
-  }
-}
-
-// 32 -> 32 weight and bias gradients on MFMA: for each tap t, dW[co][t][ci] is a GEMM with M = 16
-// output channels, N = 16 input channels and K = pixels (v_mfma_f32_16x16x32_bf16, K = 32 pixels
-// per step); db[co] is the same GEMM against a column of ones.  The MFMA takes 8 consecutive K
-// values per lane from one row of A (and of B), so the NHWC operands are staged in LDS channel-
-// major: gT[co][pixel] for the 16x16 tile's gradient (masked by M > 0), and three copies of the
-// 18x18 input halo, xs[kx][ci][halo row][16 columns] with column j holding halo column j + kx,
-// so that a tap's shifted rows start 16-byte aligned.  A K step covers two pixel rows of the
-// tile (lane group kq: row 2s + kq/2, columns 8(kq%2) .. +7); wave w takes K steps 2w and 2w+1 of
-// every tile of its block and keeps all 36 tap x channel-block accumulators.  At the end the four
-// waves' sums are added in LDS in wave order and the block writes one partial (deterministic).
-constexpr int WG_GS = 256 + 8;       // gT row (elements): 256 pixels + pad (528 B, 16 B multiple)
-constexpr int WG_XS = 18 * 16 + 8;   // xs channel row: 18 halo rows x 16 columns + pad (592 B)
-constexpr int WG_NOUT = NCH * 9 * NCH + NCH;
-
-__global__ __launch_bounds__(256) void k_wgrad32_mfma(int H, int W, int B, const __bf16* __restrict__ G,
-                                                      const __bf16* __restrict__ M,
-                                                      const __bf16* __restrict__ X,
-                                                      float* __restrict__ partials) {
-  __shared__ __attribute__((aligned(16))) __bf16 gT[NCH * WG_GS];
-  __shared__ __attribute__((aligned(16))) __bf16 xs[3 * NCH * WG_XS];
-  static_assert(sizeof(__bf16) * 3 * NCH * WG_XS >= sizeof(float) * WG_NOUT, "reduction buffer");
+// dW[co][t][ci] = sum_p G[p][co] X[p + off_t][ci],  db[co] = sum_p G[p][co], over every pixel p.
+//
+// Thin layers: 32 BF16 channels V (NHWC, zeroed where M <= 0 when M is given) against CI FP32
+// channels F ([B][H][W][CI]): K[ch][t][c] = sum_p V[p][ch] F[p + off_t][c] on VALU, FP32 FMAs of the
+// unrounded FP32 values.  V = the gradient and F = the input for conv1 (TAIL false: out = K, then
+// db[ch] = sum V).  For conv4 (TAIL true) V = its input and F = the gradient: sum_p g[p] V[p +
+// off_t] = sum_q V[q] g[q - off_t], i.e. tap 8 - t of K, out [t][ch], then db = sum of F.
+// A wave walks 16x4 pixels of a 16x16 tile at a time: lane l holds channels 2(l%16) and +1 of row
+// l/16, so a pixel's V is one coalesced dword per lane and its 9 F values are read from LDS rows
+// into registers once per tile row; sums stay in registers over all of the block's tiles.
+// 8 x 512^2: 109 us for conv1 (V and M, 268 MB) and 39 us for conv4 (134 MB); one weight per thread
+// over LDS tiles: 236 and 195 us.
+template <int CI, bool TAIL>
+__global__ __launch_bounds__(256) void k_wgrad_thin(int H, int W, int B, const __bf16* __restrict__ V,
+                                                    const __bf16* __restrict__ M, const float* __restrict__ F,
+                                                    float* __restrict__ partials) {
+  constexpr int NW = NCH * 9 * CI, NOUT = NW + (TAIL ? 1 : NCH);
+  constexpr int FS = CT + 4;  // LDS row of F (floats): 18 columns, 16-byte multiple
+  __shared__ __attribute__((aligned(16))) float sf[CI][CT + 2][FS];
+  __shared__ float red[NOUT];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int m = lane & 15, kq = lane >> 4;
-  f32x4 acc[9][2][2];
-  f32x4 accb[2];
+  const int cp = lane & 15, sub = lane >> 4;
+  float acc[CI][2][9], accb[2] = {0.0f, 0.0f};
 #pragma unroll
-  for (int t = 0; t < 9; ++t)
+  for (int c = 0; c < CI; ++c)
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-      for (int c = 0; c < 2; ++c) acc[t][a][c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  accb[0] = accb[1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  bf16x8 ones;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) ones[i] = (__bf16)1.0f;
+    for (int t = 0; t < 9; ++t) acc[c][0][t] = acc[c][1][t] = 0.0f;
   const int tiles_x = (W + CT - 1) / CT, tiles_y = (H + CT - 1) / CT;
   const long ntiles = (long)tiles_x * tiles_y * B;
   for (long tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {  // uniform over the block
@@ -449,9 +390,157 @@ __global__ __launch_bounds__(256) void k_wgrad32_mfma(int H, int W, int B, const
     const int tr = (int)(tile - b * tiles_x * tiles_y);
     const int ty0 = (tr / tiles_x) * CT, tx0 = (tr % tiles_x) * CT;
     const size_t img = (size_t)b * H * W;
-    __syncthreads();  // the previous tile's LDS reads are done
-    for (int c = threadIdx.x; c < CT * CT * 4; c += 256) {  // gradient: 256 pixels x 4 quads
-      const int pix = c >> 2, q = c & 3;
+    // this lane's row of V: 16 pixels, two channels each
+    const int gy = ty0 + 4 * wv + sub;
+    uint32_t v[CT];
+#pragma unroll
+    for (int x = 0; x < CT; ++x) {
+      v[x] = 0u;
+      if (gy < H && tx0 + x < W) {
+        const size_t off = ((img + (size_t)gy * W + tx0 + x) * NCH >> 1) + cp;
+        v[x] = ((const uint32_t*)V)[off];
+        if (M) {
+          const uint32_t mk = ((const uint32_t*)M)[off];
+          // BF16 > 0 of each half (NaN is not): the sign and magnitude as FP32
+          if (!(__builtin_bit_cast(float, mk << 16) > 0.0f)) v[x] &= 0xffff0000u;
+          if (!(__builtin_bit_cast(float, mk & 0xffff0000u) > 0.0f)) v[x] &= 0x0000ffffu;
+        }
+      }
+    }
+    __syncthreads();  // the previous tile's F has been read
+    for (int e = threadIdx.x; e < (CT + 2) * (CT + 2) * CI; e += 256) {
+      const int pix = e / CI, c = e - pix * CI;
+      const int py = pix / (CT + 2), px = pix - py * (CT + 2);
+      const int fy = ty0 + py - 1, fx = tx0 + px - 1;
+      sf[c][py][px] = (fy >= 0 && fy < H && fx >= 0 && fx < W) ? F[(img + (size_t)fy * W + fx) * CI + c] : 0.0f;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < CI; ++c) {
+      float f[3][CT + 2];
+#pragma unroll
+      for (int r = 0; r < 3; ++r)
+#pragma unroll
+        for (int x = 0; x < CT + 2; ++x) f[r][x] = sf[c][4 * wv + sub + r][x];
+#pragma unroll
+      for (int x = 0; x < CT; ++x) {
+        const float v0 = __builtin_bit_cast(float, v[x] << 16), v1 = __builtin_bit_cast(float, v[x] & 0xffff0000u);
+#pragma unroll
+        for (int t = 0; t < 9; ++t) {
+          acc[c][0][t] = fmaf(v0, f[t / 3][x + t % 3], acc[c][0][t]);
+          acc[c][1][t] = fmaf(v1, f[t / 3][x + t % 3], acc[c][1][t]);
+        }
+        if (c == 0) {
+          if constexpr (TAIL) {  // the tile's own pixels of F (0 outside the image)
+            accb[0] += (gy < H && tx0 + x < W) ? f[1][x + 1] : 0.0f;
+          } else {
+            accb[0] += v0;
+            accb[1] += v1;
+          }
+        }
+      }
+    }
+  }
+  // the wave's four rows ((0 + 1) + (2 + 3)), then the waves in order
+  auto rows = [](float v) {
+    v += __shfl_xor(v, 16);
+    return v + __shfl_xor(v, 32);
+  };
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    accb[k] = rows(accb[k]);
+#pragma unroll
+    for (int c = 0; c < CI; ++c)
+#pragma unroll
+      for (int t = 0; t < 9; ++t) acc[c][k][t] = rows(acc[c][k][t]);
+  }
+  for (int w = 0; w < 4; ++w) {
+    __syncthreads();
+    if (wv != w || sub != 0) continue;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const int ch = 2 * cp + k;
+#pragma unroll
+      for (int c = 0; c < CI; ++c)
+#pragma unroll
+        for (int t = 0; t < 9; ++t) {
+          const int o = TAIL ? (8 - t) * NCH + ch : (ch * 9 + t) * CI + c;
+          red[o] = (w ? red[o] : 0.0f) + acc[c][k][t];
+        }
+      if (!TAIL || (k == 0 && cp == 0)) {
+        const int o = NW + (TAIL ? 0 : ch);
+        red[o] = (w ? red[o] : 0.0f) + accb[k];
+      }
+    }
+  }
+  __syncthreads();
+  for (int o = threadIdx.x; o < NOUT; o += 256) partials[(size_t)blockIdx.x * NOUT + o] = red[o];
+}
+
+// 32 -> 32 weight and bias gradients on MFMA: for each tap t, dW[co][t][ci] is a GEMM with M = 16
+// output channels, N = 16 input channels and K = pixels (v_mfma_f32_16x16x32_bf16, K = 32 pixels
+// per step); db[co] is the same GEMM against a column of ones.  The MFMA takes 8 consecutive K
+// values (pixels) per lane, the activations hold a pixel's channels side by side: the tiles go to
+// LDS as they are (16-byte stores) and ds_read_b64_tr_b16 transposes on the way out -- a group of 16
+// lanes reads 4 pixels x 16 channels and each lane gets one channel's 4 pixels -- so a tap's shift
+// is only another first pixel.  A pixel's 64 bytes are two halves of 16 channels, swapped where
+// bit 1 of the pixel's index is set: any 4 consecutive pixels then cover all 32 banks once.
+// Wave w of 8 takes channel block (cb, nb) = (w/2 % 2, w % 2) and K steps 4(w/4) .. +3 of every tile
+// of its block (two pixel rows per step: lane group kq holds row 2s + kq/2, columns 8(kq%2) .. +7).
+// The next tile is loaded into registers during this one's MFMAs.  At the end the two waves of a
+// channel block are added and the block writes one partial (deterministic).
+// 8 x 512^2: 102 us for the three streams' 400 MB = 3.9 TB/s (16-bit transposing stores of three
+// shifted copies: 280 us).
+constexpr int WG_NOUT = NCH * 9 * NCH + NCH;
+constexpr int WG_T = 512;                                       // threads
+constexpr int WG_GQ = CT * CT * 4 / WG_T;                       // 16-byte quads per thread: gradient
+constexpr int WG_XQ = ((CT + 2) * (CT + 2) * 4 + WG_T - 1) / WG_T;  // and input halo
+
+typedef __attribute__((address_space(3))) __bf16 lds_bf16;
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+
+// LDS element of channel 8q of pixel pix.
+__device__ __forceinline__ int wg_at(int pix, int q) { return pix * NCH + (((q >> 1) ^ (pix >> 1 & 1)) << 4) + ((q & 1) << 3); }
+
+// 8 pixels from pix of channel block blk (16 channels), one channel per lane m of the 16-lane group.
+__device__ __forceinline__ bf16x8 wg_read(const __bf16* s, int pix, int blk, int m) {
+  const int p0 = pix + (m >> 2), p1 = p0 + 4;
+  const int c = (m & 3) << 2;
+  union { s16x4 h[2]; bf16x8 v; } u;
+  u.h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(s + p0 * NCH + ((blk ^ (p0 >> 1 & 1)) << 4) + c));
+  u.h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(s + p1 * NCH + ((blk ^ (p1 >> 1 & 1)) << 4) + c));
+  return u.v;
+}
+
+__global__ __launch_bounds__(WG_T, 4) void k_wgrad32_mfma(int H, int W, int B, const __bf16* __restrict__ G,
+                                                          const __bf16* __restrict__ M,
+                                                          const __bf16* __restrict__ X,
+                                                          float* __restrict__ partials) {
+  constexpr int GE = CT * CT * NCH, XE = (CT + 2) * (CT + 2) * NCH;
+  __shared__ __attribute__((aligned(16))) __bf16 sg[GE + XE];
+  __bf16* sx = sg + GE;
+  static_assert(sizeof(__bf16) * (GE + XE) >= sizeof(float) * WG_NOUT, "reduction buffer");
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int m = lane & 15, kq = lane >> 4;
+  const int cb = wv >> 1 & 1, nb = wv & 1, half = wv >> 2;
+  f32x4 acc[9], accb = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int t = 0; t < 9; ++t) acc[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  bf16x8 ones;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) ones[i] = (__bf16)1.0f;
+  const int tiles_x = (W + CT - 1) / CT, tiles_y = (H + CT - 1) / CT;
+  const long ntiles = (long)tiles_x * tiles_y * B;
+  bf16x8 pg[WG_GQ], px[WG_XQ];
+  auto load = [&](long tile) {
+    const long b = tile / ((long)tiles_x * tiles_y);
+    const int tr = (int)(tile - b * tiles_x * tiles_y);
+    const int ty0 = (tr / tiles_x) * CT, tx0 = (tr % tiles_x) * CT;
+    const size_t img = (size_t)b * H * W;
+#pragma unroll
+    for (int k = 0; k < WG_GQ; ++k) {
+      const int c = threadIdx.x + WG_T * k, pix = c >> 2, q = c & 3;
       const int gy = ty0 + (pix >> 4), gx = tx0 + (pix & 15);
       bf16x8 v;
 #pragma unroll
@@ -466,92 +555,115 @@ __global__ __launch_bounds__(256) void k_wgrad32_mfma(int H, int W, int B, const
             if (!((float)mk[i] > 0.0f)) v[i] = (__bf16)0.0f;
         }
       }
-#pragma unroll
-      for (int i = 0; i < 8; ++i) gT[(8 * q + i) * WG_GS + pix] = v[i];
+      pg[k] = v;
     }
-    for (int c = threadIdx.x; c < (CT + 2) * (CT + 2) * 4; c += 256) {  // input halo: 324 pixels x 4 quads
-      const int pix = c >> 2, q = c & 3;
+#pragma unroll
+    for (int k = 0; k < WG_XQ; ++k) {
+      const int c = threadIdx.x + WG_T * k, pix = c >> 2, q = c & 3;
       const int hy = pix / (CT + 2), hx = pix - hy * (CT + 2);
       const int gy = ty0 + hy - 1, gx = tx0 + hx - 1;
       bf16x8 v;
 #pragma unroll
       for (int i = 0; i < 8; ++i) v[i] = (__bf16)0.0f;
-      if (gy >= 0 && gy < H && gx >= 0 && gx < W) v = *(const bf16x8*)(X + (img + (size_t)gy * W + gx) * NCH + 8 * q);
+      if (pix < (CT + 2) * (CT + 2) && gy >= 0 && gy < H && gx >= 0 && gx < W)
+        v = *(const bf16x8*)(X + (img + (size_t)gy * W + gx) * NCH + 8 * q);
+      px[k] = v;
+    }
+  };
+  long tile = blockIdx.x;
+  if (tile < ntiles) load(tile);
+  for (; tile < ntiles; tile += gridDim.x) {  // uniform over the block
+    __syncthreads();                          // the previous tile's LDS reads are done
 #pragma unroll
-      for (int kx = 0; kx < 3; ++kx) {
-        const int j = hx - kx;
-        if (j < 0 || j >= CT) continue;
+    for (int k = 0; k < WG_GQ; ++k) {
+      const int c = threadIdx.x + WG_T * k;
+      *(bf16x8*)(sg + wg_at(c >> 2, c & 3)) = pg[k];
+    }
 #pragma unroll
-        for (int i = 0; i < 8; ++i) xs[(kx * NCH + 8 * q + i) * WG_XS + hy * CT + j] = v[i];
-      }
+    for (int k = 0; k < WG_XQ; ++k) {
+      const int c = threadIdx.x + WG_T * k;
+      if ((c >> 2) < (CT + 2) * (CT + 2)) *(bf16x8*)(sx + wg_at(c >> 2, c & 3)) = px[k];
     }
     __syncthreads();
+    if (tile + gridDim.x < ntiles) load(tile + gridDim.x);  // in flight during the MFMAs
 #pragma unroll
-    for (int ss = 0; ss < 2; ++ss) {
-      const int py = 2 * (2 * wv + ss) + (kq >> 1), px0 = (kq & 1) * 8;
+    for (int ss = 0; ss < 4; ++ss) {
+      const int py = 2 * (4 * half + ss) + (kq >> 1), px0 = (kq & 1) * 8;
       // A: gradient of output channels cb*16 + m at the 8 pixels (py, px0 .. px0 + 7)
-      const bf16x8 a0 = *(const bf16x8*)(gT + m * WG_GS + py * CT + px0);
-      const bf16x8 a1 = *(const bf16x8*)(gT + (16 + m) * WG_GS + py * CT + px0);
-      accb[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, ones, accb[0], 0, 0, 0);
-      accb[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, ones, accb[1], 0, 0, 0);
+      const bf16x8 a = wg_read(sg, py * CT + px0, cb, m);
+      if (nb == 0) accb = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, ones, accb, 0, 0, 0);  // wave-uniform
 #pragma unroll
       for (int t = 0; t < 9; ++t) {
-        const int ky = t / 3, kx = t - 3 * (t / 3);
-#pragma unroll
-        for (int nb = 0; nb < 2; ++nb) {
-          // B: input channel nb*16 + m at the same pixels shifted by the tap
-          const bf16x8 bv = *(const bf16x8*)(xs + (kx * NCH + nb * 16 + m) * WG_XS + (py + ky) * CT + px0);
-          acc[t][0][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, bv, acc[t][0][nb], 0, 0, 0);
-          acc[t][1][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, bv, acc[t][1][nb], 0, 0, 0);
-        }
+        // B: input channel nb*16 + m at the same pixels shifted by the tap
+        const bf16x8 bv = wg_read(sx, (py + t / 3) * (CT + 2) + px0 + t % 3, nb, m);
+        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bv, acc[t], 0, 0, 0);
       }
     }
   }
   // C: lane (m, kq) holds rows 4kq + i (output channels cb*16 + 4kq + i) of column m (input
-  // channel nb*16 + m).  Waves add their sums in order 0, 1, 2, 3.
-  float* red = (float*)xs;
-  for (int w = 0; w < 4; ++w) {
-    __syncthreads();
-    if (wv == w) {
+  // channel nb*16 + m).  The waves of K steps 4..7 go through LDS to those of 0..3.
+  float* red = (float*)sg;
+  float* out = partials + (size_t)blockIdx.x * WG_NOUT;
+  __syncthreads();
+#pragma unroll
+  for (int ph = 0; ph < 2; ++ph) {
+    if (half == 1 - ph) {
 #pragma unroll
       for (int t = 0; t < 9; ++t)
 #pragma unroll
-        for (int cb = 0; cb < 2; ++cb)
+        for (int i = 0; i < 4; ++i) {
+          const int o = ((cb * 16 + 4 * kq + i) * 9 + t) * NCH + nb * 16 + m;
+          if (ph == 0)
+            red[o] = acc[t][i];
+          else
+            out[o] = acc[t][i] + red[o];
+        }
+      if (nb == 0 && m == 0)
 #pragma unroll
-          for (int nb = 0; nb < 2; ++nb)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              const int o = ((cb * 16 + 4 * kq + i) * 9 + t) * NCH + nb * 16 + m;
-              red[o] = (w ? red[o] : 0.0f) + acc[t][cb][nb][i];
-            }
-      if (m == 0)
-#pragma unroll
-        for (int cb = 0; cb < 2; ++cb)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int o = NCH * 9 * NCH + cb * 16 + 4 * kq + i;
-            red[o] = (w ? red[o] : 0.0f) + accb[cb][i];
-          }
+        for (int i = 0; i < 4; ++i) {
+          const int o = NCH * 9 * NCH + cb * 16 + 4 * kq + i;
+          if (ph == 0)
+            red[o] = accb[i];
+          else
+            out[o] = accb[i] + red[o];
+        }
     }
+    if (ph == 0) __syncthreads();
   }
-  __syncthreads();
-  for (int o = threadIdx.x; o < WG_NOUT; o += 256) partials[(size_t)blockIdx.x * WG_NOUT + o] = red[o];
 }
 
-// out[o] = sum over blocks b of partials[b][o] in a fixed order (deterministic): a workgroup
-// takes 64 consecutive outputs (coalesced rows of the partials), wave w sums the blocks
-// b = w, w + 4, ... in increasing order, then the four sums are added in wave order.
-__global__ __launch_bounds__(256) void k_reduce_partials(const float* __restrict__ partials, int nblocks,
-                                                         int nout, float* __restrict__ out) {
-  __shared__ float sh[4][64];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int o = blockIdx.x * 64 + lane;
+// out[o] = sum over blocks b of partials[b][o] in a fixed order (deterministic): a workgroup of 1024
+// threads takes OUTS consecutive outputs (coalesced rows of the partials); strand s of 1024/OUTS
+// sums the blocks b = s, s + strands, ..., eight loads in flight, then the strands' sums are added
+// in order.  OUTS = 64 for the 9248 outputs of the 32 -> 32 layers, 16 for the few hundred of the
+// thin ones (512 blocks x 9248 outputs: 5.0 us; before, with 64 outputs and four strands a workgroup,
+// 42 us on average over a training step's calls).
+template <int OUTS>
+__global__ __launch_bounds__(1024) void k_reduce_partials(const float* __restrict__ partials, int nblocks,
+                                                          int nout, float* __restrict__ out) {
+  constexpr int STR = 1024 / OUTS;
+  __shared__ float sh[STR][OUTS];
+  const int c = threadIdx.x % OUTS, r = threadIdx.x / OUTS;
+  const int o = blockIdx.x * OUTS + c;
   float s = 0.0f;
-  if (o < nout)
-    for (int b = w; b < nblocks; b += 4) s += partials[(size_t)b * nout + o];
-  sh[w][lane] = s;
+  if (o < nout) {
+    int b = r;
+    for (; b + 7 * STR < nblocks; b += 8 * STR) {
+      float v[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = partials[(size_t)(b + k * STR) * nout + o];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) s += v[k];
+    }
+    for (; b < nblocks; b += STR) s += partials[(size_t)b * nout + o];
+  }
+  sh[r][c] = s;
   __syncthreads();
-  if (w == 0 && o < nout) out[o] = ((sh[0][lane] + sh[1][lane]) + sh[2][lane]) + sh[3][lane];
+  if (r == 0 && o < nout) {
+    float t = sh[0][c];
+    for (int k = 1; k < STR; ++k) t += sh[k][c];
+    out[o] = t;
+  }
 }
 
 // ---------------------------------------------------------------------- phantoms
@@ -678,13 +790,12 @@ static int conv_in_dgrad_go(sk_ctx* ctx, int cin, int B, int H, int W, const voi
   if (rc) return rc;
   if (B < 1 || H < 1 || W < 1 || !dh || !hmask || !w || !dx)
     return fail(&ctx->c, SK_EINVAL, "conv_in_dgrad: bad arguments");
-  const long npix = (long)B * H * W;
-  const dim3 grid((unsigned)((npix + 255) / 256));
+  const dim3 grid((unsigned)((long)((W + CT - 1) / CT) * ((H + CT - 1) / CT) * B));
   if (cin == 1)
-    hipLaunchKernelGGL(k_conv_in_dgrad<1>, grid, dim3(256), 0, (hipStream_t)stream, H, W, npix, (const __bf16*)dh,
+    hipLaunchKernelGGL(k_conv_in_dgrad<1>, grid, dim3(256), 0, (hipStream_t)stream, H, W, (const __bf16*)dh,
                        (const __bf16*)hmask, (const __bf16*)w, dx);
   else
-    hipLaunchKernelGGL(k_conv_in_dgrad<2>, grid, dim3(256), 0, (hipStream_t)stream, H, W, npix, (const __bf16*)dh,
+    hipLaunchKernelGGL(k_conv_in_dgrad<2>, grid, dim3(256), 0, (hipStream_t)stream, H, W, (const __bf16*)dh,
                        (const __bf16*)hmask, (const __bf16*)w, dx);
   return launched(&ctx->c, "conv_in_dgrad kernel");
 }
@@ -713,18 +824,12 @@ int sk_conv_wgrad(sk_ctx* ctx, int kind, int B, int H, int W, const void* g, con
     return fail(c, SK_EINVAL, "conv_wgrad: bad arguments");
   hipStream_t s = (hipStream_t)stream;
   const long ntiles = (long)((W + CT - 1) / CT) * ((H + CT - 1) / CT) * B;
-  long cap = 1024;
-  if (kind == 1) {  // the MFMA kernel: one resident set of blocks (queried once per device)
-    static int wg_resident[64] = {0};
-    const int dev = c->device < 64 ? c->device : 63;
-    if (!wg_resident[dev]) {
-      int cus = 0, per_cu = 0;
-      SK_HIP(c, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device));
-      SK_HIP(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_wgrad32_mfma, 256, 0));
-      wg_resident[dev] = std::max(1, cus * std::max(1, per_cu));
-    }
-    cap = wg_resident[dev];
-  }
+  // one resident set of blocks, each with one partial (queried once per device)
+  static int cus[64] = {0};
+  const int dev = c->device < 64 ? c->device : 63;
+  if (!cus[dev])
+    SK_HIP(c, hipDeviceGetAttribute(&cus[dev], hipDeviceAttributeMultiprocessorCount, c->device));
+  const long cap = kind == 1 ? 2L * cus[dev] : 4L * cus[dev];
   const int nblocks = (int)std::min<long>(ntiles, cap);
   const int nout = kind == 0 ? NCH * 9 + NCH
                              : (kind == 1 ? NCH * 9 * NCH + NCH : (kind == 2 ? 9 * NCH + 1 : NCH * 9 * 2 + NCH));
@@ -734,17 +839,23 @@ int sk_conv_wgrad(sk_ctx* ctx, int kind, int B, int H, int W, const void* g, con
   float* part = (float*)ws;
   const __bf16* Mk = (const __bf16*)mask;
   if (kind == 0)
-    hipLaunchKernelGGL((k_wgrad<NCH, 1>), dim3(nblocks), dim3(256), 0, s, H, W, B, g, Mk, x, part);
+    hipLaunchKernelGGL((k_wgrad_thin<1, false>), dim3(nblocks), dim3(256), 0, s, H, W, B, (const __bf16*)g, Mk,
+                       (const float*)x, part);
   else if (kind == 1)
-    hipLaunchKernelGGL(k_wgrad32_mfma, dim3(nblocks), dim3(256), 0, s, H, W, B, (const __bf16*)g, Mk,
+    hipLaunchKernelGGL(k_wgrad32_mfma, dim3(nblocks), dim3(WG_T), 0, s, H, W, B, (const __bf16*)g, Mk,
                        (const __bf16*)x, part);
   else if (kind == 2)
-    hipLaunchKernelGGL((k_wgrad<1, NCH>), dim3(nblocks), dim3(256), 0, s, H, W, B, g, Mk, x, part);
+    hipLaunchKernelGGL((k_wgrad_thin<1, true>), dim3(nblocks), dim3(256), 0, s, H, W, B, (const __bf16*)x,
+                       (const __bf16*)nullptr, (const float*)g, part);
   else
-    hipLaunchKernelGGL((k_wgrad<NCH, 2>), dim3(nblocks), dim3(256), 0, s, H, W, B, g, Mk, x, part);
+    hipLaunchKernelGGL((k_wgrad_thin<2, false>), dim3(nblocks), dim3(256), 0, s, H, W, B, (const __bf16*)g, Mk,
+                       (const float*)x, part);
   rc = launched(c, "wgrad kernel");
   if (rc) return rc;
-  hipLaunchKernelGGL(k_reduce_partials, dim3((nout + 63) / 64), dim3(256), 0, s, part, nblocks, nout, out);
+  if (nout > 1024)
+    hipLaunchKernelGGL(k_reduce_partials<64>, dim3((nout + 63) / 64), dim3(1024), 0, s, part, nblocks, nout, out);
+  else
+    hipLaunchKernelGGL(k_reduce_partials<16>, dim3((nout + 15) / 16), dim3(1024), 0, s, part, nblocks, nout, out);
   return launched(c, "partials reduction kernel");
 }
 
