@@ -194,6 +194,15 @@ int sk_conv_in_dgrad(sk_ctx* ctx, int B, int H, int W, const void* dh, const voi
 /* Data gradient of sk_conv_in2: dx2 [B][H][W][2]. */
 int sk_conv_in2_dgrad(sk_ctx* ctx, int B, int H, int W, const void* dh, const void* hmask,
                       const void* w, float* dx2, void* stream);
+/* The same data gradients with the ReLU derivative of the layer below in the output, so that the
+ * kernels that read it next need no mask: dh (BF16) is zeroed where h, that layer's activation, is
+ * <= 0.  sk_conv_in_dgrad_relu takes such a gradient g: dx[_2] [B][H][W][cin], cin 1 or 2. */
+int sk_conv_out_dgrad_relu(sk_ctx* ctx, int B, int H, int W, const float* g, const void* w, const void* h,
+                           void* dh, void* stream);
+int sk_conv32_dgrad_relu(sk_ctx* ctx, int B, int H, int W, const void* g, const void* w, const void* h,
+                         void* dh, void* stream);
+int sk_conv_in_dgrad_relu(sk_ctx* ctx, int cin, int B, int H, int W, const void* g, const void* w, float* dx,
+                          void* stream);
 /* Weight and bias gradients (FP32, deterministic): kind 0 = conv1, 1 = conv2/conv3 (on MFMA),
  * 2 = conv4, 3 = conv1 with two input channels (x = [B][H][W][2] FP32).  out = Cout*9*Cin weight
  * gradients then Cout bias gradients. */

@@ -57,6 +57,9 @@ SIGNATURES = {
     "sk_conv_out_dgrad": (_i, [_vp, _i, _i, _i, _vp, _vp, _vp, _vp]),
     "sk_conv_in_dgrad": (_i, [_vp, _i, _i, _i, _vp, _vp, _vp, _vp, _vp]),
     "sk_conv_in2_dgrad": (_i, [_vp, _i, _i, _i, _vp, _vp, _vp, _vp, _vp]),
+    "sk_conv_out_dgrad_relu": (_i, [_vp, _i, _i, _i, _vp, _vp, _vp, _vp, _vp]),
+    "sk_conv32_dgrad_relu": (_i, [_vp, _i, _i, _i, _vp, _vp, _vp, _vp, _vp]),
+    "sk_conv_in_dgrad_relu": (_i, [_vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp]),
     "sk_conv_wgrad": (_i, [_vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp]),
     "sk_phantoms": (_i, [_vp, _i, _i, _i, _vp, _vp, _vp]),
     "sk_sparse_build": (_i, [_vp, _vp, _i, ctypes.POINTER(_vp), _vp]),

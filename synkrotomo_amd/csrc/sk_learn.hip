@@ -52,12 +52,15 @@ constexpr int NCH = 32;   // hidden channels
 constexpr int PATCH_Q = (CT + 2) * (CT + 2) * 4;      // 16-byte quads of a patch
 constexpr int PATCH_PER_T = (PATCH_Q + 255) / 256;    // per thread
 
-template <bool MASK_IN, bool BIAS_RELU>
+// MASK_OUT: y is zeroed where omask <= 0 (the gradient of the pre-activation of the layer below, so
+// that none of its readers needs the mask again).
+template <bool MASK_IN, bool BIAS_RELU, bool MASK_OUT = false>
 __global__ __launch_bounds__(256) void k_conv32(int H, int W, long ntiles, const __bf16* __restrict__ x,
                                                 const __bf16* __restrict__ mask,
                                                 const __bf16* __restrict__ w,
                                                 const float* __restrict__ bias,
-                                                __bf16* __restrict__ y) {
+                                                __bf16* __restrict__ y,
+                                                const __bf16* __restrict__ omask = nullptr) {
   __shared__ __attribute__((aligned(16))) __bf16 sx[(CT + 2) * (CT + 2) * CP];
   __shared__ __attribute__((aligned(16))) __bf16 sw[NCH * 9 * CP];
   const int tiles_x = (W + CT - 1) / CT;
@@ -110,6 +113,16 @@ __global__ __launch_bounds__(256) void k_conv32(int H, int W, long ntiles, const
     const int r = (int)(t - b * tiles_img);
     const int tx0 = (r % tiles_x) * CT, ty0 = (r / tiles_x) * CT;
     const size_t img = (size_t)b * H * W;
+    [[maybe_unused]] bf16x4 om[4][2];
+    if constexpr (MASK_OUT) {
+#pragma unroll
+      for (int mb = 0; mb < 4; ++mb) {
+        const int oy = min(ty0 + wv * 4 + mb, H - 1), ox = min(tx0 + m, W - 1);  // in bounds; used where written
+#pragma unroll
+        for (int nb = 0; nb < 2; ++nb)
+          om[mb][nb] = *(const bf16x4*)(omask + (img + (size_t)oy * W + ox) * NCH + nb * 16 + 4 * kq);
+      }
+    }
     f32x4 acc[4][2];
     for (int a = 0; a < 4; ++a)
       for (int c = 0; c < 2; ++c) acc[a][c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -142,6 +155,7 @@ __global__ __launch_bounds__(256) void k_conv32(int H, int W, long ntiles, const
         for (int i = 0; i < 4; ++i) {
           float v = acc[mb][nb][i];
           if constexpr (BIAS_RELU) v = fmaxf(v + bias[co + i], 0.0f);
+          if constexpr (MASK_OUT) v = (float)om[mb][nb][i] > 0.0f ? v : 0.0f;
           o[i] = (__bf16)v;
         }
         *(bf16x4*)(y + (img + (size_t)oy * W + ox) * NCH + co) = o;
@@ -262,44 +276,75 @@ __global__ __launch_bounds__(256) void k_conv_out_mfma(int H, int W, const __bf1
   y[p] = res[p] + (sum + bias[0]);
 }
 
-// d h[q][ci] = sum_t w[t][ci] g[q - off_t]   (data gradient of the 32 -> 1 layer)
+// d h[q][ci] = sum_t w[t][ci] g[q - off_t]   (data gradient of the 32 -> 1 layer), zeroed where h <= 0
+// with MASK_OUT.  The block's 256 x 32 BF16 outputs go out through LDS (and its mask comes in the
+// same order): every store instruction writes 1 KB of consecutive bytes.
+template <bool MASK_OUT>
 __global__ __launch_bounds__(256) void k_conv_out_dgrad(int H, int W, long npix, const float* __restrict__ g,
                                                         const __bf16* __restrict__ w,
-                                                        __bf16* __restrict__ dh) {
+                                                        __bf16* __restrict__ dh,
+                                                        const __bf16* __restrict__ h) {
   __shared__ float sw[9 * NCH];
+  __shared__ bf16x8 st[256 * 4];
   for (int i = threadIdx.x; i < 9 * NCH; i += 256) sw[i] = (float)w[i];
+  const long p0 = (long)blockIdx.x * 256;
+  const int n = (int)min(256L, npix - p0) * 4;  // 16-byte chunks of this block's pixels
+  [[maybe_unused]] bf16x8 mk[4];
+  if constexpr (MASK_OUT) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int c = threadIdx.x + 256 * k;
+      mk[k] = ((const bf16x8*)(h + p0 * NCH))[c < n ? c : 0];
+    }
+  }
   __syncthreads();
-  const long p = (long)blockIdx.x * 256 + threadIdx.x;
-  if (p >= npix) return;
+  const long p = p0 + threadIdx.x;
   const long b = p / ((long)H * W);
   const int r = (int)(p - b * H * W);
   const int py = r / W, px = r - py * W;
   float gv[9];
+#pragma unroll
   for (int t = 0; t < 9; ++t) {
     const int yy = py - (t / 3 - 1), xx = px - (t % 3 - 1);
-    gv[t] = (yy >= 0 && yy < H && xx >= 0 && xx < W) ? g[(b * H + yy) * W + xx] : 0.0f;
+    gv[t] = (p < npix && yy >= 0 && yy < H && xx >= 0 && xx < W) ? g[(b * H + yy) * W + xx] : 0.0f;
   }
-  __bf16* out = dh + p * NCH;
+#pragma unroll
   for (int q = 0; q < 4; ++q) {
     bf16x8 o;
+#pragma unroll
     for (int i = 0; i < 8; ++i) {
       const int ci = q * 8 + i;
       float s = 0.0f;
+#pragma unroll
       for (int t = 0; t < 9; ++t) s = fmaf(sw[t * NCH + ci], gv[t], s);
       o[i] = (__bf16)s;
     }
-    *(bf16x8*)(out + q * 8) = o;
+    st[threadIdx.x * 4 + q] = o;
+  }
+  __syncthreads();
+  bf16x8* out = (bf16x8*)(dh + p0 * NCH);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int c = threadIdx.x + 256 * k;
+    if (c >= n) continue;
+    bf16x8 o = st[c];
+    if constexpr (MASK_OUT) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        if (!((float)mk[k][i] > 0.0f)) o[i] = (__bf16)0.0f;
+    }
+    out[c] = o;
   }
 }
 
-// dx[q][c] = sum_{t,co} w[co][t][c] g1[q - off_t][co],  g1 = dh * (h > 0)   (data gradient of
+// dx[q][c] = sum_{t,co} w[co][t][c] g1[q - off_t][co],  g1 = dh * (h > 0) (MASK) or dh   (data gradient of
 // k_conv_in; dx FP32 [B][H][W][CIN]).  As k_conv_out_mfma: per 16x16 tile and input channel c, each
 // of the 18x18 halo pixels of g1 gets U[p][t] = sum_co g1[p][co] w[co][t][c] for the 9 taps in one
 // MFMA per 16 pixels (products of BF16 values, exact in the FP32 accumulator's input), then each
 // output sums its 9 shifted taps.  Bound by the two activation streams: 8 x 512^2, 1.21 times 134 MB
 // each, 69 us = 4.7 TB/s (on VALU with one thread per pixel re-reading every neighbour's 32
-// channels: 851 us).
-template <int CIN>
+// channels: 851 us); 31 us for a gradient that needs no mask.
+template <int CIN, bool MASK>
 __global__ __launch_bounds__(256) void k_conv_in_dgrad(int H, int W, const __bf16* __restrict__ dh,
                                                        const __bf16* __restrict__ hmask,
                                                        const __bf16* __restrict__ w,
@@ -321,10 +366,15 @@ __global__ __launch_bounds__(256) void k_conv_in_dgrad(int H, int W, const __bf1
     for (int i = 0; i < 8; ++i) a[k][i] = (__bf16)0.0f;
     if (slot < (CT + 2) * (CT + 2) && gy >= 0 && gy < H && gx >= 0 && gx < W) {
       const size_t off = (img + (size_t)gy * W + gx) * NCH + 8 * kq;
-      const bf16x8 g = *(const bf16x8*)(dh + off), mk = *(const bf16x8*)(hmask + off);
+      const bf16x8 g = *(const bf16x8*)(dh + off);
+      if constexpr (MASK) {
+        const bf16x8 mk = *(const bf16x8*)(hmask + off);
 #pragma unroll
-      for (int i = 0; i < 8; ++i)
-        if ((float)mk[i] > 0.0f) a[k][i] = g[i];
+        for (int i = 0; i < 8; ++i)
+          if ((float)mk[i] > 0.0f) a[k][i] = g[i];
+      } else {
+        a[k] = g;
+      }
     }
   }
   const int ty = threadIdx.x >> 4, tx = threadIdx.x & 15;
@@ -366,8 +416,8 @@ __global__ __launch_bounds__(256) void k_conv_in_dgrad(int H, int W, const __bf1
 // A wave walks 16x4 pixels of a 16x16 tile at a time: lane l holds channels 2(l%16) and +1 of row
 // l/16, so a pixel's V is one coalesced dword per lane and its 9 F values are read from LDS rows
 // into registers once per tile row; sums stay in registers over all of the block's tiles.
-// 8 x 512^2: 109 us for conv1 (V and M, 268 MB) and 39 us for conv4 (134 MB); one weight per thread
-// over LDS tiles: 236 and 195 us.
+// 8 x 512^2 (134 MB of V): 41 us for either without M, 109 us with it; one weight per thread over
+// LDS tiles: 195 and 236 us.
 template <int CI, bool TAIL>
 __global__ __launch_bounds__(256) void k_wgrad_thin(int H, int W, int B, const __bf16* __restrict__ V,
                                                     const __bf16* __restrict__ M, const float* __restrict__ F,
@@ -379,6 +429,7 @@ __global__ __launch_bounds__(256) void k_wgrad_thin(int H, int W, int B, const _
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int cp = lane & 15, sub = lane >> 4;
   float acc[CI][2][9], accb[2] = {0.0f, 0.0f};
+  double sum_f = 0.0;  // TAIL: a sum of one sign-changing value per pixel, the one output without BF16 factors
 #pragma unroll
   for (int c = 0; c < CI; ++c)
 #pragma unroll
@@ -430,16 +481,26 @@ __global__ __launch_bounds__(256) void k_wgrad_thin(int H, int W, int B, const _
           acc[c][0][t] = fmaf(v0, f[t / 3][x + t % 3], acc[c][0][t]);
           acc[c][1][t] = fmaf(v1, f[t / 3][x + t % 3], acc[c][1][t]);
         }
-        if (c == 0) {
-          if constexpr (TAIL) {  // the tile's own pixels of F (0 outside the image)
-            accb[0] += (gy < H && tx0 + x < W) ? f[1][x + 1] : 0.0f;
-          } else {
-            accb[0] += v0;
-            accb[1] += v1;
-          }
+        if (!TAIL && c == 0) {
+          accb[0] += v0;
+          accb[1] += v1;
         }
       }
+      if constexpr (TAIL) {  // the row's own 16 pixels of F, in pairs, then to the FP64 sum
+        float r[CT];
+#pragma unroll
+        for (int x = 0; x < CT; ++x) r[x] = (gy < H && tx0 + x < W) ? f[1][x + 1] : 0.0f;
+#pragma unroll
+        for (int n = CT / 2; n > 0; n >>= 1)
+#pragma unroll
+          for (int x = 0; x < n; ++x) r[x] += r[x + n];
+        sum_f += (double)r[0];
+      }
     }
+  }
+  if constexpr (TAIL) {
+    sum_f += __shfl_xor(sum_f, 16);
+    sum_f += __shfl_xor(sum_f, 32);
   }
   // the wave's four rows ((0 + 1) + (2 + 3)), then the waves in order
   auto rows = [](float v) {
@@ -448,7 +509,7 @@ __global__ __launch_bounds__(256) void k_wgrad_thin(int H, int W, int B, const _
   };
 #pragma unroll
   for (int k = 0; k < 2; ++k) {
-    accb[k] = rows(accb[k]);
+    accb[k] = TAIL ? (float)sum_f : rows(accb[k]);
 #pragma unroll
     for (int c = 0; c < CI; ++c)
 #pragma unroll
@@ -489,7 +550,7 @@ __global__ __launch_bounds__(256) void k_wgrad_thin(int H, int W, int B, const _
 // of its block (two pixel rows per step: lane group kq holds row 2s + kq/2, columns 8(kq%2) .. +7).
 // The next tile is loaded into registers during this one's MFMAs.  At the end the two waves of a
 // channel block are added and the block writes one partial (deterministic).
-// 8 x 512^2: 102 us for the three streams' 400 MB = 3.9 TB/s (16-bit transposing stores of three
+// 8 x 512^2: 82 us for the two streams' 268 MB, 102 us with M (16-bit transposing stores of three
 // shifted copies: 280 us).
 constexpr int WG_NOUT = NCH * 9 * NCH + NCH;
 constexpr int WG_T = 512;                                       // threads
@@ -642,10 +703,10 @@ template <int OUTS>
 __global__ __launch_bounds__(1024) void k_reduce_partials(const float* __restrict__ partials, int nblocks,
                                                           int nout, float* __restrict__ out) {
   constexpr int STR = 1024 / OUTS;
-  __shared__ float sh[STR][OUTS];
+  __shared__ double sh[STR][OUTS];
   const int c = threadIdx.x % OUTS, r = threadIdx.x / OUTS;
   const int o = blockIdx.x * OUTS + c;
-  float s = 0.0f;
+  double s = 0.0;  // FP64: the sums of a bias gradient cancel, and the adds hide behind the loads
   if (o < nout) {
     int b = r;
     for (; b + 7 * STR < nblocks; b += 8 * STR) {
@@ -653,16 +714,16 @@ __global__ __launch_bounds__(1024) void k_reduce_partials(const float* __restric
 #pragma unroll
       for (int k = 0; k < 8; ++k) v[k] = partials[(size_t)(b + k * STR) * nout + o];
 #pragma unroll
-      for (int k = 0; k < 8; ++k) s += v[k];
+      for (int k = 0; k < 8; ++k) s += (double)v[k];
     }
-    for (; b < nblocks; b += STR) s += partials[(size_t)b * nout + o];
+    for (; b < nblocks; b += STR) s += (double)partials[(size_t)b * nout + o];
   }
   sh[r][c] = s;
   __syncthreads();
   if (r == 0 && o < nout) {
-    float t = sh[0][c];
+    double t = sh[0][c];
     for (int k = 1; k < STR; ++k) t += sh[k][c];
-    out[o] = t;
+    out[o] = (float)t;
   }
 }
 
@@ -701,8 +762,8 @@ static int check_ctx(sk_ctx* ctx) {
 
 extern "C" {
 
-int sk_conv32(sk_ctx* ctx, int B, int H, int W, const void* x, const void* mask, const void* w,
-              const float* bias, void* y, void* stream) {
+static int conv32_go(sk_ctx* ctx, int B, int H, int W, const void* x, const void* mask, const void* w,
+                     const float* bias, void* y, const void* omask, void* stream) {
   int rc = check_ctx(ctx);
   if (rc) return rc;
   if (B < 1 || B > 65535 || H < 1 || W < 1 || !x || !w || !y)
@@ -720,17 +781,30 @@ int sk_conv32(sk_ctx* ctx, int B, int H, int W, const void* x, const void* mask,
   const long resident = (long)cus[dev] * per_cu[dev];
   dim3 grid((unsigned)std::min(ntiles, resident));
   hipStream_t s = (hipStream_t)stream;
-  const __bf16 *X = (const __bf16*)x, *Mk = (const __bf16*)mask, *Wt = (const __bf16*)w;
+  const __bf16 *X = (const __bf16*)x, *Mk = (const __bf16*)mask, *Wt = (const __bf16*)w, *Om = (const __bf16*)omask;
   __bf16* Y = (__bf16*)y;
-  if (mask && relu)
-    hipLaunchKernelGGL((k_conv32<true, true>), grid, dim3(256), 0, s, H, W, ntiles, X, Mk, Wt, bias, Y);
+  if (omask)
+    hipLaunchKernelGGL((k_conv32<false, false, true>), grid, dim3(256), 0, s, H, W, ntiles, X, Mk, Wt, bias, Y, Om);
+  else if (mask && relu)
+    hipLaunchKernelGGL((k_conv32<true, true>), grid, dim3(256), 0, s, H, W, ntiles, X, Mk, Wt, bias, Y, Om);
   else if (mask)
-    hipLaunchKernelGGL((k_conv32<true, false>), grid, dim3(256), 0, s, H, W, ntiles, X, Mk, Wt, bias, Y);
+    hipLaunchKernelGGL((k_conv32<true, false>), grid, dim3(256), 0, s, H, W, ntiles, X, Mk, Wt, bias, Y, Om);
   else if (relu)
-    hipLaunchKernelGGL((k_conv32<false, true>), grid, dim3(256), 0, s, H, W, ntiles, X, Mk, Wt, bias, Y);
+    hipLaunchKernelGGL((k_conv32<false, true>), grid, dim3(256), 0, s, H, W, ntiles, X, Mk, Wt, bias, Y, Om);
   else
-    hipLaunchKernelGGL((k_conv32<false, false>), grid, dim3(256), 0, s, H, W, ntiles, X, Mk, Wt, bias, Y);
+    hipLaunchKernelGGL((k_conv32<false, false>), grid, dim3(256), 0, s, H, W, ntiles, X, Mk, Wt, bias, Y, Om);
   return launched(&ctx->c, "conv32 kernel");
+}
+
+int sk_conv32(sk_ctx* ctx, int B, int H, int W, const void* x, const void* mask, const void* w,
+              const float* bias, void* y, void* stream) {
+  return conv32_go(ctx, B, H, W, x, mask, w, bias, y, nullptr, stream);
+}
+
+int sk_conv32_dgrad_relu(sk_ctx* ctx, int B, int H, int W, const void* g, const void* w, const void* h, void* dh,
+                         void* stream) {
+  if (ctx && !h) return fail(&ctx->c, SK_EINVAL, "conv32_dgrad_relu: bad arguments");
+  return conv32_go(ctx, B, H, W, g, nullptr, w, nullptr, dh, h, stream);
 }
 
 static int conv_in_go(sk_ctx* ctx, int cin, int B, int H, int W, const float* x, const void* w, const float* bias,
@@ -773,41 +847,67 @@ int sk_conv_out(sk_ctx* ctx, int B, int H, int W, const void* h, const void* w, 
   return launched(&ctx->c, "conv_out kernel");
 }
 
-int sk_conv_out_dgrad(sk_ctx* ctx, int B, int H, int W, const float* g, const void* w, void* dh,
-                      void* stream) {
+static int conv_out_dgrad_go(sk_ctx* ctx, int B, int H, int W, const float* g, const void* w, const void* h,
+                             void* dh, void* stream) {
   int rc = check_ctx(ctx);
   if (rc) return rc;
   if (B < 1 || H < 1 || W < 1 || !g || !w || !dh) return fail(&ctx->c, SK_EINVAL, "conv_out_dgrad: bad arguments");
   const long npix = (long)B * H * W;
-  hipLaunchKernelGGL(k_conv_out_dgrad, dim3((unsigned)((npix + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
-                     H, W, npix, g, (const __bf16*)w, (__bf16*)dh);
+  const dim3 grid((unsigned)((npix + 255) / 256));
+  if (h)
+    hipLaunchKernelGGL(k_conv_out_dgrad<true>, grid, dim3(256), 0, (hipStream_t)stream, H, W, npix, g,
+                       (const __bf16*)w, (__bf16*)dh, (const __bf16*)h);
+  else
+    hipLaunchKernelGGL(k_conv_out_dgrad<false>, grid, dim3(256), 0, (hipStream_t)stream, H, W, npix, g,
+                       (const __bf16*)w, (__bf16*)dh, (const __bf16*)nullptr);
   return launched(&ctx->c, "conv_out_dgrad kernel");
 }
 
+int sk_conv_out_dgrad(sk_ctx* ctx, int B, int H, int W, const float* g, const void* w, void* dh,
+                      void* stream) {
+  return conv_out_dgrad_go(ctx, B, H, W, g, w, nullptr, dh, stream);
+}
+
+int sk_conv_out_dgrad_relu(sk_ctx* ctx, int B, int H, int W, const float* g, const void* w, const void* h, void* dh,
+                           void* stream) {
+  if (ctx && !h) return fail(&ctx->c, SK_EINVAL, "conv_out_dgrad_relu: bad arguments");
+  return conv_out_dgrad_go(ctx, B, H, W, g, w, h, dh, stream);
+}
+
+}  // extern "C"
+
+template <bool MASK>
 static int conv_in_dgrad_go(sk_ctx* ctx, int cin, int B, int H, int W, const void* dh, const void* hmask,
                             const void* w, float* dx, void* stream) {
   int rc = check_ctx(ctx);
   if (rc) return rc;
-  if (B < 1 || H < 1 || W < 1 || !dh || !hmask || !w || !dx)
+  if (cin < 1 || cin > 2 || B < 1 || H < 1 || W < 1 || !dh || (MASK && !hmask) || !w || !dx)
     return fail(&ctx->c, SK_EINVAL, "conv_in_dgrad: bad arguments");
   const dim3 grid((unsigned)((long)((W + CT - 1) / CT) * ((H + CT - 1) / CT) * B));
   if (cin == 1)
-    hipLaunchKernelGGL(k_conv_in_dgrad<1>, grid, dim3(256), 0, (hipStream_t)stream, H, W, (const __bf16*)dh,
+    hipLaunchKernelGGL((k_conv_in_dgrad<1, MASK>), grid, dim3(256), 0, (hipStream_t)stream, H, W, (const __bf16*)dh,
                        (const __bf16*)hmask, (const __bf16*)w, dx);
   else
-    hipLaunchKernelGGL(k_conv_in_dgrad<2>, grid, dim3(256), 0, (hipStream_t)stream, H, W, (const __bf16*)dh,
+    hipLaunchKernelGGL((k_conv_in_dgrad<2, MASK>), grid, dim3(256), 0, (hipStream_t)stream, H, W, (const __bf16*)dh,
                        (const __bf16*)hmask, (const __bf16*)w, dx);
   return launched(&ctx->c, "conv_in_dgrad kernel");
 }
 
+extern "C" {
+
 int sk_conv_in_dgrad(sk_ctx* ctx, int B, int H, int W, const void* dh, const void* hmask,
                      const void* w, float* dx, void* stream) {
-  return conv_in_dgrad_go(ctx, 1, B, H, W, dh, hmask, w, dx, stream);
+  return conv_in_dgrad_go<true>(ctx, 1, B, H, W, dh, hmask, w, dx, stream);
 }
 
 int sk_conv_in2_dgrad(sk_ctx* ctx, int B, int H, int W, const void* dh, const void* hmask,
                       const void* w, float* dx2, void* stream) {
-  return conv_in_dgrad_go(ctx, 2, B, H, W, dh, hmask, w, dx2, stream);
+  return conv_in_dgrad_go<true>(ctx, 2, B, H, W, dh, hmask, w, dx2, stream);
+}
+
+int sk_conv_in_dgrad_relu(sk_ctx* ctx, int cin, int B, int H, int W, const void* g, const void* w, float* dx,
+                          void* stream) {
+  return conv_in_dgrad_go<false>(ctx, cin, B, H, W, g, nullptr, w, dx, stream);
 }
 
 // kind 0: conv1 (G = 32-ch gradient masked by h1, X = fp32 image) -> dW [32][9], db [32]

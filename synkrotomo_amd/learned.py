@@ -95,31 +95,30 @@ class _Correction(torch.autograd.Function):
         B, H, W = gy.shape
         dev = gy.device
 
-        def wgrad(kind, g, mask, x, n):
+        def wgrad(kind, g, x, n):
             out = torch.empty(n, dtype=torch.float32, device=dev)
-            _chk(L.sk_conv_wgrad(h, kind, B, H, W, _ptr(g), None if mask is None else _ptr(mask),
-                                 _ptr(x), _ptr(out), s), ctx, "wgrad")
+            _chk(L.sk_conv_wgrad(h, kind, B, H, W, _ptr(g), None, _ptr(x), _ptr(out), s), ctx, "wgrad")
             return out
 
-        # conv4 (32 -> 1, residual)
-        g4 = wgrad(2, gy, None, h3, 9 * NCH + 1)
+        # conv4 (32 -> 1, residual); each activation gradient is written as the gradient of the
+        # pre-activation (dh * (h > 0)), which is what its weight and data gradients read
+        g4 = wgrad(2, gy, h3, 9 * NCH + 1)
         dh3 = torch.empty_like(h3)
-        _chk(L.sk_conv_out_dgrad(h, B, H, W, _ptr(gy), _ptr(w4b), _ptr(dh3), s), ctx, "conv4 dgrad")
-        # conv3, conv2 (32 -> 32): gradient wrt the pre-activation = dh * (h > 0)
-        g3 = wgrad(1, dh3, h3, h2, NCH * 9 * NCH + NCH)
+        _chk(L.sk_conv_out_dgrad_relu(h, B, H, W, _ptr(gy), _ptr(w4b), _ptr(h3), _ptr(dh3), s), ctx, "conv4 dgrad")
+        # conv3, conv2 (32 -> 32)
+        g3 = wgrad(1, dh3, h2, NCH * 9 * NCH + NCH)
         w3t = w3b.flip(1, 2).permute(3, 1, 2, 0).contiguous()
         dh2 = torch.empty_like(h2)
-        _chk(L.sk_conv32(h, B, H, W, _ptr(dh3), _ptr(h3), _ptr(w3t), None, _ptr(dh2), s), ctx, "conv3 dgrad")
-        g2 = wgrad(1, dh2, h2, h1, NCH * 9 * NCH + NCH)
+        _chk(L.sk_conv32_dgrad_relu(h, B, H, W, _ptr(dh3), _ptr(w3t), _ptr(h2), _ptr(dh2), s), ctx, "conv3 dgrad")
+        g2 = wgrad(1, dh2, h1, NCH * 9 * NCH + NCH)
         w2t = w2b.flip(1, 2).permute(3, 1, 2, 0).contiguous()
         dh1 = torch.empty_like(h1)
-        _chk(L.sk_conv32(h, B, H, W, _ptr(dh2), _ptr(h2), _ptr(w2t), None, _ptr(dh1), s), ctx, "conv2 dgrad")
+        _chk(L.sk_conv32_dgrad_relu(h, B, H, W, _ptr(dh2), _ptr(w2t), _ptr(h1), _ptr(dh1), s), ctx, "conv2 dgrad")
         # conv1 (cin -> 32)
         n1 = NCH * 9 * cin
-        g1 = wgrad(0 if cin == 1 else 3, dh1, h1, inp, n1 + NCH)
+        g1 = wgrad(0 if cin == 1 else 3, dh1, inp, n1 + NCH)
         dinp = torch.empty_like(inp)
-        dgrad = L.sk_conv_in_dgrad if cin == 1 else L.sk_conv_in2_dgrad
-        _chk(dgrad(h, B, H, W, _ptr(dh1), _ptr(h1), _ptr(w1b), _ptr(dinp), s), ctx, "conv1 dgrad")
+        _chk(L.sk_conv_in_dgrad_relu(h, cin, B, H, W, _ptr(dh1), _ptr(w1b), _ptr(dinp), s), ctx, "conv1 dgrad")
         n2, n4 = NCH * 9 * NCH, 9 * NCH
         gw1 = g1[:n1].view(NCH, 3, 3) if cin == 1 else g1[:n1].view(NCH, 3, 3, cin)
         return (dinp, gy, gw1, g1[n1:], g2[:n2].view(NCH, 3, 3, NCH), g2[n2:],

@@ -55,3 +55,30 @@ def test_first_layers_data_gradient_is_exact_on_integers(ctx, B, H, W, cin):
     g1 = dh.double() * (mask > 0)
     ref = sum(_shifted(g1, 8 - t).reshape(-1, 32) @ w[:, t].double() for t in range(9))
     assert torch.equal(dx.double().reshape(-1, cin), ref)
+
+
+@pytest.mark.parametrize("B,H,W", SIZES)
+def test_masked_data_gradients_equal_masking_afterwards(ctx, B, H, W):
+    """The gradients written with the ReLU derivative of the layer below are, bit for bit, the plain
+    ones masked; and the first layer's from such a gradient is the one that masks it itself."""
+    from synkrotomo_amd import _native as nat
+    from synkrotomo_amd.projector import _ptr, _stream
+    L, c, st = nat.lib(), ctx.handle, _stream(ctx.device)
+    gen = torch.Generator(device="cuda").manual_seed(W)
+    rnd = lambda *shape: torch.randn(shape, device="cuda", generator=gen)  # noqa: E731
+    h = torch.relu(rnd(B, H, W, 32)).to(torch.bfloat16)
+    zero = torch.zeros((), dtype=torch.bfloat16, device="cuda")
+    g, w4 = rnd(B, H, W), rnd(9, 32).to(torch.bfloat16)
+    a, b = torch.empty_like(h), torch.empty_like(h)
+    nat.check(L.sk_conv_out_dgrad(c, B, H, W, _ptr(g), _ptr(w4), _ptr(a), st), c)
+    nat.check(L.sk_conv_out_dgrad_relu(c, B, H, W, _ptr(g), _ptr(w4), _ptr(h), _ptr(b), st), c)
+    assert torch.equal(torch.where(h > 0, a, zero), b)
+    x, w = rnd(B, H, W, 32).to(torch.bfloat16), rnd(32, 9, 32).to(torch.bfloat16)
+    nat.check(L.sk_conv32(c, B, H, W, _ptr(x), None, _ptr(w), None, _ptr(a), st), c)
+    nat.check(L.sk_conv32_dgrad_relu(c, B, H, W, _ptr(x), _ptr(w), _ptr(h), _ptr(b), st), c)
+    assert torch.equal(torch.where(h > 0, a, zero), b)
+    w1 = rnd(32, 9).to(torch.bfloat16)
+    d0, d1 = torch.empty_like(g), torch.empty_like(g)
+    nat.check(L.sk_conv_in_dgrad(c, B, H, W, _ptr(a), _ptr(h), _ptr(w1), _ptr(d0), st), c)
+    nat.check(L.sk_conv_in_dgrad_relu(c, 1, B, H, W, _ptr(b), _ptr(w1), _ptr(d1), st), c)
+    assert torch.equal(d0, d1)
