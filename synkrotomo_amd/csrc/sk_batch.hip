@@ -5,7 +5,7 @@
 // the slices of one geometry): a problem set holds groups of independent problems, each
 // group with its own geometry (image size, angles, bins).  One iteration is two persistent
 // launches sized to fill the chip once: in k_fpg_persist (fast mode) every workgroup pulls
-// (problem, image, line group, 64-bin block) items of the grouped staged forward projector
+// (problem, images, line group, 64-bin block) items of the grouped staged forward projector
 // from a global work counter (k_fps_persist: (problem, image, line, 256-bin block) items of
 // the one-line staged kernel) (k_fp_persist: waves pull 64-bin items of the per-wave walk, exact mode or
 // segments wider than the staging buffer); in k_bp_persist every block pulls (problem,
@@ -131,11 +131,11 @@ __global__ __launch_bounds__(FPS_RAYS, 8) void k_fps_persist(const BatchArgs a, 
 }
 
 // Grouped staged forward items (fast mode, every group has a line-group table): one
-// workgroup per item of FPG_BINS bins of one line group of one image, groups fastest, claimed
-// as in k_fps_persist; the per-row step only (the exact per-block step's registers would
-// spill here).  Two buffers of (FPG_ROWS + 1) * 64 * CPL floats of dynamic LDS for the
-// largest CPL of the set.
-__global__ __launch_bounds__(FPS_RAYS, 8) void k_fpg_persist(const BatchArgs a, unsigned* __restrict__ ctr) {
+// workgroup per item of FPG_BINS bins of one line group of S images, groups fastest, claimed
+// as in k_fps_persist.  CPLMAX: the largest chunk count of the set; dynamic LDS: fpg_lds_floats.
+template <int S, int CPLMAX>
+__global__ __launch_bounds__(FPS_RAYS, S == 1 ? 8 : (CPLMAX == 2 ? 5 : 4)) void k_fpg_persist(
+    const BatchArgs a, unsigned* __restrict__ ctr) {
   extern __shared__ float4 seg4[];
   __shared__ unsigned item_sh;
   if (blockIdx.x == 0 && threadIdx.x == 0) ctr[1] = 0u;  // the bp queue of this iteration
@@ -154,18 +154,19 @@ __global__ __launch_bounds__(FPS_RAYS, 8) void k_fpg_persist(const BatchArgs a, 
     const int g = (int)(rem - (long)wb * B.fp_units);
     const int4 grp = B.fp.groups[u32(g)];
     const int cpl = u32(grp.x >> 24);
-    if (cpl <= 2)
-      fpg_item<FP_SIRT, 2, 1, false>(B.fp, grp, u32(wb), u32(bz), (float*)seg4);
-    else if (cpl == 3)
-      fpg_item<FP_SIRT, 3, 1, false>(B.fp, grp, u32(wb), u32(bz), (float*)seg4);
+    if (CPLMAX == 2 || cpl <= 2)
+      fpg_item<FP_SIRT, 2, S, false>(B.fp, grp, u32(wb), u32(bz), (float*)seg4);
+    else if (CPLMAX == 3 || cpl == 3)
+      fpg_item<FP_SIRT, CPLMAX >= 3 ? 3 : 2, S, false>(B.fp, grp, u32(wb), u32(bz), (float*)seg4);
     else
-      fpg_item<FP_SIRT, 4, 1, false>(B.fp, grp, u32(wb), u32(bz), (float*)seg4);
+      fpg_item<FP_SIRT, CPLMAX >= 4 ? 4 : 2, S, false>(B.fp, grp, u32(wb), u32(bz), (float*)seg4);
   }
 }
 
-template <bool EXACT, int NC, bool DR1, int PPT>
+// Tiles of S images (S > 1: 16 x 32 tiles, the hoisted fast path).
+template <bool EXACT, int NC, bool DR1, int PPT, int S>
 __global__ __launch_bounds__(256) void k_bp_persist(const BatchArgs a, unsigned* __restrict__ ctr) {
-  extern __shared__ float2 win[];
+  extern __shared__ float4 win[];
   __shared__ BpLineLds lsh[BP_LB];
   __shared__ unsigned item_sh;
   if (blockIdx.x == 0 && threadIdx.x == 0) ctr[2] = 0u;  // the fp queue of the next iteration
@@ -187,7 +188,7 @@ __global__ __launch_bounds__(256) void k_bp_persist(const BatchArgs a, unsigned*
       tx = (int)(t & 0xffffu);
       ty = (int)(t >> 16);
     }
-    bp_item<EXACT, BP_SIRT, W_REF, NC, DR1, PPT>(B.bp, u32(tx), u32(ty), u32(bz), win, lsh);
+    bp_item<EXACT, BP_SIRT, W_REF, NC, DR1, PPT, S>(B.bp, u32(tx), u32(ty), u32(bz), (float2*)win, lsh);
   }
 }
 
@@ -201,40 +202,89 @@ struct BatchPlan {
   // every group has a line-group table.
   int fp_mode = 2;
   int fpg_cpl = 0;  // mode 5: the largest chunk count of the set's line groups
+  int fp_images = 1;  // images per forward item (mode 5) and per backprojector tile
+  int bp_images = 1;
   int bp_ppt = 4;
   unsigned* d_ctr = nullptr;
   int Wmax = 0;
   bool dr1 = true;
+  int nc = 0;         // candidates per pixel of the hoisted backprojector, 0: the general path
+  const void *kfp = nullptr, *kbp = nullptr;
+  size_t fp_lds = 0, bp_lds = 0;
 };
 
-static size_t fpg_lds(int cpl) { return sizeof(float) * fpg_lds_floats(FpgShape<1>::nbuf, 1, cpl, false); }
+// Pixels per lane of the persistent backprojector for one image at a time (16 x 16*PPT tiles): 4
+// by default (16x64 tiles: 3.11 s vs 3.23 s with 16x32 on the four large groups of the batched
+// configuration, equal on small groups); SYNKRO_BATCH_BP_PPT=2 selects 16x32 tiles.
 
-// Pixels per lane of the persistent backprojector (16 x 16*PPT tiles): 4 by default (16x64
-// tiles: 3.11 s vs 3.23 s with 16x32 on the four large groups of the batched configuration,
-// equal on small groups); SYNKRO_BATCH_BP_PPT=2 selects 16x32 tiles.
+// The kernels of a plan.
+static const void* fp_kernel(const BatchPlan& p, bool ex) {
+  if (p.fp_mode == 5) {
+    const int c = p.fpg_cpl;
+    if (p.fp_images == 4)
+      return c == 2 ? (const void*)k_fpg_persist<4, 2> : (c == 3 ? (const void*)k_fpg_persist<4, 3> : (const void*)k_fpg_persist<4, 4>);
+    if (p.fp_images == 2)
+      return c == 2 ? (const void*)k_fpg_persist<2, 2> : (c == 3 ? (const void*)k_fpg_persist<2, 3> : (const void*)k_fpg_persist<2, 4>);
+    return c == 2 ? (const void*)k_fpg_persist<1, 2> : (c == 3 ? (const void*)k_fpg_persist<1, 3> : (const void*)k_fpg_persist<1, 4>);
+  }
+  if (p.fp_mode == 4) return (const void*)k_fps_persist;
+  const void* exact[4] = {(const void*)k_fp_persist<true, 1, false>, (const void*)k_fp_persist<true, 2, false>,
+                          (const void*)k_fp_persist<true, 1, true>, (const void*)k_fp_persist<true, 2, true>};
+  const void* fast[4] = {(const void*)k_fp_persist<false, 1, false>, (const void*)k_fp_persist<false, 2, false>,
+                         (const void*)k_fp_persist<false, 1, true>, (const void*)k_fp_persist<false, 2, true>};
+  return (ex ? exact : fast)[p.fp_mode & 3];
+}
 
-template <bool EXACT, int NC, bool DR1>
-static int launch_iteration(Ctx* c, const BatchPlan& plan, int fp_grid, int bp_grid, hipStream_t s) {
-  if (plan.fp_mode == 5)
-    hipLaunchKernelGGL(k_fpg_persist, dim3(fp_grid), dim3(FPS_RAYS), fpg_lds(plan.fpg_cpl), s, plan.args,
-                       plan.d_ctr);
-  else if (plan.fp_mode == 4)
-    hipLaunchKernelGGL(k_fps_persist, dim3(fp_grid), dim3(FPS_RAYS), sizeof(float) * FPS_CS * FPS_MAXW, s,
-                       plan.args, plan.d_ctr);
-  else if (plan.fp_mode == 0)
-    hipLaunchKernelGGL((k_fp_persist<EXACT, 1, false>), dim3(fp_grid), dim3(FP_BLOCK), 0, s, plan.args, plan.d_ctr);
-  else if (plan.fp_mode == 1)
-    hipLaunchKernelGGL((k_fp_persist<EXACT, 2, false>), dim3(fp_grid), dim3(FP_BLOCK), 0, s, plan.args, plan.d_ctr);
-  else if (plan.fp_mode == 2)
-    hipLaunchKernelGGL((k_fp_persist<EXACT, 1, true>), dim3(fp_grid), dim3(FP_BLOCK), 0, s, plan.args, plan.d_ctr);
-  else
-    hipLaunchKernelGGL((k_fp_persist<EXACT, 2, true>), dim3(fp_grid), dim3(FP_BLOCK), 0, s, plan.args, plan.d_ctr);
-  const size_t lds = sizeof(float2) * BP_LB * (size_t)plan.Wmax;
-  if (plan.bp_ppt == 4)
-    hipLaunchKernelGGL((k_bp_persist<EXACT, NC, DR1, 4>), dim3(bp_grid), dim3(256), lds, s, plan.args, plan.d_ctr);
-  else
-    hipLaunchKernelGGL((k_bp_persist<EXACT, NC, DR1, 2>), dim3(bp_grid), dim3(256), lds, s, plan.args, plan.d_ctr);
+template <int NC>
+static const void* bp_kernel_nc(const BatchPlan& p) {
+  switch (p.bp_images) {
+    case 8: return (const void*)k_bp_persist<false, NC, false, 2, 8>;
+    case 4: return (const void*)k_bp_persist<false, NC, false, 2, 4>;
+    case 2: return (const void*)k_bp_persist<false, NC, false, 2, 2>;
+    default:
+      return p.bp_ppt == 4 ? (const void*)k_bp_persist<false, NC, false, 4, 1>
+                           : (const void*)k_bp_persist<false, NC, false, 2, 1>;
+  }
+}
+
+static const void* bp_kernel(const BatchPlan& p, bool ex) {
+  if (ex && p.dr1)
+    return p.bp_ppt == 4 ? (const void*)k_bp_persist<true, 2, true, 4, 1> : (const void*)k_bp_persist<true, 2, true, 2, 1>;
+  if (ex)
+    return p.bp_ppt == 4 ? (const void*)k_bp_persist<true, 0, false, 4, 1> : (const void*)k_bp_persist<true, 0, false, 2, 1>;
+  if (p.nc == 2) return bp_kernel_nc<2>(p);
+  if (p.nc > 0) return bp_kernel_nc<4>(p);
+  return p.bp_ppt == 4 ? (const void*)k_bp_persist<false, 0, false, 4, 1> : (const void*)k_bp_persist<false, 0, false, 2, 1>;
+}
+
+static int launch_iteration(Ctx* c, BatchPlan& plan, int fp_grid, int bp_grid, hipStream_t s) {
+  void* args[] = {&plan.args, &plan.d_ctr};
+  SK_HIP(c, hipLaunchKernel(plan.kfp, dim3(fp_grid), dim3(FPS_RAYS), args, plan.fp_lds, s));
+  SK_HIP(c, hipLaunchKernel(plan.kbp, dim3(bp_grid), dim3(256), args, plan.bp_lds, s));
   return launched(c, "persistent SIRT kernels");
+}
+
+// Images per item, of the given sizes, by least total cost: a problem of b images costs ceil(b/S)
+// items, and an item of S images cost[S] of one image's (measured on 64 x 512^2, 512 angles).  A size
+// that leaves the set fewer than two items per CU is not taken: its items only get longer.
+static int images_per_item(const sk_problem* problems, int count, const int* sizes, const double* cost, int n,
+                           long (*items)(const Geom&)) {
+  int best = 1;
+  double least = 0.0;
+  for (int k = 0; k < n; k++) {
+    double total = 0.0;
+    long all = 0;
+    for (int i = 0; i < count; i++) {
+      const Geom& G = problems[i].geom->g;
+      const long groups = (problems[i].batch + sizes[k] - 1) / sizes[k];
+      all += groups * items(G);
+      total += (double)groups * cost[k] * G.N * (double)G.N * G.A;
+    }
+    if (k > 0 && (all < 512 || total >= least)) continue;
+    least = total;
+    best = sizes[k];
+  }
+  return best;
 }
 
 static int persistent_grid(Ctx* c, const void* kernel, int block, size_t lds, int* out) {
@@ -310,7 +360,31 @@ int sk_sirt_batched(sk_ctx* ctx, const sk_problem* problems, int count, int iter
     else
       plan.fp_mode = want & 3;
   }
+  plan.nc = 2;
+  for (int i = 0; i < count; i++) {
+    const Geom& G = problems[i].geom->g;
+    plan.dr1 = plan.dr1 && G.bp_two_cand;
+    if (!G.bp_nc || !plan.nc)
+      plan.nc = 0;
+    else if (G.bp_nc != 2)
+      plan.nc = 4;  // serves 1 to 4: a further candidate's length is 0
+  }
+  if (!ex && plan.fp_mode == 5) {
+    const int sizes[3] = {1, 2, 4};
+    const double cost[3] = {1.0, 1.5, 2.33};
+    plan.fp_images = images_per_item(problems, count, sizes, cost, 3, [](const Geom& G) {
+      return (long)G.n_fpg * ((G.R + FPG_BINS - 1) / FPG_BINS);
+    });
+  }
+  if (!ex && plan.nc) {
+    const int sizes[4] = {1, 2, 4, 8};
+    const double cost[4] = {1.0, 1.39, 1.9, 3.4};
+    plan.bp_images = images_per_item(problems, count, sizes, cost, 4, [](const Geom& G) {
+      return (long)((G.N + BP_TW - 1) / BP_TW) * ((G.N + 31) / 32);
+    });
+  }
   if (const char* m = getenv("SYNKRO_BATCH_BP_PPT")) plan.bp_ppt = atoi(m) == 2 ? 2 : 4;
+  if (plan.bp_images > 1) plan.bp_ppt = 2;
   const int ppt = plan.bp_ppt;
   const int fp_item_bins =
       plan.fp_mode == 5 ? FPG_BINS : (plan.fp_mode == 4 ? FPS_RAYS : 64 * ((plan.fp_mode & 1) ? 2 : 1));
@@ -331,10 +405,10 @@ int sk_sirt_batched(sk_ctx* ctx, const sk_problem* problems, int count, int iter
     B.bp_ty = (G.N + 16 * ppt - 1) / (16 * ppt);
     B.fp_begin = args.fp_total;
     B.bp_begin = args.bp_total;
-    args.fp_total += (long)P.batch * B.fp_units * B.fp_wb;
-    args.bp_total += (long)P.batch * B.bp_tx * B.bp_ty;
+    if (!ex && plan.nc) B.bp.W = bp_window_bins(ppt, G.drho, plan.nc);
+    args.fp_total += (long)((P.batch + plan.fp_images - 1) / plan.fp_images) * B.fp_units * B.fp_wb;
+    args.bp_total += (long)((P.batch + plan.bp_images - 1) / plan.bp_images) * B.bp_tx * B.bp_ty;
     plan.Wmax = std::max(plan.Wmax, B.bp.W);
-    plan.dr1 = plan.dr1 && G.bp_two_cand;
     args.p[oi] = B;
   }
   if (args.bp_total >= (1L << 32))
@@ -342,37 +416,30 @@ int sk_sirt_batched(sk_ctx* ctx, const sk_problem* problems, int count, int iter
   if (sizeof(float2) * BP_LB * (size_t)plan.Wmax > 60 * 1024)
     return fail(c, SK_EINVAL, "backprojection window exceeds LDS");
 
-  const size_t lds = sizeof(float2) * BP_LB * (size_t)plan.Wmax;
+  // occupancy (and so the persistent grids) of the kernels that will run
   int fp_grid = 0, bp_grid = 0;
-  // occupancy (and so the persistent grid) of the forward kernel that will run
-  const void* kfp_ex[4] = {(const void*)k_fp_persist<true, 1, false>, (const void*)k_fp_persist<true, 2, false>,
-                           (const void*)k_fp_persist<true, 1, true>, (const void*)k_fp_persist<true, 2, true>};
-  const void* kfp_fast[4] = {(const void*)k_fp_persist<false, 1, false>, (const void*)k_fp_persist<false, 2, false>,
-                             (const void*)k_fp_persist<false, 1, true>, (const void*)k_fp_persist<false, 2, true>};
-  const void* kfp = plan.fp_mode == 5   ? (const void*)k_fpg_persist
-                    : plan.fp_mode == 4 ? (const void*)k_fps_persist
-                                        : (ex ? kfp_ex[plan.fp_mode & 3] : kfp_fast[plan.fp_mode & 3]);
-  const void* kbp2 =
-      plan.dr1 ? (ex ? (const void*)k_bp_persist<true, 2, true, 2> : (const void*)k_bp_persist<false, 2, true, 2>)
-               : (ex ? (const void*)k_bp_persist<true, 0, false, 2> : (const void*)k_bp_persist<false, 0, false, 2>);
-  const void* kbp4 =
-      plan.dr1 ? (ex ? (const void*)k_bp_persist<true, 2, true, 4> : (const void*)k_bp_persist<false, 2, true, 4>)
-               : (ex ? (const void*)k_bp_persist<true, 0, false, 4> : (const void*)k_bp_persist<false, 0, false, 4>);
-  const void* kbp = plan.bp_ppt == 4 ? kbp4 : kbp2;
-  rc = plan.fp_mode == 5   ? persistent_grid(c, kfp, FPS_RAYS, fpg_lds(plan.fpg_cpl), &fp_grid)
-       : plan.fp_mode == 4 ? persistent_grid(c, kfp, FPS_RAYS, sizeof(float) * FPS_CS * FPS_MAXW, &fp_grid)
-                           : persistent_grid(c, kfp, FP_BLOCK, 0, &fp_grid);
-  if (!rc) rc = persistent_grid(c, kbp, 256, lds, &bp_grid);
+  plan.kfp = fp_kernel(plan, ex);
+  plan.kbp = bp_kernel(plan, ex);
+  plan.fp_lds = plan.fp_mode == 5 ? sizeof(float) * fpg_lds_floats(plan.fp_images == 1 ? FpgShape<1>::nbuf : 1,
+                                                                   plan.fp_images, plan.fpg_cpl, false)
+                                  : (plan.fp_mode == 4 ? sizeof(float) * FPS_CS * FPS_MAXW : 0);
+  plan.bp_lds = sizeof(float) * BP_LB * (size_t)plan.Wmax * (1 + plan.bp_images);
+  rc = persistent_grid(c, plan.kfp, FPS_RAYS, plan.fp_lds, &fp_grid);
+  if (!rc) rc = persistent_grid(c, plan.kbp, 256, plan.bp_lds, &bp_grid);
   if (rc) return rc;
   if (getenv("SYNKRO_VERBOSE"))
-    fprintf(stderr, "sk_sirt_batched: %d groups, fp mode %d items %ld (grid %d), bp 16x%d tiles items %ld (grid %d), W %d\n",
-            count, plan.fp_mode, args.fp_total, fp_grid, 16 * plan.bp_ppt, args.bp_total, bp_grid, plan.Wmax);
+    fprintf(stderr,
+            "sk_sirt_batched: %d groups, fp mode %d x %d images items %ld (grid %d), bp 16x%d tiles x %d images items "
+            "%ld (grid %d), W %d\n",
+            count, plan.fp_mode, plan.fp_images, args.fp_total, fp_grid, 16 * plan.bp_ppt, plan.bp_images,
+            args.bp_total, bp_grid, plan.Wmax);
 
   // Everything the graph's kernel arguments bake in: a later call with the same key replays it.
   std::vector<unsigned long long> key;
   key.reserve(8 + 6 * (size_t)count);
   for (unsigned long long v : {(unsigned long long)count, (unsigned long long)iters, (unsigned long long)ex,
                                (unsigned long long)plan.fp_mode, (unsigned long long)plan.bp_ppt,
+                               (unsigned long long)plan.fp_images, (unsigned long long)plan.bp_images,
                                (unsigned long long)(uintptr_t)ws, (unsigned long long)fp_grid,
                                (unsigned long long)bp_grid})
     key.push_back(v);
@@ -404,12 +471,7 @@ int sk_sirt_batched(sk_ctx* ctx, const sk_problem* problems, int count, int iter
     rc = launched(c, "counter reset");
   }
   for (int it = 0; it < iters && rc == SK_OK; it++) {
-    if (plan.dr1)
-      rc = ex ? launch_iteration<true, 2, true>(c, plan, fp_grid, bp_grid, cs)
-              : launch_iteration<false, 2, true>(c, plan, fp_grid, bp_grid, cs);
-    else
-      rc = ex ? launch_iteration<true, 0, false>(c, plan, fp_grid, bp_grid, cs)
-              : launch_iteration<false, 0, false>(c, plan, fp_grid, bp_grid, cs);
+    rc = launch_iteration(c, plan, fp_grid, bp_grid, cs);
   }
   hipGraph_t graph = nullptr;
   hipError_t e = hipStreamEndCapture(cs, &graph);

@@ -90,3 +90,32 @@ def test_sirt_of_a_batch_is_each_slices_own(ctx, batch):
             assert torch.equal(x[k], one), k
     finally:
         geo.set_variants(-1, -1)
+
+
+# (groups of (N, angles, bins, bin width), images per group): items of 1, 2, 4 and 8 images, groups
+# that leave a remainder, bin widths with one to four candidates mixed, and the narrow bins of the
+# general path
+BATCHES = [
+    ([(128, 200, 182, 1.0), (96, 150, 137, 1.0)], 2),
+    ([(128, 200, 182, 1.0), (96, 150, 137, 1.0), (200, 90, 283, 1.0)], 7),
+    ([(256, 400, 363, 1.0), (64, 90, 91, 1.0)], 9),
+    ([(256, 400, 363, 1.0), (128, 120, 400, 0.5), (130, 77, 100, 2.0), (96, 60, 350, 0.4)], 5),
+    ([(64, 90, 320, 0.3)], 3),
+]
+
+
+@pytest.mark.parametrize("sizes,batch", BATCHES)
+def test_batched_sirt_equals_each_slice_alone(ctx, sizes, batch):
+    from synkrotomo_amd.projector import sirt_batched
+    gen = torch.Generator(device="cuda").manual_seed(batch)
+    groups = []
+    for k, (N, A, R, drho) in enumerate(sizes):
+        geo = _geometry(ctx, N, A, R, 0.0, drho)
+        b = batch + (k == 1)
+        groups.append((geo, torch.zeros(b, N, N, device="cuda"), torch.rand(b, A, R, device="cuda", generator=gen)))
+    sirt_batched(groups, 3)
+    for geo, x, sino in groups:
+        for i in (0, x.shape[0] - 1):
+            one = torch.zeros(geo.N, geo.N, device="cuda")
+            geo.sirt_(one, sino[i].contiguous(), 3)
+            assert torch.equal(x[i], one), (geo.N, i)
