@@ -39,7 +39,7 @@ __global__ __launch_bounds__(256, bp_waves_per_simd(NC, PPT)) void k_bp(BpParams
 constexpr int BP_IMAGES_PPT = 2;
 
 template <int MODE, int WEIGHTS, int NC, int S>
-__global__ __launch_bounds__(256, S == 8 ? 3 : (S == 4 ? 6 - NC / 3 : 8)) void k_bp_images(BpParams P) {
+__global__ __launch_bounds__(256, S == 8 ? 3 : (S == 4 ? 5 : 7)) void k_bp_images(BpParams P) {
   extern __shared__ float4 win4[];
   __shared__ BpLineLds lsh[BP_LB];
   int tx = blockIdx.x, ty = blockIdx.y;
@@ -57,7 +57,7 @@ BpParams bp_params(const Geom* g, const BpArgs& a, int ppt) {
   const unsigned* order =
       g->d_bp_order ? g->d_bp_order + g->bp_order_off[ppt == 1 ? 0 : (ppt == 2 ? 1 : 2)] : nullptr;
   return BpParams{g->d_lines, g->A, g->R, g->N, g->ncand, bp_window_bins(ppt, g->drho, g->ncand), a.batch,
-                  g->n_steep, g->rho0, g->drho, a.sino, a.out, a.outT, a.colinv, g->d_inter, order};
+                  g->n_steep, g->rho0, g->drho, 1.0f / g->drho, a.sino, a.out, a.outT, a.colinv, g->d_inter, order};
 }
 
 template <bool EXACT, int MODE, int WEIGHTS, int NC, bool DR1, int PPT>

@@ -403,7 +403,7 @@ struct BpParams {
   const Line* lines;
   int A, R, N, ncand, W, batch;
   int nsteep;           // lines [0, nsteep) are steep, the rest flat
-  float rho0, drho;
+  float rho0, drho, idr;  // idr = 1 / drho
   const float* sino;    // [batch][A][R]
   float* out;           // [batch][N][N]  (BP_SIRT: the image, updated in place)
   float* outT;          // BP_SIRT: transposed copy of the updated image
@@ -435,9 +435,10 @@ struct alignas(16) BpLineLds {
                  // (tile_binade), else 0
   float slope;   // the line's (read here with the rest of the record: no scalar load per line)
   float rs;      // 1/|slope| on LINE_NEWTON lines (fast path), else 0
-  float cost;    // the line's (window staging)
+  int flags;     // the line's
   float wscale;  // factor of the staged values: lbase, or lbase/dx when dx > 0
-  int orig;
+  unsigned row;  // window staging: byte offsets of the window's first bin in the sinogram and in the
+  unsigned tab;  // intercept table (mod 2^32; used where both are below 2^32 bytes)
   int tie;       // hoisted fast path, tile with one binade: the step is a rounding tie (dx = 0)
 };
 
@@ -536,6 +537,13 @@ __device__ __forceinline__ void bp_item(const BpParams& P, int tile_x, int tile_
 #pragma unroll
   for (int m = 0; m < S; ++m)
     sb[m] = P.sino + (size_t)(S == 1 ? bz : min(img0 + m, P.batch - 1)) * P.A * P.R;
+  // Sinogram and intercept table below 2^32 bytes: 32-bit offsets into range-checked buffers.
+  const bool small = P.inter && (long)P.A * P.R < (1L << 30);
+  const int nbytes = small ? (int)((unsigned)P.A * (unsigned)P.R * 4u) : 0;
+  const __amdgpu_buffer_rsrc_t tab_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)P.inter, 0, nbytes, BUF_DWORD3);
+  __amdgpu_buffer_rsrc_t sino_rsrc[S];
+#pragma unroll
+  for (int m = 0; m < S; ++m) sino_rsrc[m] = __builtin_amdgcn_make_buffer_rsrc((void*)sb[m], 0, nbytes, BUF_DWORD3);
   float* win_x = reinterpret_cast<float*>(win);                  // S > 1: intercepts
   V* win_v = reinterpret_cast<V*>(win_x + LB * W);               // S > 1: values (LB*W*4 is a multiple of 16)
   const int X = X0 + tx;
@@ -568,24 +576,31 @@ __device__ __forceinline__ void bp_item(const BpParams& P, int tile_x, int tile_
       const float cx0 = (float)((fl ? Y0 : X0) - h), cy0 = (float)((fl ? X0 : Y0) - h);
       const float cx1 = cx0 + (float)((fl ? TH : BP_TW) - 1);
       const float cy1 = cy0 + (float)((fl ? BP_TW : TH) - 1);
-      auto first = [&](float x, float y) {  // t / 1 = t: no division for unit bins
-        return unit ? cand_s<true>(L, x, y, P.rho0, P.drho) : cand_s<false>(L, x, y, P.rho0, P.drho);
+      // the lowest index of the corners: division by drho and ceil are monotone, so of the lowest
+      // rho - rho0 (t / 1 = t: no division for unit bins)
+      auto corner = [&](float x, float y) {
+        return L.cost * ((x + 0.5f) - L.fc) + L.sint * ((y + 0.5f) - L.fs) - P.rho0;
       };
-      const float smin = fminf(fminf(first(cx0, cy0), first(cx1, cy0)), fminf(first(cx0, cy1), first(cx1, cy1)));
+      float smin = fminf(fminf(corner(cx0, cy0), corner(cx1, cy0)), fminf(corner(cx0, cy1), corner(cx1, cy1)));
+      if (!unit) {
+        asm volatile("");  // a branch: as a select, unit bins would pay for the division
+        smin = smin / P.drho;
+      }
+      smin = ceilf(smin);
       BpLineLds e;
       // The hoisted fast path starts the window one bin lower: its index may round one bin
       // below the reference's at the tile's lowest corner (the top keeps a one-bin margin).
       e.w0 = (int)smin - (REV ? 1 : 0);
       e.ci = e.si = e.cst = 0.0f;
       if constexpr (FASTREF) {
-        const float idr = unit ? 1.0f : 1.0f / P.drho;
-        e.ci = L.cost * idr;
-        e.si = L.sint * idr;
-        e.cst = -(fmaf(L.cost, L.fc, L.sint * L.fs) + P.rho0) * idr;
+        e.ci = L.cost * P.idr;
+        e.si = L.sint * P.idr;
+        e.cst = -(fmaf(L.cost, L.fc, L.sint * L.fs) + P.rho0) * P.idr;
       }
-      e.cost = L.cost;
       e.slope = L.slope;
-      e.orig = L.orig;
+      e.row = 4u * ((unsigned)L.orig * (unsigned)P.R + (unsigned)e.w0);
+      e.tab = 4u * ((unsigned)(l0 + (int)threadIdx.x) * (unsigned)P.R + (unsigned)e.w0);
+      e.flags = L.flags;
       e.rs = (L.flags & LINE_NEWTON) ? 1.0f / fabsf(L.slope) : 0.0f;
       const int eb = ebin[fl ? 1 : 0];
       const bool exd = REV && eb >= 0 && !(L.flags & LINE_DEGEN);
@@ -597,42 +612,83 @@ __device__ __forceinline__ void bp_item(const BpParams& P, int tile_x, int tile_
     __syncthreads();
     // Window staging, flattened over (line, bin): the 256 threads take entries e = jj*W + k of
     // the block's nl windows in turn (a wave per line would leave most lanes of its second
-    // pass over a 70-bin window idle).  e / W by a multiply-high: exact for e < 2^32 / W.
+    // pass over a 70-bin window idle), U at a time so that their loads are in flight together.
+    // The step from one entry to a thread's next, 256 = dj*W + dk, is uniform.
+    auto stage = [&](int e, int k, float inter, float (&p)[S], bool in, float wscale) {
+#pragma unroll
+      for (int m = 0; m < S; ++m) {
+        p[m] = in ? p[m] : 0.0f;
+        if constexpr (FASTREF) p[m] = p[m] * wscale;
+      }
+      const int at = REV ? e + W - 1 - 2 * k : e;  // jj*W + (W - 1 - k), or jj*W + k
+      if constexpr (S == 1) {
+        win[at] = make_float2(inter, p[0]);
+      } else {
+        win_x[at] = inter;
+        V v;
+#pragma unroll
+        for (int m = 0; m < S; ++m) v[m] = p[m];
+        win_v[at] = v;
+      }
+    };
+    // backprojection.fut:57-58: r = s'*drho + rho0, then r/cost -- from the geometry's table for
+    // bins of the sinogram; bins outside it are rare: divide
+    auto divided = [&](int jj, int k) {
+      return ((float)(lsh[jj].w0 + k) * P.drho + P.rho0) / P.lines[l0 + jj].cost;
+    };
     {
+      constexpr int U = PPT == 4 ? 3 : (PPT == 2 ? 5 : 4);
       const int total = nl * W;
-      const unsigned Mw = 0xffffffffu / (unsigned)W + 1u;
-      for (int e = threadIdx.x; e < total; e += 256) {
-        const int jj = (int)__umulhi((unsigned)e, Mw);
-        const int k = e - jj * W;
-        const int sp = lsh[jj].w0 + k;
-        const bool in = sp >= 0 && sp < P.R;
-        // backprojection.fut:57-58: r = s'*drho + rho0, then r/cost (from the geometry's table
-        // for bins of the sinogram; bins outside it are rare: divide)
-        float inter;
-        if (in && P.inter)
-          inter = P.inter[(l0 + jj) * P.R + sp];
-        else
-          inter = ((float)sp * P.drho + P.rho0) / lsh[jj].cost;
-        float p[S];
+      const int dj = 256 / W, dk = 256 - dj * W;
+      int jj = (int)threadIdx.x / W, k = (int)threadIdx.x - jj * W;
+      if (small) {
+        for (int e0 = threadIdx.x; e0 < total; e0 += 256 * U) {
+          int line[U], kk[U];
+          float inter[U], p[U][S];
 #pragma unroll
-        for (int m = 0; m < S; ++m) {
-          if constexpr (MODE == BP_ONES_INV) {
-            p[m] = in ? 1.0f : 0.0f;
-          } else {
-            const float v = sb[m][(size_t)lsh[jj].orig * P.R + (in ? sp : 0)];  // in bounds either way
-            p[m] = in ? v : 0.0f;
+          for (int u = 0; u < U; ++u) {
+            line[u] = e0 + 256 * u < total ? jj : 0;
+            kk[u] = k;
+            // an offset past the end reads 0, one in another row is replaced below
+            inter[u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(tab_rsrc, lsh[line[u]].tab + 4 * k, 0, 0));
+#pragma unroll
+            for (int m = 0; m < S; ++m) {
+              if constexpr (MODE == BP_ONES_INV)
+                p[u][m] = 1.0f;
+              else
+                p[u][m] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(sino_rsrc[m], lsh[line[u]].row + 4 * k, 0, 0));
+            }
+            k += dk;
+            jj += dj;
+            if (k >= W) {
+              k -= W;
+              ++jj;
+            }
           }
-          if constexpr (FASTREF) p[m] = p[m] * lsh[jj].wscale;
-        }
-        const int at = jj * W + (REV ? W - 1 - k : k);
-        if constexpr (S == 1) {
-          win[at] = make_float2(inter, p[0]);
-        } else {
-          win_x[at] = inter;
-          V v;
 #pragma unroll
-          for (int m = 0; m < S; ++m) v[m] = p[m];
-          win_v[at] = v;
+          for (int u = 0; u < U; ++u) {
+            if (e0 + 256 * u >= total) break;
+            const bool in = (unsigned)(lsh[line[u]].w0 + kk[u]) < (unsigned)P.R;
+            if (!in) inter[u] = divided(line[u], kk[u]);
+            stage(e0 + 256 * u, kk[u], inter[u], p[u], in, lsh[line[u]].wscale);
+          }
+        }
+      } else {  // 2^32 bytes or more: 64-bit offsets
+        for (int e = threadIdx.x; e < total; e += 256) {
+          const int sp = lsh[jj].w0 + k;
+          const bool in = sp >= 0 && sp < P.R;
+          const size_t row = (size_t)P.lines[l0 + jj].orig * P.R + (in ? sp : 0);  // in bounds either way
+          float p[S];
+#pragma unroll
+          for (int m = 0; m < S; ++m) p[m] = MODE == BP_ONES_INV ? 1.0f : sb[m][row];
+          const float inter = in && P.inter ? P.inter[(size_t)(l0 + jj) * P.R + sp] : divided(jj, k);
+          stage(e, k, inter, p, in, lsh[jj].wscale);
+          k += dk;
+          jj += dj;
+          if (k >= W) {
+            k -= W;
+            ++jj;
+          }
         }
       }
     }
@@ -772,7 +828,7 @@ __device__ __forceinline__ void bp_item(const BpParams& P, int tile_x, int tile_
         const bool exact_step = ebin[part] >= 0;  // uniform: the tile's binade for this part
         const bool all_slots = part == 0 || fslots == (1 << PPT) - 1;  // uniform
         for (int jr = j_begin; jr < j_end;) {  // uniform: scalar loop over the runs
-          const int f = P.lines[l0 + jr].flags;
+          const int f = __builtin_amdgcn_readfirstlane(lsh[jr].flags);
           const int je = min(jr + (f >> LINE_RUN_SHIFT), j_end);
           if (f & LINE_DEGEN)
             run(std::integral_constant<int, 2>{}, none{}, jr, je);
@@ -807,7 +863,7 @@ __device__ __forceinline__ void bp_item(const BpParams& P, int tile_x, int tile_
           while (tm) {  // uniform
             const int jj = __builtin_ctzll(tm);
             tm &= tm - 1;
-            if (P.lines[l0 + jj].flags & LINE_SLOPE_POS)
+            if (__builtin_amdgcn_readfirstlane(lsh[jj].flags) & LINE_SLOPE_POS)
               line_body(std::integral_constant<int, 0>{}, none{}, jj);
             else
               line_body(std::integral_constant<int, 1>{}, none{}, jj);
