@@ -150,10 +150,10 @@ static void bp_go_ex(bool ex, int variant, const Geom* g, const BpArgs& a, hipSt
 // The tile height of a geometry that was not tuned, on a context whose option is 0: the tallest of
 // 64 and 32 rows that leaves 1024 tiles (4 workgroups per CU), else 16.  Taller tiles share a
 // line's constants among more pixels, but the walk over the lines is serial and needs workgroups
-// enough to hide it: 512^2, 358 angles: 76, 88, 136 us for 16, 32, 64 rows; 768^2, 537: 224, 178,
-// 221; 1024^2, 716: 415, 337, 333; 2048^2, 1433: 3008, 2383, 2179.  Four candidates a pixel keep
-// 64-row tiles from 8 waves per SIMD (1024^2, 716 angles, bins of 0.4: 821, 786, 1051).  Exact mode's divisions hide the
-// rest at 16 rows (1024^2, 700: 989, 1040, 1148).
+// enough to hide it: 512^2, 358 angles: 72, 84, 123 us for 16, 32, 64 rows; 768^2, 537: 199, 171,
+// 196; 1024^2, 716: 403, 321, 314; 2048^2, 1433: 3008, 2383, 2179.  Four candidates a pixel keep
+// 64-row tiles from 8 waves per SIMD (1024^2, 716 angles, bins of 0.4: 821, 786, 1051).  Exact mode's
+// divisions hide the rest at 16 rows (1024^2, 700: 989, 1040, 1148).
 static int bp_variant_default(const Geom* g, int batch) {
   const long across = (g->N + BP_TW - 1) / BP_TW;
   for (int v = g->bp_nc == 4 ? 1 : 2; v > 0; --v) {
