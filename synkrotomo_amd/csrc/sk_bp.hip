@@ -95,17 +95,21 @@ static void bp_go_images_s(int images, const Geom* g, const BpArgs& a, hipStream
 }
 
 // Images per workgroup of the fast backprojector, 1 = the one-image kernels.  Below about a
-// workgroup per CU more images only lengthen each one (the walk over the lines is serial): 256^2,
-// 179 angles (128 tiles of 16 x 32), us for 1, 2 and 4 images per workgroup: 3 images 40.6, 48.4,
-// 53.9; 6 images 58.2, 52.5, 56.2; 16 images 103, 73.8, 61.3.  512^2, 358 angles (512 tiles):
-// 2 images 114, 95.7, 107; 3 images 149, 130, 110; 8 images 336, 220, 150, and 8 per workgroup
-// 140.  Bins off about unit width (1, 3 or 4 candidates) have the 4-image kernel only.
+// workgroup per CU more images only lengthen each one (the walk over the lines is serial).  us for 1,
+// 2 and 4 images per workgroup: 512^2, 804 angles (512 tiles of 16 x 32): 2 images 245, 200, 224; 3
+// images 318, 274, 224; 640^2, 450: 2 images 187, 141, 165; 4 images 328, 223, 166.  Eight share more
+// but fit 3 workgroups per CU (4 images: 5), so a launch pays where it ends within the first 768 or
+// where the rounds are many; us for 4 and 8 per workgroup, 8 images, 400 angles: 512^2 with 358 (512
+// workgroups of 8) 166 and 145; 608^2 (722) 248 and 200; 640^2 (800) 255 and 291; 768^2 (1152) 311 and
+// 320; 896^2 (1568) 425 and 459; 1024^2 (2048) 530 and 501.  Bins off about unit width (1, 3 or 4
+// candidates) have the 4-image kernel only.
 int bp_images(const Geom* g, int batch) {
   if (!g->bp_nc) return 1;
   const int TH = 16 * BP_IMAGES_PPT;
   const long tiles = (long)((g->N + BP_TW - 1) / BP_TW) * ((g->N + TH - 1) / TH);
   if (g->bp_nc != 2) return batch >= 3 && tiles * ((batch + 3) / 4) >= 256 ? 4 : 1;
-  if (batch >= 7 && tiles * ((batch + 7) / 8) >= 512) return 8;
+  const long eights = tiles * ((batch + 7) / 8);
+  if (batch >= 7 && ((eights >= 512 && eights <= 768) || eights >= 1920)) return 8;
   if (batch >= 3 && tiles * ((batch + 3) / 4) >= 256) return 4;
   if (batch >= 2 && tiles * ((batch + 1) / 2) >= 384) return 2;
   return 1;

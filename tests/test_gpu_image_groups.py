@@ -41,9 +41,9 @@ def test_projection_of_a_batch_is_each_images_own(ctx, name, N, A, R, start, drh
         geo.set_variants(-1, -1)
 
 
-# the batches run 2, 4, 4, 8 and 8 images per workgroup at 440^2 (28 x 14 tiles of 16 x 32); bins
+# the batches run 2, 4, 4, 4, 4 and 8 images per workgroup at 440^2 (28 x 14 tiles of 16 x 32); bins
 # of 0.9 have two candidates per pixel too, of 0.4, 0.5 and 2 four, three and one (4 images or 1)
-@pytest.mark.parametrize("batch,drho", [(2, 1.0), (3, 1.0), (6, 1.0), (11, 1.0), (16, 0.9), (2, 0.5), (6, 0.4),
+@pytest.mark.parametrize("batch,drho", [(2, 1.0), (3, 1.0), (6, 1.0), (11, 1.0), (16, 0.9), (40, 1.0), (2, 0.5), (6, 0.4),
                                         (6, 0.5), (6, 2.0)])
 @pytest.mark.parametrize("op", ["bp", "bp_adjoint"])
 def test_backprojection_of_a_batch_is_each_images_own(ctx, op, batch, drho):
@@ -61,8 +61,9 @@ def test_backprojection_of_a_batch_is_each_images_own(ctx, op, batch, drho):
         geo.set_variants(-1, -1)
 
 
-def test_sirt_update_of_a_batch_is_each_slices_own(ctx):
-    N, A, R, batch = 440, 37, 631, 9
+@pytest.mark.parametrize("batch", [9, 40])  # 4 and 8 images per workgroup
+def test_sirt_update_of_a_batch_is_each_slices_own(ctx, batch):
+    N, A, R = 440, 37, 631
     geo = _geometry(ctx, N, A, R, 0.0, 1.0)
     b = torch.rand(batch, A, R, device="cuda", generator=torch.Generator(device="cuda").manual_seed(3))
     x = torch.zeros(batch, N, N, device="cuda")
