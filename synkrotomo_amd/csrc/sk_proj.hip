@@ -72,6 +72,47 @@ __global__ __launch_bounds__(FP_BLOCK) void k_fp_listed(FpParams P, const int* _
   fp_item<false, FP_PLAIN, W_ADJ, DR1, 1>(P, list[blockIdx.y], blockIdx.x * FP_WAVES + wave, blockIdx.z);
 }
 
+// B^T at the image's corners: the rays of every line that cross less than two pixels' length, with
+// the backprojector's lengths.  A.x forms a row as vb + f*(vo - vb): a ray that leaves most of a
+// row's length outside gets its short part from 1 - f, 6e-8 off however short, and divided by a row
+// sum of 1e-3 (the gradient of a SIRT step) that is 6e-5 of the result.  The outermost corner of a
+// line is at (frame) x = -+h, y = -+h by the signs of cost and sint; a chord at distance d from
+// it is d/|cost*sint| long and lies in the last rows there.  per_end bins from each end's corner on.
+// 8 images of 512^2, 360 angles: 6 us of 330.
+constexpr int RIM_ROWS = 4;  // two rows of a chord (|slope| <= 1), the one it ends in, one for rounding
+template <bool DR1>
+__global__ __launch_bounds__(256) void k_bpt_rims(FpParams P, int per_end) {
+  const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x;
+  const size_t line = t / (2 * per_end);
+  if (line >= (size_t)P.A) return;
+  const int q = (int)(t - line * (2 * per_end));
+  const bool high = q >= per_end;
+  const Line L = P.lines[line];
+  if (L.flags & LINE_DEGEN) return;
+  const int N = P.N, h = N >> 1;
+  const float reach = (float)h * (fabsf(L.cost) + fabsf(L.sint));
+  const float edge = ((high ? reach : -reach) - P.rho0) / P.drho;  // bin of the corner
+  const int r = high ? (int)ceilf(edge) - (q - per_end) : (int)floorf(edge) + q;
+  if (r < 0 || r >= P.R) return;
+  const float d = (high ? edge - (float)r : (float)r - edge) * P.drho;
+  if (d > 2.0f * fabsf(L.cost * L.sint)) return;
+  const bool upper = (L.sint > 0.0f) == high;  // the corner's rows
+  const int i0 = upper ? max(h - RIM_ROWS, -h) : -h, i1 = min(i0 + RIM_ROWS, h);
+  const float* src = ((L.flags & LINE_FLAT) ? P.imgT : P.img) + (size_t)blockIdx.y * N * N;
+  const float icpt = (P.rho0 + (float)r * P.drho) / L.cost;  // forwardprojection.fut:33-34
+  float sum = 0.0f;
+  for (int i = i0; i < i1; ++i) {
+    const float xbot = (float)i * L.slope + icpt, xtop = xbot + L.slope;
+    const int Xb = (int)floorf(xbot), Xt = (int)floorf(xtop);
+    auto part = [&](int X) {
+      const float len = bp_entry<false, DR1>(L, X, (float)i, xbot, xtop, r, P.ncand, P.rho0, P.drho);
+      return (unsigned)(X + h) < (unsigned)N ? len * src[(size_t)(i + h) * N + X + h] : 0.0f;
+    };
+    sum = sum + (part(Xb) + (Xb == Xt ? 0.0f : part(Xt)));
+  }
+  P.out[(size_t)blockIdx.y * P.A * P.R + (size_t)L.orig * P.R + r] = sum;
+}
+
 // ------------------------------------------------------------- staged A.x (fast mode)
 // A workgroup holds FPS_RAYS consecutive bins of one line, one ray per lane.  Frame rows go
 // in blocks of FPS_ROWS: for each row the columns any of the workgroup's rays can touch (a
@@ -252,9 +293,10 @@ int launch_fp(Ctx* c, const Geom* g, FpMode mode, const FpArgs& a, hipStream_t s
 // B^T.v.  Fast mode: on a line that is not degenerate the backprojector's length of a ray in a
 // pixel is the forward projector's (both are the part of the row's x-range inside the pixel over
 // the range, and a ray with a nonzero length lies within sqrt(2)/2 of the pixel's centre, so it is
-// one of the pixel's candidates): those lines are A.v, by whichever kernel A.x runs.  The
-// degenerate lines (theta ~ 0, pi/2: a ray on a pixel edge counts in A and not in B) are walked
-// again with the backprojector's own lengths, one launch over their table indices.  8 images of
+// one of the pixel's candidates): those lines are A.v, by whichever kernel A.x runs, but for the
+// short rays at the image's corners (k_bpt_rims).  The degenerate lines (theta ~ 0, pi/2: a ray on
+// a pixel edge counts in A and not in B) are walked again with the backprojector's own lengths, one
+// launch over their table indices.  8 images of
 // 512^2, 360 angles: 1249 us with every line on that walk (60 VALU a row and two dependent global
 // gathers), 330 us like this.
 int launch_fp_bpt(Ctx* c, const Geom* g, const FpArgs& a, hipStream_t s) {
@@ -264,13 +306,23 @@ int launch_fp_bpt(Ctx* c, const Geom* g, const FpArgs& a, hipStream_t s) {
     dr1 ? fp_go<true, FP_PLAIN, W_ADJ, true, 1>(g, a, s) : fp_go<true, FP_PLAIN, W_ADJ, false, 1>(g, a, s);
     return launched(c, "backprojection-transpose kernel");
   }
-  const int rc = launch_fp(c, g, FP_PLAIN, a, s);
+  int rc = launch_fp(c, g, FP_PLAIN, a, s);
+  if (rc) return rc;
+  // a chord of two pixels lies within a distance of 1 of its corner (|cost*sint| <= 1/2)
+  const int per_end = (int)fmin(ceil(1.0 / g->drho) + 2.0, (double)g->R);
+  const FpParams P = fp_params(g, a);
+  const dim3 rims((unsigned)(((size_t)g->A * 2 * per_end + 255) / 256), (unsigned)a.batch);
+  if (dr1)
+    hipLaunchKernelGGL((k_bpt_rims<true>), rims, dim3(256), 0, s, P, per_end);
+  else
+    hipLaunchKernelGGL((k_bpt_rims<false>), rims, dim3(256), 0, s, P, per_end);
+  rc = launched(c, "backprojection-transpose kernel");
   if (rc || !g->n_degen) return rc;
   const dim3 grid((unsigned)((g->R + FP_BLOCK - 1) / FP_BLOCK), (unsigned)g->n_degen, (unsigned)a.batch);
   if (dr1)
-    hipLaunchKernelGGL((k_fp_listed<true>), grid, dim3(FP_BLOCK), 0, s, fp_params(g, a), g->d_degen);
+    hipLaunchKernelGGL((k_fp_listed<true>), grid, dim3(FP_BLOCK), 0, s, P, g->d_degen);
   else
-    hipLaunchKernelGGL((k_fp_listed<false>), grid, dim3(FP_BLOCK), 0, s, fp_params(g, a), g->d_degen);
+    hipLaunchKernelGGL((k_fp_listed<false>), grid, dim3(FP_BLOCK), 0, s, P, g->d_degen);
   return launched(c, "backprojection-transpose kernel");
 }
 

@@ -63,3 +63,19 @@ def test_operators_against_the_oracles_matrices(ctx, name, N, ang, R, rz, dr, va
             assert rel_l2(btv[k].ravel(), ref) <= 2e-6
         else:
             assert not np.any(btv[k])
+
+
+# Rays that cut less than two pixels' length off a corner: a SIRT step's gradient divides them by
+# that length, so each has to be right by itself.  An image of ones: at most 8 entries, each within
+# about 4 ulp of the oracle's (4.8e-7), and 8 additions: 1e-6; 2e-6 leaves a factor of two.
+@pytest.mark.parametrize("N,A,R,rz,dr", [(250, 142, 284, -174.9, 1.25), (64, 200, 91, -45.37, 1.0),
+                                         (130, 97, 740, -92.2, 0.25), (2, 31, 21, -2.0, 0.2)])
+def test_transpose_of_short_rays(ctx, N, A, R, rz, dr):
+    ang = (np.arange(A) * np.pi / A + 0.1).astype(np.float32)
+    geo = ctx.geometry(ang, rz, dr, R, N)
+    got = geo.bp_transpose(torch.ones(N, N, device="cuda")).cpu().numpy().ravel()
+    rp, c, vals = oracle.bp_csr(ang, rz, dr, R, N)
+    ref = np.bincount(c, weights=vals.astype(np.float64), minlength=A * R)
+    short = (ref > 0) & (ref < 2)
+    assert short.sum() > 10
+    np.testing.assert_allclose(got[short], ref[short], rtol=2e-6)
