@@ -113,6 +113,95 @@ __global__ __launch_bounds__(256) void k_bpt_rims(FpParams P, int per_end) {
   P.out[(size_t)blockIdx.y * P.A * P.R + (size_t)L.orig * P.R + r] = sum;
 }
 
+// --------------------------------------------------------- small images (fast mode)
+// The whole image in LDS: cell (y, x) at fpl_origin(N) + y*pitch + x, with zeros two cells wide
+// around it (a row's right border is the next row's left one).  The pitch is odd, so lanes along a
+// column fall into different banks as well.
+constexpr int FPL_MAX_N = 80;  // 28 KB of LDS
+__host__ __device__ constexpr int fpl_pitch(int N) { return (N + 2) | 1; }
+__host__ __device__ constexpr int fpl_origin(int N) { return 2 * fpl_pitch(N) + 2; }
+__host__ __device__ constexpr int fpl_cells(int N) { return fpl_origin(N) + (N + 2) * fpl_pitch(N); }
+
+// Rows [i0, i1) of one ray per lane; column c of frame row i is cells[(c * cs + i * rs)].  Columns
+// are held to [-2, N], whose cells c and c + 1 past the image are 0 like a load outside it.
+template <bool POS, bool NT>
+__device__ __forceinline__ float fpl_rows(const float* cells, int N, int h, int i0, int i1, int cs, int rs,
+                                          float slope, float icpt, float rslope) {
+  float sum = 0.0f, fi = (float)i0;  // exact
+  const int cofs = h - (POS ? 0 : 1);
+  const float* row = cells + (i0 + h) * rs;
+  auto step = [&](const float* at, float f) {
+    const float xb = f * slope + icpt, xt = xb + slope;
+    const int c = min(max(floor_to_int(xb) + cofs, -2), N) * cs;
+    const float va = at[c], vc = at[c + cs];
+    return POS ? fp_row_add<true, NT>(sum, xb, xt, va, vc, rslope) : fp_row_add<false, NT>(sum, xb, xt, vc, va, rslope);
+  };
+#pragma unroll 4
+  for (int i = i0; i < i1; ++i, fi += 1.0f, row += rs) sum = step(row, fi);
+  return sum;
+}
+
+// One image of a small geometry: a wave per 64 bins of a line, four to a workgroup, all bins of all
+// lines in turn; grid (workgroups, images).  The walk (row range, fractions, order of the sums) is
+// fp_item's, with the two pixels of a row from LDS: no transposed copy and no load latency per row.
+// What is left is launch, the copy and a serial walk of N rows at one wave per SIMD: 64^2 and 90
+// angles, calls back to back, 7.9 us against 9.0 for the transposed copy and the per-wave kernel
+// (6.7 at 16^2, where only the launch is left).
+template <int MODE>
+__global__ __launch_bounds__(256) void k_fp_lds(FpParams P) {
+  extern __shared__ float lds[];
+  const int N = P.N, Q = fpl_pitch(N), h = N >> 1, origin = fpl_origin(N), end = origin + N * Q;
+  const float* img = P.img + (size_t)blockIdx.y * N * N;
+  {
+    const int dj = 256 / N, dk = 256 - dj * N;
+    int y = (int)threadIdx.x / N, x = (int)threadIdx.x - y * N;
+#pragma unroll 8
+    for (int e = threadIdx.x; e < N * N; e += 256) {
+      lds[origin + y * Q + x] = img[e];
+      x += dk;
+      y += dj;
+      if (x >= N) {
+        x -= N;
+        ++y;
+      }
+    }
+    for (int e = threadIdx.x; e < origin; e += 256) lds[e] = 0.0f;
+    for (int e = end + threadIdx.x; e < fpl_cells(N); e += 256) lds[e] = 0.0f;
+    for (int r = threadIdx.x; r < N; r += 256)
+      for (int e = N; e < Q; ++e) lds[origin + r * Q + e] = 0.0f;
+  }
+  __syncthreads();
+  const int blocks = (P.R + 63) / 64;
+  const int item = __builtin_amdgcn_readfirstlane(blockIdx.x * FP_WAVES + (threadIdx.x >> 6));
+  const int j = item / blocks, first = (item - j * blocks) * 64;
+  if (j >= P.A) return;
+  const int r = first + (threadIdx.x & 63), last = min(first + 63, P.R - 1);
+  const Line L = P.lines[j];
+  const float icpt = (P.rho0 + (float)r * P.drho) / L.cost;  // forwardprojection.fut:33-34
+  int a0, a1, b0, b1;
+  row_clip(L.slope, (P.rho0 + (float)first * P.drho) / L.cost, h, a0, a1);
+  row_clip(L.slope, (P.rho0 + (float)last * P.drho) / L.cost, h, b0, b1);
+  const int i0 = __builtin_amdgcn_readfirstlane(min(a0, b0)), i1 = __builtin_amdgcn_readfirstlane(max(a1, b1));
+  const bool flat = L.flags & LINE_FLAT, nt = L.flags & LINE_NEWTON;
+  const int cs = flat ? Q : 1, rs = flat ? 1 : Q;
+  const float rslope = nt ? 1.0f / fabsf(L.slope) : 0.0f;
+  const float* cells = lds + origin;
+  float s;
+  if (L.flags & LINE_SLOPE_POS)
+    s = nt ? fpl_rows<true, true>(cells, N, h, i0, i1, cs, rs, L.slope, icpt, rslope)
+           : fpl_rows<true, false>(cells, N, h, i0, i1, cs, rs, L.slope, icpt, 0.0f);
+  else
+    s = nt ? fpl_rows<false, true>(cells, N, h, i0, i1, cs, rs, L.slope, icpt, rslope)
+           : fpl_rows<false, false>(cells, N, h, i0, i1, cs, rs, L.slope, icpt, 0.0f);
+  if (r >= P.R) return;
+  s = s * L.lbase;
+  const size_t o = (size_t)blockIdx.y * P.A * P.R + (size_t)L.orig * P.R + r;
+  if constexpr (MODE == FP_PLAIN)
+    P.out[o] = s;
+  else  // SIRT.fut:33-36: R * (b - A x)
+    P.out[o] = P.rowinv[(size_t)L.orig * P.R + r] * (P.b[o] - s);
+}
+
 // ------------------------------------------------------------- staged A.x (fast mode)
 // A workgroup holds FPS_RAYS consecutive bins of one line, one ray per lane.  Frame rows go
 // in blocks of FPS_ROWS: for each row the columns any of the workgroup's rays can touch (a
@@ -248,18 +337,45 @@ static void fp_go_grouped(const Geom* g, const FpArgs& a, hipStream_t s) {
   }
 }
 
+// Workgroups of four 64-bin waves that a call has.
+static long fp_workgroups(const Geom* g, int batch) {
+  return ((long)g->A * ((g->R + 63) / 64) + FP_WAVES - 1) / FP_WAVES * batch;
+}
+
 // The kernel of a geometry that was not tuned, on a context whose option is 0: the grouped one (and
 // below it what a geometry without line groups, or exact mode, falls back to).  From 128^2 to
 // 2048^2, angle counts 0.35 N to 1.6 N and bins of 0.5 to 2 it is the fastest or within 0.3 us of
 // the fastest (one ray per lane, the default before, us against grouped: 128^2 and 89 angles 13.5,
 // 13.2; 256^2 and 179 30.6, 21.1; 512^2 and 358 91, 59; 2048^2 and 1433 3662, 1750).  Smaller
 // images take a few rows only and the short per-wave kernel is as fast (64^2, 100 angles: 9.0,
-// 9.5), with a tenth of the code to fetch on a first call.
-static int fp_variant_default(const Geom* g) { return g->N < 128 ? 3 : 7; }
+// 9.5), with a tenth of the code to fetch on a first call, until a batch fills the chip: per-wave and
+// grouped, 96^2 and 150 angles 11.6, 11.1 (1 image), 32, 20 (16), 99, 40 (64); 64^2 and 90 angles 9.0,
+// 9.2; 16, 14; 43, 19.
+static int fp_variant_default(const Geom* g, int batch) {
+  return g->N < 128 && fp_workgroups(g, batch) < 512 ? 3 : 7;
+}
+
+// Whether a call takes k_fp_lds, the same way as the rule above: the image is small enough to be
+// copied by every workgroup (us with it and with the better of the other two and their transposed
+// copy: 64^2 and 90 angles 7.9, 9.0; 80^2 and 126 9.4, 10.2; 96^2 and 150 12.0, 11.1; 120^2 and 190
+// 13.4, 13.0), and no more than the three workgroups per CU or so that hide it (64^2 and 90 angles: 4
+// images 8.0, 9.4; 16 images, 720 workgroups, 10.9, 13.8; with half bins, 1440 workgroups, 15.4, 12.8).
+static bool fp_in_lds(const Ctx* c, const Geom* g, int batch) {
+  return !c->exact && g->fp_variant < 0 && !c->fp_variant && g->N <= FPL_MAX_N && fp_workgroups(g, batch) <= 768;
+}
 
 int launch_fp(Ctx* c, const Geom* g, FpMode mode, const FpArgs& a, hipStream_t s) {
   const bool ex = c->exact != 0;
-  int v = g->fp_variant >= 0 ? g->fp_variant : (c->fp_variant ? c->fp_variant : fp_variant_default(g));
+  if (mode != FP_ONES_INV && fp_in_lds(c, g, a.batch)) {
+    const dim3 grid((unsigned)fp_workgroups(g, 1), a.batch);
+    const size_t lds = sizeof(float) * fpl_cells(g->N);
+    if (mode == FP_PLAIN)
+      hipLaunchKernelGGL((k_fp_lds<FP_PLAIN>), grid, dim3(256), lds, s, fp_params(g, a));
+    else
+      hipLaunchKernelGGL((k_fp_lds<FP_SIRT>), grid, dim3(256), lds, s, fp_params(g, a));
+    return launched(c, "forward projection kernel");
+  }
+  int v = g->fp_variant >= 0 ? g->fp_variant : (c->fp_variant ? c->fp_variant : fp_variant_default(g, a.batch));
   if (v == 7) {
     if (!ex && g->d_fpg && mode != FP_ONES_INV) {
       if (mode == FP_PLAIN)
@@ -350,7 +466,7 @@ int sk_fp(sk_ctx* ctx, sk_geom* g, int batch, const float* d_img, float* d_sino,
   const Geom& G = g->g;
   hipStream_t s = (hipStream_t)stream;
   const float* imgT = d_img;
-  if (G.n_steep < G.A) {
+  if (G.n_steep < G.A && !fp_in_lds(c, &G, batch)) {
     void* ws = nullptr;
     rc = scratch(c, sizeof(float) * (size_t)batch * G.N * G.N, s, &ws);
     if (rc) return rc;

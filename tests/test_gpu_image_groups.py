@@ -41,6 +41,27 @@ def test_projection_of_a_batch_is_each_images_own(ctx, name, N, A, R, start, drh
         geo.set_variants(-1, -1)
 
 
+# images held in LDS (up to 80^2, few workgroups) against the per-wave kernel: sizes around a wave
+# and a workgroup, the largest and the first past it, bins past both edges of the image,
+# fewer items than waves, batches on both sides of the bound on workgroups
+@pytest.mark.parametrize("N,A,R,drho,batch", [(2, 1, 3, 1.0, 1), (6, 5, 9, 0.5, 2), (62, 7, 200, 0.7, 1),
+                                              (64, 90, 91, 1.0, 1), (64, 90, 91, 1.0, 17), (64, 90, 91, 1.0, 18),
+                                              (78, 33, 64, 2.5, 3), (80, 126, 65, 1.0, 2), (82, 20, 117, 1.0, 2)])
+def test_small_images_in_lds_give_the_per_wave_kernels_bits(ctx, N, A, R, drho, batch):
+    geo = _geometry(ctx, N, A, R, 0.0, drho)
+    gen = torch.Generator(device="cuda").manual_seed(N)
+    x = torch.randn(batch, N, N, device="cuda", generator=gen)
+    x[-1] *= 1e6
+    b = torch.rand(batch, A, R, device="cuda", generator=gen)
+    got, step = geo.fp(x), geo.sirt_(x.clone(), b, 2)
+    geo.set_variants(3, 0)
+    try:
+        assert torch.equal(got, geo.fp(x))
+        assert torch.equal(step, geo.sirt_(x.clone(), b, 2))
+    finally:
+        geo.set_variants(-1, -1)
+
+
 # the batches run 2, 4, 4, 4, 4 and 8 images per workgroup at 440^2 (28 x 14 tiles of 16 x 32); bins
 # of 0.9 have two candidates per pixel too, of 0.4, 0.5 and 2 four, three and one (4 images or 1)
 @pytest.mark.parametrize("batch,drho", [(2, 1.0), (3, 1.0), (6, 1.0), (11, 1.0), (16, 0.9), (40, 1.0), (2, 0.5), (6, 0.4),
