@@ -412,7 +412,8 @@ __global__ __launch_bounds__(256) void k_conv_in_dgrad(int H, int W, const __bf1
 // channels F ([B][H][W][CI]): K[ch][t][c] = sum_p V[p][ch] F[p + off_t][c] on VALU, FP32 FMAs of the
 // unrounded FP32 values.  V = the gradient and F = the input for conv1 (TAIL false: out = K, then
 // db[ch] = sum V).  For conv4 (TAIL true) V = its input and F = the gradient: sum_p g[p] V[p +
-// off_t] = sum_q V[q] g[q - off_t], i.e. tap 8 - t of K, out [t][ch], then db = sum of F.
+// off_t] = sum_q V[q] g[q - off_t], i.e. tap 8 - t of K, out [t][ch], then db = sum of F (as two
+// floats, high and low part).
 // A wave walks 16x4 pixels of a 16x16 tile at a time: lane l holds channels 2(l%16) and +1 of row
 // l/16, so a pixel's V is one coalesced dword per lane and its 9 F values are read from LDS rows
 // into registers once per tile row; sums stay in registers over all of the block's tiles.
@@ -422,14 +423,17 @@ template <int CI, bool TAIL>
 __global__ __launch_bounds__(256) void k_wgrad_thin(int H, int W, int B, const __bf16* __restrict__ V,
                                                     const __bf16* __restrict__ M, const float* __restrict__ F,
                                                     float* __restrict__ partials) {
-  constexpr int NW = NCH * 9 * CI, NOUT = NW + (TAIL ? 1 : NCH);
+  constexpr int NW = NCH * 9 * CI, NOUT = NW + (TAIL ? 2 : NCH);
   constexpr int FS = CT + 4;  // LDS row of F (floats): 18 columns, 16-byte multiple
   __shared__ __attribute__((aligned(16))) float sf[CI][CT + 2][FS];
   __shared__ float red[NOUT];
+  [[maybe_unused]] __shared__ double red_f[4];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int cp = lane & 15, sub = lane >> 4;
   float acc[CI][2][9], accb[2] = {0.0f, 0.0f};
-  double sum_f = 0.0;  // TAIL: a sum of one sign-changing value per pixel, the one output without BF16 factors
+  // TAIL: a sum of one sign-changing value per pixel, the one output without BF16 factors: it can
+  // cancel to any size, so it stays in FP64 up to the output (a block's partial is two floats)
+  double sum_f = 0.0;
 #pragma unroll
   for (int c = 0; c < CI; ++c)
 #pragma unroll
@@ -486,21 +490,16 @@ __global__ __launch_bounds__(256) void k_wgrad_thin(int H, int W, int B, const _
           accb[1] += v1;
         }
       }
-      if constexpr (TAIL) {  // the row's own 16 pixels of F, in pairs, then to the FP64 sum
-        float r[CT];
+      if constexpr (TAIL) {  // the row's own 16 pixels of F
 #pragma unroll
-        for (int x = 0; x < CT; ++x) r[x] = (gy < H && tx0 + x < W) ? f[1][x + 1] : 0.0f;
-#pragma unroll
-        for (int n = CT / 2; n > 0; n >>= 1)
-#pragma unroll
-          for (int x = 0; x < n; ++x) r[x] += r[x + n];
-        sum_f += (double)r[0];
+        for (int x = 0; x < CT; ++x) sum_f += (gy < H && tx0 + x < W) ? (double)f[1][x + 1] : 0.0;
       }
     }
   }
   if constexpr (TAIL) {
     sum_f += __shfl_xor(sum_f, 16);
     sum_f += __shfl_xor(sum_f, 32);
+    if (lane == 0) red_f[wv] = sum_f;
   }
   // the wave's four rows ((0 + 1) + (2 + 3)), then the waves in order
   auto rows = [](float v) {
@@ -509,7 +508,7 @@ __global__ __launch_bounds__(256) void k_wgrad_thin(int H, int W, int B, const _
   };
 #pragma unroll
   for (int k = 0; k < 2; ++k) {
-    accb[k] = TAIL ? (float)sum_f : rows(accb[k]);
+    if (!TAIL) accb[k] = rows(accb[k]);
 #pragma unroll
     for (int c = 0; c < CI; ++c)
 #pragma unroll
@@ -528,10 +527,14 @@ __global__ __launch_bounds__(256) void k_wgrad_thin(int H, int W, int B, const _
           const int o = TAIL ? (8 - t) * NCH + ch : (ch * 9 + t) * CI + c;
           red[o] = (w ? red[o] : 0.0f) + acc[c][k][t];
         }
-      if (!TAIL || (k == 0 && cp == 0)) {
-        const int o = NW + (TAIL ? 0 : ch);
-        red[o] = (w ? red[o] : 0.0f) + accb[k];
-      }
+      if constexpr (!TAIL) red[NW + ch] = (w ? red[NW + ch] : 0.0f) + accb[k];
+    }
+  }
+  if constexpr (TAIL) {
+    if (threadIdx.x == 0) {
+      const double f = (red_f[0] + red_f[1]) + (red_f[2] + red_f[3]);
+      red[NW] = (float)f;
+      red[NW + 1] = (float)(f - (double)red[NW]);
     }
   }
   __syncthreads();
@@ -693,7 +696,8 @@ __global__ __launch_bounds__(WG_T, 4) void k_wgrad32_mfma(int H, int W, int B, c
   }
 }
 
-// out[o] = sum over blocks b of partials[b][o] in a fixed order (deterministic): a workgroup of 1024
+// out[o] = sum over blocks b of partials[b][o], rows of `row` floats (nout, or nout + 1 with the last
+// output's low parts behind it), in a fixed order (deterministic): a workgroup of 1024
 // threads takes OUTS consecutive outputs (coalesced rows of the partials); strand s of 1024/OUTS
 // sums the blocks b = s, s + strands, ..., eight loads in flight, then the strands' sums are added
 // in order.  OUTS = 64 for the 9248 outputs of the 32 -> 32 layers, 16 for the few hundred of the
@@ -701,22 +705,26 @@ __global__ __launch_bounds__(WG_T, 4) void k_wgrad32_mfma(int H, int W, int B, c
 // 42 us on average over a training step's calls).
 template <int OUTS>
 __global__ __launch_bounds__(1024) void k_reduce_partials(const float* __restrict__ partials, int nblocks,
-                                                          int nout, float* __restrict__ out) {
+                                                          int nout, int row, float* __restrict__ out) {
   constexpr int STR = 1024 / OUTS;
   __shared__ double sh[STR][OUTS];
   const int c = threadIdx.x % OUTS, r = threadIdx.x / OUTS;
   const int o = blockIdx.x * OUTS + c;
   double s = 0.0;  // FP64: the sums of a bias gradient cancel, and the adds hide behind the loads
-  if (o < nout) {
+  auto column = [&](int col) {
     int b = r;
     for (; b + 7 * STR < nblocks; b += 8 * STR) {
       float v[8];
 #pragma unroll
-      for (int k = 0; k < 8; ++k) v[k] = partials[(size_t)(b + k * STR) * nout + o];
+      for (int k = 0; k < 8; ++k) v[k] = partials[(size_t)(b + k * STR) * row + col];
 #pragma unroll
       for (int k = 0; k < 8; ++k) s += (double)v[k];
     }
-    for (; b < nblocks; b += STR) s += (double)partials[(size_t)b * nout + o];
+    for (; b < nblocks; b += STR) s += (double)partials[(size_t)b * row + col];
+  };
+  if (o < nout) {
+    column(o);
+    if (o == nout - 1 && row > nout) column(nout);
   }
   sh[r][c] = s;
   __syncthreads();
@@ -933,8 +941,9 @@ int sk_conv_wgrad(sk_ctx* ctx, int kind, int B, int H, int W, const void* g, con
   const int nblocks = (int)std::min<long>(ntiles, cap);
   const int nout = kind == 0 ? NCH * 9 + NCH
                              : (kind == 1 ? NCH * 9 * NCH + NCH : (kind == 2 ? 9 * NCH + 1 : NCH * 9 * 2 + NCH));
+  const int row = nout + (kind == 2 ? 1 : 0);  // floats of a block's partial
   void* ws = nullptr;
-  rc = scratch(c, sizeof(float) * (size_t)nblocks * nout, s, &ws);
+  rc = scratch(c, sizeof(float) * (size_t)nblocks * row, s, &ws);
   if (rc) return rc;
   float* part = (float*)ws;
   const __bf16* Mk = (const __bf16*)mask;
@@ -953,9 +962,11 @@ int sk_conv_wgrad(sk_ctx* ctx, int kind, int B, int H, int W, const void* g, con
   rc = launched(c, "wgrad kernel");
   if (rc) return rc;
   if (nout > 1024)
-    hipLaunchKernelGGL(k_reduce_partials<64>, dim3((nout + 63) / 64), dim3(1024), 0, s, part, nblocks, nout, out);
+    hipLaunchKernelGGL(k_reduce_partials<64>, dim3((nout + 63) / 64), dim3(1024), 0, s, part, nblocks, nout, row,
+                       out);
   else
-    hipLaunchKernelGGL(k_reduce_partials<16>, dim3((nout + 15) / 16), dim3(1024), 0, s, part, nblocks, nout, out);
+    hipLaunchKernelGGL(k_reduce_partials<16>, dim3((nout + 15) / 16), dim3(1024), 0, s, part, nblocks, nout, row,
+                       out);
   return launched(c, "partials reduction kernel");
 }
 

@@ -82,3 +82,19 @@ def test_masked_data_gradients_equal_masking_afterwards(ctx, B, H, W):
     nat.check(L.sk_conv_in_dgrad(c, B, H, W, _ptr(a), _ptr(h), _ptr(w1), _ptr(d0), st), c)
     nat.check(L.sk_conv_in_dgrad_relu(c, 1, B, H, W, _ptr(b), _ptr(w1), _ptr(d1), st), c)
     assert torch.equal(d0, d1)
+
+
+# Sums that cancel to about 1e-6 of their terms: partials of two floats and FP64 sums keep 2^-40 of
+# the terms, so the output is the FP64 sum rounded once (6e-8) or beside it (1.2e-7).
+@pytest.mark.parametrize("B,H,W", [(1, 66, 66), (2, 17, 33), (5, 256, 256)])
+def test_last_layers_bias_gradient_cancels_in_64_bits(ctx, B, H, W):
+    from synkrotomo_amd import _native as nat
+    from synkrotomo_amd.projector import _ptr, _stream
+    g = torch.randn((B, H, W, 1), device="cuda", generator=torch.Generator(device="cuda").manual_seed(W))
+    g.view(-1)[7] -= g.double().sum().float() + 1e-3
+    x = torch.zeros((B, H, W, 32), device="cuda", dtype=torch.bfloat16)
+    out = torch.empty(9 * 32 + 1, device="cuda")
+    nat.check(nat.lib().sk_conv_wgrad(ctx.handle, 2, B, H, W, _ptr(g), None, _ptr(x), _ptr(out),
+                                      _stream(ctx.device)), ctx.handle, "wgrad")
+    want = g.double().sum().item()
+    assert want != 0.0 and abs(out[-1].item() - want) <= 1.2e-7 * abs(want)
