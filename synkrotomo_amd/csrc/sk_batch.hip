@@ -7,18 +7,17 @@
 // launches sized to fill the chip once: in k_fpg_persist (fast mode) every workgroup pulls
 // (problem, images, line group, 64-bin block) items of the grouped staged forward projector
 // from a global work counter (k_fps_persist: (problem, image, line, 256-bin block) items of
-// the one-line staged kernel) (k_fp_persist: waves pull 64-bin items of the per-wave walk, exact mode or
-// segments wider than the staging buffer); in k_bp_persist every block pulls (problem,
-// image, tile) items, queued largest-problem first so the tail of the queue is made of the
-// shortest items.  The fp kernel resets the bp counter and the
-// bp kernel the fp slot, so the whole iteration sequence (a reset kernel, then fp/bp pairs)
-// is captured once into a hipGraph and launched once.
+// the one-line staged kernel; k_fp_persist: waves pull 64-bin items of the per-wave walk, exact
+// mode or segments wider than the staging buffer); in k_bp_persist every block pulls (problem,
+// images, tile) items, queued largest-problem first so the tail of the queue is made of the
+// shortest items.  The fp kernel resets the bp counter and the bp kernel the fp slot, so the
+// whole iteration sequence (a reset kernel, then fp/bp pairs) is captured once into a hipGraph
+// and launched once.
 //
 // Autotuner: times the fp variants (per-wave kernels with 1, 2 or 4 rays per lane, staged
-// kernels) and the bp variants (16x16,
-// 16x32 or 16x64 pixel tiles) on a geometry with HIP events and keeps the fastest.  All
-// variants evaluate the same expressions in the same order per ray and per pixel, so the
-// choice never changes results.
+// kernels) and the bp variants (16x16, 16x32 or 16x64 pixel tiles) on a geometry with HIP events
+// and keeps the fastest.  All variants evaluate the same expressions in the same order per ray
+// and per pixel, so the choice never changes results.
 #include <algorithm>
 #include <cstdlib>
 #include <vector>

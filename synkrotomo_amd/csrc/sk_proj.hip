@@ -20,6 +20,8 @@
 //               lines adjacent in slope, 16 bins of each line per wave, so the staged segment
 //               of a block is two to four chunks of 64 columns instead of six; blocks of 16
 //               rows.  Same walk, for 1, 2 or 4 images at once.
+//   k_fp_lds    A.x of images up to 80 x 80: the whole image in LDS, the per-wave walk from there.
+//   k_fp_listed, k_bpt_rims  the rays of B^T that A.x does not give (launch_fp_bpt).
 //
 // The work items themselves live in sk_kern.h (shared with the persistent kernels).
 // With SK_OPT_EXACT the results are bitwise those of the sequential FP32 restatement of
@@ -64,12 +66,54 @@ __global__ __launch_bounds__(FP_BLOCK) void k_fp(FpParams P) {
     fp_item<EXACT, MODE, WEIGHTS, DR1, RPT>(P, blockIdx.x, blockIdx.y * FP_WAVES + wave, blockIdx.z);
 }
 
-// The walk of k_fp with the backprojector's lengths over the listed lines (B^T of the degenerate
-// lines).  Grid (bin blocks, listed lines, images).
+// B^T of the listed (degenerate) lines: every row of 64 bins with the backprojector's lengths.  Few
+// rays and two gathers a row, so latency bounds it: LISTED_WAVES waves of a workgroup take a run of
+// the rows each, four rows' loads in flight, and their sums are added in order.  B^T of 8 images of
+// 512^2, 360 angles, two of them such lines: 355 us with one wave walking all rows, 199 us like this
+// (A.x: 199).  Grid (bins / 64, listed lines, images).
+constexpr int LISTED_WAVES = 16;
 template <bool DR1>
-__global__ __launch_bounds__(FP_BLOCK) void k_fp_listed(FpParams P, const int* __restrict__ list) {
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  fp_item<false, FP_PLAIN, W_ADJ, DR1, 1>(P, list[blockIdx.y], blockIdx.x * FP_WAVES + wave, blockIdx.z);
+__global__ __launch_bounds__(64 * LISTED_WAVES) void k_fp_listed(FpParams P, const int* __restrict__ list) {
+  __shared__ float part[LISTED_WAVES][64];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const Line L = P.lines[list[blockIdx.y]];
+  const int N = P.N, h = N >> 1;
+  const int first = blockIdx.x * 64, r = first + lane, last = min(first + 63, P.R - 1);
+  const float icpt = (P.rho0 + (float)r * P.drho) / L.cost;  // forwardprojection.fut:33-34
+  int a0, a1, b0, b1;
+  row_clip(L.slope, (P.rho0 + (float)first * P.drho) / L.cost, h, a0, a1);
+  row_clip(L.slope, (P.rho0 + (float)last * P.drho) / L.cost, h, b0, b1);
+  const int i0 = __builtin_amdgcn_readfirstlane(min(a0, b0)), i1 = __builtin_amdgcn_readfirstlane(max(a1, b1));
+  const int run = (max(i1 - i0, 0) + LISTED_WAVES - 1) / LISTED_WAVES;
+  const int w0 = i0 + run * wave, w1 = min(w0 + run, i1);
+  const float* src = ((L.flags & LINE_FLAT) ? P.imgT : P.img) + (size_t)blockIdx.z * N * N;
+  float sum = 0.0f;
+  for (int i = w0; i < w1; i += 4) {
+    float xbot[4], vb[4], vt[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {  // rows past the run: an empty descriptor reads 0
+      xbot[q] = (float)(i + q) * L.slope + icpt;
+      const __amdgpu_buffer_rsrc_t row = row_rsrc(src + (size_t)(i + h + q) * N, i + q < w1 ? N : 0);
+      vb[q] = row_load(row, (int)floorf(xbot[q]) + h);
+      vt[q] = row_load(row, (int)floorf(xbot[q] + L.slope) + h);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if (i + q >= w1) break;  // uniform
+      const float xtop = xbot[q] + L.slope;
+      const int Xb = (int)floorf(xbot[q]), Xt = (int)floorf(xtop);
+      auto term = [&](int X, float v) {
+        const float len = bp_entry<false, DR1>(L, X, (float)(i + q), xbot[q], xtop, r, P.ncand, P.rho0, P.drho);
+        return (unsigned)(X + h) < (unsigned)N ? len * v : 0.0f;
+      };
+      sum = sum + (term(Xb, vb[q]) + (Xb == Xt ? 0.0f : term(Xt, vt[q])));
+    }
+  }
+  part[wave][lane] = sum;
+  __syncthreads();
+  if (wave != 0 || r >= P.R) return;
+  for (int w = 1; w < LISTED_WAVES; ++w) sum = sum + part[w][lane];
+  P.out[(size_t)blockIdx.z * P.A * P.R + (size_t)L.orig * P.R + r] = sum;
 }
 
 // B^T at the image's corners: the rays of every line that cross less than two pixels' length, with
@@ -78,7 +122,7 @@ __global__ __launch_bounds__(FP_BLOCK) void k_fp_listed(FpParams P, const int* _
 // sum of 1e-3 (the gradient of a SIRT step) that is 6e-5 of the result.  The outermost corner of a
 // line is at (frame) x = -+h, y = -+h by the signs of cost and sint; a chord at distance d from
 // it is d/|cost*sint| long and lies in the last rows there.  per_end bins from each end's corner on.
-// 8 images of 512^2, 360 angles: 6 us of 330.
+// 8 images of 512^2, 360 angles: 6 us of 199.
 constexpr int RIM_ROWS = 4;  // two rows of a chord (|slope| <= 1), the one it ends in, one for rounding
 template <bool DR1>
 __global__ __launch_bounds__(256) void k_bpt_rims(FpParams P, int per_end) {
@@ -220,8 +264,6 @@ __global__ __launch_bounds__(FPS_RAYS) void k_fp_staged(FpParams P) {
   fps_item<MODE, NBUF>(P, blockIdx.x, blockIdx.y, blockIdx.z, (float*)seg4);
 }
 
-// Grouped staged A.x (variant 7): grid (line groups, bin blocks of FPG_BINS, images).
-// Dynamic LDS: NBUF * (FPG_ROWS + 1) * 64 * (the geometry's largest CPL) floats.
 // Grouped staged A.x (variant 7) of S images at once: grid (line groups, bin blocks of FPG_BINS,
 // images / S).  CPLMAX: the largest chunk count of the geometry's groups.  Dynamic LDS:
 // fpg_lds_floats.
@@ -412,9 +454,8 @@ int launch_fp(Ctx* c, const Geom* g, FpMode mode, const FpArgs& a, hipStream_t s
 // one of the pixel's candidates): those lines are A.v, by whichever kernel A.x runs, but for the
 // short rays at the image's corners (k_bpt_rims).  The degenerate lines (theta ~ 0, pi/2: a ray on
 // a pixel edge counts in A and not in B) are walked again with the backprojector's own lengths, one
-// launch over their table indices.  8 images of
-// 512^2, 360 angles: 1249 us with every line on that walk (60 VALU a row and two dependent global
-// gathers), 330 us like this.
+// launch over their table indices.  8 images of 512^2, 360 angles: 1249 us with every line on that
+// walk (60 VALU a row and two dependent global gathers), 199 us like this.
 int launch_fp_bpt(Ctx* c, const Geom* g, const FpArgs& a, hipStream_t s) {
   const bool ex = c->exact != 0 || !g->index_safe;
   const bool dr1 = g->drho == 1.0f;
@@ -434,11 +475,11 @@ int launch_fp_bpt(Ctx* c, const Geom* g, const FpArgs& a, hipStream_t s) {
     hipLaunchKernelGGL((k_bpt_rims<false>), rims, dim3(256), 0, s, P, per_end);
   rc = launched(c, "backprojection-transpose kernel");
   if (rc || !g->n_degen) return rc;
-  const dim3 grid((unsigned)((g->R + FP_BLOCK - 1) / FP_BLOCK), (unsigned)g->n_degen, (unsigned)a.batch);
+  const dim3 grid((unsigned)((g->R + 63) / 64), (unsigned)g->n_degen, (unsigned)a.batch);
   if (dr1)
-    hipLaunchKernelGGL((k_fp_listed<true>), grid, dim3(FP_BLOCK), 0, s, P, g->d_degen);
+    hipLaunchKernelGGL((k_fp_listed<true>), grid, dim3(64 * LISTED_WAVES), 0, s, P, g->d_degen);
   else
-    hipLaunchKernelGGL((k_fp_listed<false>), grid, dim3(FP_BLOCK), 0, s, P, g->d_degen);
+    hipLaunchKernelGGL((k_fp_listed<false>), grid, dim3(64 * LISTED_WAVES), 0, s, P, g->d_degen);
   return launched(c, "backprojection-transpose kernel");
 }
 
