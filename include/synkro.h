@@ -196,7 +196,8 @@ int sk_conv_in2_dgrad(sk_ctx* ctx, int B, int H, int W, const void* dh, const vo
                       const void* w, float* dx2, void* stream);
 /* The same data gradients with the ReLU derivative of the layer below in the output, so that the
  * kernels that read it next need no mask: dh (BF16) is zeroed where h, that layer's activation, is
- * <= 0.  sk_conv_in_dgrad_relu takes such a gradient g: dx[_2] [B][H][W][cin], cin 1 or 2. */
+ * <= 0.  w: the layer's forward weights (sk_conv32_dgrad_relu flips and transposes them itself).
+ * sk_conv_in_dgrad_relu takes such a gradient g: dx[_2] [B][H][W][cin], cin 1 or 2. */
 int sk_conv_out_dgrad_relu(sk_ctx* ctx, int B, int H, int W, const float* g, const void* w, const void* h,
                            void* dh, void* stream);
 int sk_conv32_dgrad_relu(sk_ctx* ctx, int B, int H, int W, const void* g, const void* w, const void* h,

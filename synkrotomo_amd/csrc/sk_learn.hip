@@ -12,8 +12,11 @@
 //                 blocks compute 16x16-pixel x 32-channel tiles from an LDS-staged 18x18x32
 //                 input patch (the next tile's patch loaded during the MFMAs) and the 32x9x32
 //                 weights, staged once per block.  The same kernel computes the data
-//                 gradient (weights flipped and transposed on the host side), with the ReLU
-//                 derivative of the layer's output fused into the staging of its input.
+//                 gradient: with weights that the caller flipped and transposed, the ReLU derivative
+//                 of the layer's output in the staging of its input (mask); or with the forward
+//                 weights, flipped while they are staged, and the derivative of the layer below in
+//                 its output (omask; four library launches less in a backward pass of the
+//                 network: 285 and 259 us for one of 7 images of 86^2, where launches count).
 //   k_conv_in     1 or 2 -> 32 (288 MACs per pixel and input channel) on VALU with fused bias and
 //                 ReLU, in FP32 on the FP32 input (the image, or the image and the SIRT update
 //                 direction interleaved); the data gradient of the last layer likewise.
@@ -67,7 +70,13 @@ __global__ __launch_bounds__(256) void k_conv32(int H, int W, long ntiles, const
   const long tiles_img = (long)tiles_x * ((H + CT - 1) / CT);
   for (int c = threadIdx.x; c < NCH * 9 * 4; c += 256) {
     const int row = c >> 2, q = c & 3;  // row = co*9 + tap
-    *(bf16x8*)(sw + row * CP + q * 8) = *(const bf16x8*)(w + row * NCH + q * 8);
+    const bf16x8 v = *(const bf16x8*)(w + row * NCH + q * 8);
+    if constexpr (MASK_OUT) {  // a data gradient: the forward weights flipped and transposed
+      const int co = row / 9, tap = row - 9 * co;
+      for (int i = 0; i < 8; ++i) sw[((q * 8 + i) * 9 + 8 - tap) * CP + co] = v[i];
+    } else {
+      *(bf16x8*)(sw + row * CP + q * 8) = v;
+    }
   }
   bf16x8 pf[PATCH_PER_T];
   auto load_patch = [&](long t) {

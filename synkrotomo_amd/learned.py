@@ -107,13 +107,11 @@ class _Correction(torch.autograd.Function):
         _chk(L.sk_conv_out_dgrad_relu(h, B, H, W, _ptr(gy), _ptr(w4b), _ptr(h3), _ptr(dh3), s), ctx, "conv4 dgrad")
         # conv3, conv2 (32 -> 32)
         g3 = wgrad(1, dh3, h2, NCH * 9 * NCH + NCH)
-        w3t = w3b.flip(1, 2).permute(3, 1, 2, 0).contiguous()
         dh2 = torch.empty_like(h2)
-        _chk(L.sk_conv32_dgrad_relu(h, B, H, W, _ptr(dh3), _ptr(w3t), _ptr(h2), _ptr(dh2), s), ctx, "conv3 dgrad")
+        _chk(L.sk_conv32_dgrad_relu(h, B, H, W, _ptr(dh3), _ptr(w3b), _ptr(h2), _ptr(dh2), s), ctx, "conv3 dgrad")
         g2 = wgrad(1, dh2, h1, NCH * 9 * NCH + NCH)
-        w2t = w2b.flip(1, 2).permute(3, 1, 2, 0).contiguous()
         dh1 = torch.empty_like(h1)
-        _chk(L.sk_conv32_dgrad_relu(h, B, H, W, _ptr(dh2), _ptr(w2t), _ptr(h1), _ptr(dh1), s), ctx, "conv2 dgrad")
+        _chk(L.sk_conv32_dgrad_relu(h, B, H, W, _ptr(dh2), _ptr(w2b), _ptr(h1), _ptr(dh1), s), ctx, "conv2 dgrad")
         # conv1 (cin -> 32)
         n1 = NCH * 9 * cin
         g1 = wgrad(0 if cin == 1 else 3, dh1, inp, n1 + NCH)

@@ -74,7 +74,8 @@ def test_masked_data_gradients_equal_masking_afterwards(ctx, B, H, W):
     nat.check(L.sk_conv_out_dgrad_relu(c, B, H, W, _ptr(g), _ptr(w4), _ptr(h), _ptr(b), st), c)
     assert torch.equal(torch.where(h > 0, a, zero), b)
     x, w = rnd(B, H, W, 32).to(torch.bfloat16), rnd(32, 9, 32).to(torch.bfloat16)
-    nat.check(L.sk_conv32(c, B, H, W, _ptr(x), None, _ptr(w), None, _ptr(a), st), c)
+    wt = w.flip(1).permute(2, 1, 0).contiguous()
+    nat.check(L.sk_conv32(c, B, H, W, _ptr(x), None, _ptr(wt), None, _ptr(a), st), c)
     nat.check(L.sk_conv32_dgrad_relu(c, B, H, W, _ptr(x), _ptr(w), _ptr(h), _ptr(b), st), c)
     assert torch.equal(torch.where(h > 0, a, zero), b)
     w1 = rnd(32, 9).to(torch.bfloat16)
