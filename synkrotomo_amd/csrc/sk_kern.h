@@ -67,6 +67,17 @@ __device__ __forceinline__ void row_clip(float slope, float icpt, int h, int& i0
   i1 = min(h, (int)ceilf(tmax) + 3);
 }
 
+// The frame rows [i0, i1) in which a ray of a line that is not degenerate can cross the image, one
+// more at each end: row i spans x from i*slope + icpt to slope more, and crosses where that meets
+// [-h, h].  The image is taken 1e-6 wider for the rounding of the intercept and of x (below 3e-7*h
+// together for |x| <= h + 1), whose effect on the row grows as 1/|slope|.
+__device__ __forceinline__ void row_span(float slope, float icpt, int h, int& i0, int& i1) {
+  const float w = (float)h * 1.000001f;
+  const float ta = (-w - icpt) / slope, tb = (w - icpt) / slope;
+  i0 = max(-h, (int)floorf(fmaxf(fminf(ta, tb), -(float)h)) - 1);
+  i1 = min(h, (int)ceilf(fminf(fmaxf(ta, tb), (float)h)) + 1);
+}
+
 // First candidate ray of a pixel (backprojection.fut:51-54).
 template <bool DR1>
 __device__ __forceinline__ float cand_s(const Line& L, float xmin, float ymin, float rho0,

@@ -121,9 +121,11 @@ __global__ __launch_bounds__(64 * LISTED_WAVES) void k_fp_listed(FpParams P, con
 // row's length outside gets its short part from 1 - f, 6e-8 off however short, and divided by a row
 // sum of 1e-3 (the gradient of a SIRT step) that is 6e-5 of the result.  The outermost corner of a
 // line is at (frame) x = -+h, y = -+h by the signs of cost and sint; a chord at distance d from
-// it is d/|cost*sint| long and lies in the last rows there.  per_end bins from each end's corner on.
-// 8 images of 512^2, 360 angles: 6 us of 199.
-constexpr int RIM_ROWS = 4;  // two rows of a chord (|slope| <= 1), the one it ends in, one for rounding
+// it is d/|cost*sint| long.  per_end bins from each end's corner on.  d only picks the rays (FP32:
+// on a nearly axis-parallel line its error can exceed the whole range of short chords); the rows of
+// a picked ray come from its own intercept, and one that crosses more of them than a short chord
+// can is left as it is, A.x being right for it.  8 images of 512^2, 360 angles: 6 us of 199.
+constexpr int RIM_ROWS = 32;  // a short chord: 3 rows, one more at each end, and 2e-6*h/|slope| <= 17 for rounding
 template <bool DR1>
 __global__ __launch_bounds__(256) void k_bpt_rims(FpParams P, int per_end) {
   const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x;
@@ -140,10 +142,11 @@ __global__ __launch_bounds__(256) void k_bpt_rims(FpParams P, int per_end) {
   if (r < 0 || r >= P.R) return;
   const float d = (high ? edge - (float)r : (float)r - edge) * P.drho;
   if (d > 2.0f * fabsf(L.cost * L.sint)) return;
-  const bool upper = (L.sint > 0.0f) == high;  // the corner's rows
-  const int i0 = upper ? max(h - RIM_ROWS, -h) : -h, i1 = min(i0 + RIM_ROWS, h);
-  const float* src = ((L.flags & LINE_FLAT) ? P.imgT : P.img) + (size_t)blockIdx.y * N * N;
   const float icpt = (P.rho0 + (float)r * P.drho) / L.cost;  // forwardprojection.fut:33-34
+  int i0, i1;
+  row_span(L.slope, icpt, h, i0, i1);
+  if (i1 - i0 > RIM_ROWS) return;
+  const float* src = ((L.flags & LINE_FLAT) ? P.imgT : P.img) + (size_t)blockIdx.y * N * N;
   float sum = 0.0f;
   for (int i = i0; i < i1; ++i) {
     const float xbot = (float)i * L.slope + icpt, xtop = xbot + L.slope;
