@@ -21,7 +21,7 @@
 //               of a block is two to four chunks of 64 columns instead of six; blocks of 16
 //               rows.  Same walk, for 1, 2 or 4 images at once.
 //   k_fp_lds    A.x of images up to 80 x 80: the whole image in LDS, the per-wave walk from there.
-//   k_fp_listed, k_bpt_rims  the rays of B^T that A.x does not give (launch_fp_bpt).
+//   k_fp_listed, k_bpt_rays  the rays of B^T that A.x does not give (launch_fp_bpt).
 //
 // The work items themselves live in sk_kern.h (shared with the persistent kernels).
 // With SK_OPT_EXACT the results are bitwise those of the sequential FP32 restatement of
@@ -116,37 +116,36 @@ __global__ __launch_bounds__(64 * LISTED_WAVES) void k_fp_listed(FpParams P, con
   P.out[(size_t)blockIdx.z * P.A * P.R + (size_t)L.orig * P.R + r] = sum;
 }
 
-// B^T at the image's corners: the rays of every line that cross less than two pixels' length, with
-// the backprojector's lengths.  A.x forms a row as vb + f*(vo - vb): a ray that leaves most of a
-// row's length outside gets its short part from 1 - f, 6e-8 off however short, and divided by a row
-// sum of 1e-3 (the gradient of a SIRT step) that is 6e-5 of the result.  The outermost corner of a
-// line is at (frame) x = -+h, y = -+h by the signs of cost and sint; a chord at distance d from
-// it is d/|cost*sint| long.  per_end bins from each end's corner on.  d only picks the rays (FP32:
-// on a nearly axis-parallel line its error can exceed the whole range of short chords); the rows of
-// a picked ray come from its own intercept, and one that crosses more of them than a short chord
-// can is left as it is, A.x being right for it.  8 images of 512^2, 360 angles: 6 us of 199.
+// B^T of the rays for which A.x does not do, with the backprojector's lengths; one thread a ray of a
+// line that is not degenerate, the row sums in order.  A.x forms a row as vb + f*(vo - vb):
+// - A ray that leaves most of a row's length outside gets its short part from 1 - f, 6e-8 off however
+//   short, and divided by a row sum of 1e-3 (the gradient of a SIRT step) that is 6e-5 of the
+//   result: rays that cross less than two pixels' length.  The outermost corners of a line are at
+//   (frame) x = -+h, y = -+h by the signs of cost and sint; a chord at distance d from one is
+//   d/|cost*sint| long.  d only picks the rays (FP32: on a nearly axis-parallel line its error can
+//   exceed the whole range of short chords); the rows come from the ray's own intercept, and a ray
+//   that crosses more of them than a short chord can is left as it is, A.x being right for it.
+// - A pixel that is not finite, or two whose difference overflows, reach every ray that passes beside
+//   them (0*inf), and A.x is then not finite, whatever follows: those rays are walked again.
+// Two divisions, a load and a store's mask per ray: 8 images of 512^2, 360 angles: 6 us of 199.
 constexpr int RIM_ROWS = 32;  // a short chord: 3 rows, one more at each end, and 2e-6*h/|slope| <= 17 for rounding
 template <bool DR1>
-__global__ __launch_bounds__(256) void k_bpt_rims(FpParams P, int per_end) {
-  const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x;
-  const size_t line = t / (2 * per_end);
-  if (line >= (size_t)P.A) return;
-  const int q = (int)(t - line * (2 * per_end));
-  const bool high = q >= per_end;
-  const Line L = P.lines[line];
-  if (L.flags & LINE_DEGEN) return;
+__global__ __launch_bounds__(256) void k_bpt_rays(FpParams P) {
+  const Line L = P.lines[blockIdx.y];
+  const int r = (int)(blockIdx.x * 256 + threadIdx.x);
+  if (r >= P.R || (L.flags & LINE_DEGEN)) return;
   const int N = P.N, h = N >> 1;
+  float* out = P.out + (size_t)blockIdx.z * P.A * P.R + (size_t)L.orig * P.R + r;
+  const bool finite = (__builtin_bit_cast(unsigned, *out) & 0x7f800000u) != 0x7f800000u;
   const float reach = (float)h * (fabsf(L.cost) + fabsf(L.sint));
-  const float edge = ((high ? reach : -reach) - P.rho0) / P.drho;  // bin of the corner
-  const int r = high ? (int)ceilf(edge) - (q - per_end) : (int)floorf(edge) + q;
-  if (r < 0 || r >= P.R) return;
-  const float d = (high ? edge - (float)r : (float)r - edge) * P.drho;
-  if (d > 2.0f * fabsf(L.cost * L.sint)) return;
+  const float low = (-reach - P.rho0) / P.drho, high = (reach - P.rho0) / P.drho;  // bins of the corners
+  const float d = fminf((float)r - low, high - (float)r) * P.drho;
+  if (finite && d > 2.0f * fabsf(L.cost * L.sint)) return;
   const float icpt = (P.rho0 + (float)r * P.drho) / L.cost;  // forwardprojection.fut:33-34
   int i0, i1;
   row_span(L.slope, icpt, h, i0, i1);
-  if (i1 - i0 > RIM_ROWS) return;
-  const float* src = ((L.flags & LINE_FLAT) ? P.imgT : P.img) + (size_t)blockIdx.y * N * N;
+  if (finite && (i0 >= i1 || i1 - i0 > RIM_ROWS)) return;
+  const float* src = ((L.flags & LINE_FLAT) ? P.imgT : P.img) + (size_t)blockIdx.z * N * N;
   float sum = 0.0f;
   for (int i = i0; i < i1; ++i) {
     const float xbot = (float)i * L.slope + icpt, xtop = xbot + L.slope;
@@ -157,7 +156,7 @@ __global__ __launch_bounds__(256) void k_bpt_rims(FpParams P, int per_end) {
     };
     sum = sum + (part(Xb) + (Xb == Xt ? 0.0f : part(Xt)));
   }
-  P.out[(size_t)blockIdx.y * P.A * P.R + (size_t)L.orig * P.R + r] = sum;
+  *out = sum;
 }
 
 // --------------------------------------------------------- small images (fast mode)
@@ -455,7 +454,7 @@ int launch_fp(Ctx* c, const Geom* g, FpMode mode, const FpArgs& a, hipStream_t s
 // pixel is the forward projector's (both are the part of the row's x-range inside the pixel over
 // the range, and a ray with a nonzero length lies within sqrt(2)/2 of the pixel's centre, so it is
 // one of the pixel's candidates): those lines are A.v, by whichever kernel A.x runs, but for the
-// short rays at the image's corners (k_bpt_rims).  The degenerate lines (theta ~ 0, pi/2: a ray on
+// short rays at the image's corners and those that are not finite (k_bpt_rays).  The degenerate lines (theta ~ 0, pi/2: a ray on
 // a pixel edge counts in A and not in B) are walked again with the backprojector's own lengths, one
 // launch over their table indices.  8 images of 512^2, 360 angles: 1249 us with every line on that
 // walk (60 VALU a row and two dependent global gathers), 199 us like this.
@@ -468,14 +467,12 @@ int launch_fp_bpt(Ctx* c, const Geom* g, const FpArgs& a, hipStream_t s) {
   }
   int rc = launch_fp(c, g, FP_PLAIN, a, s);
   if (rc) return rc;
-  // a chord of two pixels lies within a distance of 1 of its corner (|cost*sint| <= 1/2)
-  const int per_end = (int)fmin(ceil(1.0 / g->drho) + 2.0, (double)g->R);
   const FpParams P = fp_params(g, a);
-  const dim3 rims((unsigned)(((size_t)g->A * 2 * per_end + 255) / 256), (unsigned)a.batch);
+  const dim3 rays((unsigned)((g->R + 255) / 256), (unsigned)g->A, (unsigned)a.batch);
   if (dr1)
-    hipLaunchKernelGGL((k_bpt_rims<true>), rims, dim3(256), 0, s, P, per_end);
+    hipLaunchKernelGGL((k_bpt_rays<true>), rays, dim3(256), 0, s, P);
   else
-    hipLaunchKernelGGL((k_bpt_rims<false>), rims, dim3(256), 0, s, P, per_end);
+    hipLaunchKernelGGL((k_bpt_rays<false>), rays, dim3(256), 0, s, P);
   rc = launched(c, "backprojection-transpose kernel");
   if (rc || !g->n_degen) return rc;
   const dim3 grid((unsigned)((g->R + 63) / 64), (unsigned)g->n_degen, (unsigned)a.batch);

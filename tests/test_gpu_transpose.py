@@ -29,3 +29,41 @@ def test_transpose_far_from_the_detectors_first_bin(ctx, N, rz, dr, R, angles):
     ref = np.bincount(c, weights=vals.astype(np.float64), minlength=ang.size * R)
     assert (ref > 2).sum() > 20
     np.testing.assert_allclose(got, ref, rtol=5e-6, atol=1e-5)
+
+
+# Pixels that are not finite, and neighbours of either sign whose difference overflows: a ray is as the
+# matrix has it -- infinite or NaN where it crosses such a pixel, and elsewhere the sum of the
+# pixels it does cross -- in every kernel of A.x (the image in LDS, one image, four at a time, per
+# wave).  No angle is a multiple of 45 degrees, so no ray lies on pixel edges or corners.  Finite
+# rays: 4.8e-7 and 6e-8 per addition of the sum of magnitudes, at most 3 N / 2 entries.
+@pytest.mark.parametrize("N,A,R,dr,batch,variant", [(64, 20, 91, 1.0, 1, -1), (130, 30, 185, 1.0, 1, 7),
+                                                    (130, 30, 140, 1.4, 1, 3), (440, 37, 631, 1.0, 5, -1),
+                                                    (66, 11, 420, 0.25, 2, -1)])
+def test_transpose_of_pixels_that_are_not_finite(ctx, N, A, R, dr, batch, variant):
+    ang = ((np.arange(A) + 0.37) * np.pi / A).astype(np.float32)
+    rz = -(R - 1) / 2 * dr + 0.3
+    rng = np.random.default_rng(N)
+    v = rng.standard_normal((batch, N, N)).astype(np.float32)
+    v[0, N // 2, N // 3] = np.inf
+    v[0, N // 4, N // 2 + 1] = -np.inf
+    v[0, 0, 0] = np.inf
+    v[-1, N // 3, N // 2] = np.nan
+    v[-1, N - 2, 1:3] = 2e38, -2e38
+    geo = ctx.geometry(ang, rz, dr, R, N)
+    geo.set_variants(variant, -1)
+    try:
+        got = geo.bp_transpose(torch.from_numpy(v).cuda()).cpu().numpy().reshape(batch, -1)
+    finally:
+        geo.set_variants(-1, -1)
+    rp, c, vals = oracle.bp_csr(ang, rz, dr, R, N)
+    rows = np.repeat(np.arange(N * N), np.diff(rp))
+    keep = vals > 0
+    for k in range(batch):
+        x = v[k].ravel().astype(np.float64)[rows[keep]]
+        w = vals[keep].astype(np.float64)
+        bad = np.bincount(c[keep], weights=~np.isfinite(x), minlength=A * R) > 0
+        np.testing.assert_array_equal(~np.isfinite(got[k]), bad)
+        x = np.where(np.isfinite(x), x, 0)
+        ref = np.bincount(c[keep], weights=w * x, minlength=A * R)
+        mag = np.bincount(c[keep], weights=w * np.abs(x), minlength=A * R)
+        assert np.all(np.abs(got[k] - ref)[~bad] <= (4.8e-7 + 1.5 * N * 6e-8) * mag[~bad])
