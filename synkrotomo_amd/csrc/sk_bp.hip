@@ -123,6 +123,15 @@ static void bp_go_nc(const Geom* g, const BpArgs& a, hipStream_t s) {
     else
       bp_go<true, MODE, WEIGHTS, 0, false, PPT>(g, a, s);
   } else {
+    if constexpr (WEIGHTS == W_ADJ) {
+      if (!g->index_safe) {
+        if (g->bp_two_cand)
+          bp_go<false, MODE, W_ADJ, 2, true, 1>(g, a, s);
+        else
+          bp_go<false, MODE, W_ADJ, 0, false, 1>(g, a, s);
+        return;
+      }
+    }
     switch (g->bp_nc) {
       case 1: bp_go<false, MODE, WEIGHTS, 1, false, PPT>(g, a, s); break;
       case 2: bp_go<false, MODE, WEIGHTS, 2, false, PPT>(g, a, s); break;
@@ -175,7 +184,7 @@ int launch_bp(Ctx* c, const Geom* g, BpMode mode, BpWeights w, const BpArgs& a, 
   if (sizeof(float2) * BP_LB * (size_t)bp_window_bins(1, g->drho, g->ncand) > 60 * 1024)
     return fail(c, SK_EINVAL, "backprojection window exceeds LDS (deltarho too small)");
   if (w == W_ADJ && mode != BP_PLAIN) return fail(c, SK_EINVAL, "adjoint weights support plain mode only");
-  const int images = ex || mode == BP_ONES_INV ? 1 : bp_images(g, a.batch);
+  const int images = ex || mode == BP_ONES_INV || (w == W_ADJ && !g->index_safe) ? 1 : bp_images(g, a.batch);
   if (images > 1) {
     if (w == W_ADJ)
       bp_go_images_s<BP_PLAIN, W_ADJ>(images, g, a, s);
@@ -190,7 +199,7 @@ int launch_bp(Ctx* c, const Geom* g, BpMode mode, BpWeights w, const BpArgs& a, 
       case BP_SIRT: bp_go_ex<BP_SIRT, W_REF>(ex, v, g, a, s); break;
     }
   } else {
-    bp_go_ex<BP_PLAIN, W_ADJ>(ex || !g->index_safe, v, g, a, s);
+    bp_go_ex<BP_PLAIN, W_ADJ>(ex, v, g, a, s);
   }
   return launched(c, "backprojection kernel");
 }

@@ -527,12 +527,14 @@ __device__ __forceinline__ void bp_item(const BpParams& P, int tile_x, int tile_
   static_assert(S == 1 || (!EXACT && NC > 0), "several images: the hoisted fast path");
   constexpr int LB = BP_LB;  // the same for every kernel: a block's tie lines are summed at its end
   static_assert(LB <= 64, "one lane per line of a block");
-  // Fast mode: slope sign hoisted per line, lbase folded into the staged value.  W_ADJ takes the
-  // same lengths: on a line that is not degenerate, intersect_fact of a candidate is the forward
-  // projector's length of that ray in that pixel (both are the part of the row's x-range inside
-  // the pixel over the range; neither counts a ray that only touches an edge), so only the
-  // degenerate lines, whose rays can lie on pixel edges, are weighed differently.
-  constexpr bool FASTREF = !EXACT;
+  // Fast mode: slope sign hoisted per line, lbase folded into the staged value.  Hoisted (NC > 0),
+  // W_ADJ takes the same lengths: on a line that is not degenerate, intersect_fact of a candidate
+  // is the forward projector's length of that ray in that pixel (both are the part of the row's
+  // x-range inside the pixel over the range; neither counts a ray that only touches an edge), so
+  // only the degenerate lines, whose rays can lie on pixel edges, are weighed differently.  Where
+  // it does not run hoisted (NC = 0; DR1 with two candidates: the fast index is not safe) W_ADJ
+  // keeps the reference's index and the forward projector's own lengths.
+  constexpr bool FASTREF = !EXACT && !(WEIGHTS == W_ADJ && (NC == 0 || DR1));
   // The hoisted fast path keeps each line's window in descending bin order, so that the
   // candidate address comes from floor(-t) (one conversion) instead of ceil(t).
   constexpr bool REV = FASTREF && NC > 0;
@@ -908,7 +910,10 @@ __device__ __forceinline__ void bp_item(const BpParams& P, int tile_x, int tile_
           const float xbase = ymin * L.slope;  // backprojection.fut:55
           const float2* wrow;
           if constexpr (FASTREF) {
-            // general path (any geometry): the fast index, clamped into the window
+            // general path (any geometry): the fast index, clamped into the window.  The candidates
+            // are read one by one: their number is not known here, and an array of them is scratch
+            // memory (256^2, 89 angles, bins of 0.25, 1 and 16 images: 113 and 978 us, 51 and 194
+            // without it).
             const float t = part == 0 ? fmaf(lc.si, yh[q], tb) : fmaf(lc.ci, xh[q], tb);
             wrow = win + jj * W + min(max((int)ceilf(t) - lc.w0, 0), W - ncand);
           } else {
@@ -922,46 +927,35 @@ __device__ __forceinline__ void bp_item(const BpParams& P, int tile_x, int tile_
             // clamp only guards geometries so far off-centre that rho rounds by whole bins.
             wrow = win + jj * W + min(max((int)ceilf(t) - lc.w0, 0), W - ncand);
           }
-          constexpr int KC = NC > 0 ? NC : 16;
-          float2 ev[KC];  // fast mode: all candidates read before the per-line branches
-          if constexpr (FASTREF) {
-#pragma unroll
-            for (int k = 0; k < KC; ++k)
-              if (NC > 0 || k < ncand) ev[k] = wrow[k];
-          }
           if (FASTREF && !degen) {
             // Non-degenerate lines: max(min(a, b), 0) == med3(a, b, 0) because a and b
             // cannot both be negative when the ray's x-range has positive length; the
             // fraction m/diff is then >= 0, so min(., 1) is a clamp to [0, 1].
             if (pos) {
-#pragma unroll
-              for (int k = 0; k < KC; ++k) {
-                if (NC == 0 && k >= ncand) break;
-                const float xb = xbase + ev[k].x;
+              for (int k = 0; k < ncand; ++k) {
+                const float2 e = wrow[k];
+                const float xb = xbase + e.x;
                 const float xt = xb + L.slope;
                 const float m = __builtin_amdgcn_fmed3f(xt - xmin, xmin1 - xb, 0.0f);
                 const float f = fminf(fmaxf(m * fast_rcp(xt - xb), 0.0f), 1.0f);
-                acc[q][0] = fmaf(f, ev[k].y, acc[q][0]);
+                acc[q][0] = fmaf(f, e.y, acc[q][0]);
               }
             } else {
-#pragma unroll
-              for (int k = 0; k < KC; ++k) {
-                if (NC == 0 && k >= ncand) break;
-                const float xb = xbase + ev[k].x;
+              for (int k = 0; k < ncand; ++k) {
+                const float2 e = wrow[k];
+                const float xb = xbase + e.x;
                 const float xt = xb + L.slope;
                 const float m = __builtin_amdgcn_fmed3f(xb - xmin, xmin1 - xt, 0.0f);
                 const float f = fminf(fmaxf(m * fast_rcp(xb - xt), 0.0f), 1.0f);
-                acc[q][0] = fmaf(f, ev[k].y, acc[q][0]);
+                acc[q][0] = fmaf(f, e.y, acc[q][0]);
               }
             }
           } else if (FASTREF) {
             // degenerate line: general form with the m == 0 case, lbase already in e.y
-#pragma unroll
-            for (int k = 0; k < KC; ++k) {
-              if (NC == 0 && k >= ncand) break;
-              const float l =
-                  cand_len<false, WEIGHTS>(xbase + ev[k].x, L.slope, 1.0f, xmin, xmin1, true);
-              acc[q][0] = fmaf(l, ev[k].y, acc[q][0]);
+            for (int k = 0; k < ncand; ++k) {
+              const float2 e = wrow[k];
+              const float l = cand_len<false, WEIGHTS>(xbase + e.x, L.slope, 1.0f, xmin, xmin1, true);
+              acc[q][0] = fmaf(l, e.y, acc[q][0]);
             }
           } else {
             // reference order: the line's candidates summed, then added to the pixel
