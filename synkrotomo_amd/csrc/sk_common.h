@@ -43,11 +43,16 @@ struct Geom {
   // Unit bins with two candidates per pixel and |rho0| + N < 2^20: the exact backprojector's
   // specialised loop applies.
   bool bp_two_cand = false;
-  // The fast candidate index is off by less than 0.4 bin (|rho0| + N < 2^20 bins), so it drops no
-  // ray with a nonzero length: the fast A^T and B^T apply.
+  // The fast A^T and B^T apply (|rho0| <= 4 N).  They do not take the reference's candidate index: A^T a
+  // faster one, B^T (A.x) none, and where the reference's rounds across a pixel's outermost ray
+  // they count another ray, or one more.  Each index is within 2 ulp of |rho0| + N of its value, so
+  // such a ray is shorter than 8 of these ulps: at 4 N, 3e-6 N pixels, three times that of a centred
+  // detector.  Near 45 degrees at |rho0| = 1e6 it is a tenth of a pixel (64^2, bins of 2: A^T 9e-4
+  // off in the 2-norm).
   bool index_safe = false;
-  // Candidates per pixel (1..4) of the hoisted fast backprojector, whose fast index needs no clamp;
-  // 0 where it does not apply (index not safe, or bins narrower than 0.354: the general path).
+  // Candidates per pixel (1..4) of the hoisted fast backprojector, whose fast index needs no clamp
+  // (it is off by less than 0.4 bin: |rho0| + N < 2^20 bins); 0 where it does not apply (farther, or
+  // bins narrower than 0.354: the general path, by the same index with a clamp).
   int bp_nc = 0;
   // Row-segment width (floats) the staged forward projector needs for 256 consecutive bins.
   int fps_w = 0;

@@ -336,8 +336,8 @@ int sk_geom_create(sk_ctx* ctx, const float* angles_host, int A, float rho0, flo
   Geom& G = g->g;
   G.A = A; G.R = R; G.N = N; G.rho0 = rho0; G.drho = drho; G.ncand = ncand;
   G.bp_two_cand = drho == 1.0f && ncand == 2 && std::fabs((double)rho0) + N < (double)(1 << 20);
-  G.index_safe = std::fabs((double)rho0) + N < (double)(1 << 20) * drho;
-  G.bp_nc = G.index_safe && ncand <= 4 ? ncand : 0;
+  G.index_safe = std::fabs((double)rho0) <= 4.0 * N;
+  G.bp_nc = ncand <= 4 && std::fabs((double)rho0) + N < (double)(1 << 20) * drho ? ncand : 0;
   G.device = c->device;
   G.n_steep = build_lines(angles_host, A, G.lines, N);
   {

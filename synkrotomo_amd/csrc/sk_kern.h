@@ -513,7 +513,8 @@ __device__ __forceinline__ float binade_step(float slope, int e) {
 // order.  Fast mode keeps the reference's xbot/xtop (so each length fraction is the
 // reference's up to the reciprocal) but computes the candidate index with fewer roundings:
 // a pixel whose rounded index moves by one bin gains or loses only a bin at distance
-// >= sqrt(2)/2 from its centre, where the intersection length is zero.
+// >= sqrt(2)/2 from its centre (to the index's rounding, a few ulp of |rho0| + N), where the
+// intersection length is zero.
 //
 // S > 1 (the hoisted fast path): images bz*S .. bz*S + S-1 at once (an image past the last one
 // repeats it and is not written).  A candidate's index, LDS position and length do not depend on

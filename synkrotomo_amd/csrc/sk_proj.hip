@@ -459,10 +459,12 @@ int launch_fp(Ctx* c, const Geom* g, FpMode mode, const FpArgs& a, hipStream_t s
 // launch over their table indices.  8 images of 512^2, 360 angles: 1249 us with every line on that
 // walk (60 VALU a row and two dependent global gathers), 199 us like this.
 int launch_fp_bpt(Ctx* c, const Geom* g, const FpArgs& a, hipStream_t s) {
-  const bool ex = c->exact != 0 || !g->index_safe;
   const bool dr1 = g->drho == 1.0f;
-  if (ex) {
-    dr1 ? fp_go<true, FP_PLAIN, W_ADJ, true, 1>(g, a, s) : fp_go<true, FP_PLAIN, W_ADJ, false, 1>(g, a, s);
+  if (c->exact || !g->index_safe) {
+    if (c->exact)
+      dr1 ? fp_go<true, FP_PLAIN, W_ADJ, true, 1>(g, a, s) : fp_go<true, FP_PLAIN, W_ADJ, false, 1>(g, a, s);
+    else
+      dr1 ? fp_go<false, FP_PLAIN, W_ADJ, true, 1>(g, a, s) : fp_go<false, FP_PLAIN, W_ADJ, false, 1>(g, a, s);
     return launched(c, "backprojection-transpose kernel");
   }
   int rc = launch_fp(c, g, FP_PLAIN, a, s);

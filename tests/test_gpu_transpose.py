@@ -2,9 +2,11 @@
 oracle's matrix in FP64."""
 import numpy as np
 import pytest
+import scipy.sparse as sp
 import torch
 
 import oracle
+from conftest import rel_l2
 
 pytestmark = pytest.mark.gpu
 
@@ -67,3 +69,24 @@ def test_transpose_of_pixels_that_are_not_finite(ctx, N, A, R, dr, batch, varian
         ref = np.bincount(c[keep], weights=w * x, minlength=A * R)
         mag = np.bincount(c[keep], weights=w * np.abs(x), minlength=A * R)
         assert np.all(np.abs(got[k] - ref)[~bad] <= (4.8e-7 + 1.5 * N * 6e-8) * mag[~bad])
+
+
+# Pixels at whose outermost ray the candidate index rounds: on lines that are not degenerate A^T and B
+# have the same lengths, and both follow the reference's index, so A^T r is the oracle's B r and B^T v
+# its B^T v, at the largest |rhozero| as well as where the fast paths end (4 N) and just past them.
+# Tolerance as in test_gpu_adjoints.py.
+@pytest.mark.parametrize("N,rz,dr", [(64, -999000.3, 1.0), (64, -943000.7, 0.9), (32, -524000.2, 0.5), (64, -999900.3, 2.0),
+                                     (64, -255.9, 1.0), (64, -256.1, 1.0), (64, -255.9, 0.25)])
+def test_transpose_and_adjoint_with_the_references_candidates(ctx, N, rz, dr):
+    ang = (np.pi / 4 + np.array([-0.05, -0.011, -0.003, 0.0007, 0.004, 0.02])).astype(np.float32)
+    A, R = ang.size, int((-rz + N) / dr)
+    rng = np.random.default_rng(3)
+    y = rng.standard_normal((A, R)).astype(np.float32)
+    v = rng.standard_normal((N, N)).astype(np.float32)
+    geo = ctx.geometry(ang, rz, dr, R, N)
+    aty = geo.bp_adjoint(torch.from_numpy(y).cuda()).cpu().numpy().ravel()
+    btv = geo.bp_transpose(torch.from_numpy(v).cuda()).cpu().numpy().ravel()
+    rp, c, vals = oracle.bp_csr(ang, rz, dr, R, N)
+    B = sp.csr_matrix((vals.astype(np.float64), c, rp), shape=(N * N, A * R))
+    assert rel_l2(aty, B @ y.ravel().astype(np.float64)) <= 2e-6
+    assert rel_l2(btv, B.T @ v.ravel().astype(np.float64)) <= 2e-6
