@@ -457,10 +457,17 @@ int launch_fp(Ctx* c, const Geom* g, FpMode mode, const FpArgs& a, hipStream_t s
 // short rays at the image's corners and those that are not finite (k_bpt_rays).  The degenerate lines (theta ~ 0, pi/2: a ray on
 // a pixel edge counts in A and not in B) are walked again with the backprojector's own lengths, one
 // launch over their table indices.  8 images of 512^2, 360 angles: 1249 us with every line on that
-// walk (60 VALU a row and two dependent global gathers), 199 us like this.
+// walk (60 VALU a row and two dependent global gathers), 199 us like this.  Small images take few
+// rows, and one launch of that walk is as fast as two or three (us, walk and this: with degenerate
+// lines 16^2 and 22 angles 8.2, 11.2; 24^2 and 33 angles 11.3, 12.5; 32^2 and 44 angles 14.8, 13.5;
+// without them 8.2, 8.9; 11.3, 9.9) until a batch fills the chip (16^2, 256 images: 23.7, 17.4).
+static bool bpt_walks(const Geom* g, int batch) {
+  return !g->index_safe || (g->N < (g->n_degen ? 32 : 24) && fp_workgroups(g, batch) <= 768);
+}
+
 int launch_fp_bpt(Ctx* c, const Geom* g, const FpArgs& a, hipStream_t s) {
   const bool dr1 = g->drho == 1.0f;
-  if (c->exact || !g->index_safe) {
+  if (c->exact || bpt_walks(g, a.batch)) {
     if (c->exact)
       dr1 ? fp_go<true, FP_PLAIN, W_ADJ, true, 1>(g, a, s) : fp_go<true, FP_PLAIN, W_ADJ, false, 1>(g, a, s);
     else

@@ -90,3 +90,20 @@ def test_transpose_and_adjoint_with_the_references_candidates(ctx, N, rz, dr):
     B = sp.csr_matrix((vals.astype(np.float64), c, rp), shape=(N * N, A * R))
     assert rel_l2(aty, B @ y.ravel().astype(np.float64)) <= 2e-6
     assert rel_l2(btv, B.T @ v.ravel().astype(np.float64)) <= 2e-6
+
+
+# Small images walk every line with the backprojector's lengths until a batch fills the chip; both ways
+# on each side of the line, with degenerate lines and without.  Tolerance as in test_gpu_adjoints.py.
+@pytest.mark.parametrize("N,A,first,batch", [(22, 16, 0.013, 1), (24, 16, 0.013, 1), (30, 21, 0.0, 1), (32, 21, 0.0, 1),
+                                             (16, 22, 0.0, 128), (16, 22, 0.0, 129)])
+def test_transpose_of_small_images(ctx, N, A, first, batch):
+    ang = (np.arange(A) * np.pi / A + first).astype(np.float32)
+    R = int(np.ceil(np.sqrt(2.0) * N)) + 1
+    rz = -(R - 1) / 2 + 0.2
+    v = np.random.default_rng(N).standard_normal((batch, N, N)).astype(np.float32)
+    geo = ctx.geometry(ang, rz, 1.0, R, N)
+    got = geo.bp_transpose(torch.from_numpy(v).cuda()).cpu().numpy()
+    rp, c, vals = oracle.bp_csr(ang, rz, 1.0, R, N)
+    B = sp.csr_matrix((vals.astype(np.float64), c, rp), shape=(N * N, A * R))
+    for k in {0, batch // 2, batch - 1}:
+        assert rel_l2(got[k].ravel(), B.T @ v[k].ravel().astype(np.float64)) <= 2e-6
