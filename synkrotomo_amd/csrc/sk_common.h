@@ -142,7 +142,7 @@ enum BpWeights { W_REF = 0, W_ADJ = 1 };
 
 struct FpArgs {
   const float* img;    // [batch][N][N]  (unused in FP_ONES_INV)
-  const float* imgT;   // [batch][N][N] transposed copy (flat lines)
+  const float* imgT;   // [batch][N][N] transposed copy (flat lines); img where the call needs none (fp_in_lds)
   float* out;          // [batch][A][R]
   const float* b;      // FP_SIRT: measured sinogram [batch][A][R]
   const float* rowinv; // FP_SIRT: [A][R]
@@ -160,6 +160,7 @@ int launched(Ctx* c, const char* what);
 int launch_transpose(Ctx* c, const float* in, float* out, int N, int batch, hipStream_t s);
 int fp_rays_per_lane(int variant);
 int bp_pixels_per_lane(int variant);
+bool fp_in_lds(const Ctx* c, const Geom* g, int batch);
 int launch_fp(Ctx* c, const Geom* g, FpMode mode, const FpArgs& a, hipStream_t s);
 int launch_fp_bpt(Ctx* c, const Geom* g, const FpArgs& a, hipStream_t s);
 int launch_bp(Ctx* c, const Geom* g, BpMode mode, BpWeights w, const BpArgs& a, hipStream_t s);

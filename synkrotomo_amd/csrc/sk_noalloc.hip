@@ -4,9 +4,9 @@
 // context's growable scratch, which is (re)allocated with hipMalloc on first use and whenever
 // a larger batch arrives.  Callers that may not allocate (code under hipGraph capture, tight
 // serving loops, harnesses that forbid hipMalloc) use sk_fp_noalloc instead: the same kernels,
-// with the transposed copy in `scratch`, a fixed device array that lives as long as the
-// process.  Its device address is looked up once per device (sk_create, with the device
-// current) and passed to the kernels; the array's name is never used as a device address.
+// with the transposed copy (where they need one) in `scratch`, a fixed device array that lives
+// as long as the process.  Its device address is looked up once per device (sk_create, with the
+// device current) and passed to the kernels; the array's name is never used as a device address.
 //
 // One array per GPU, shared by every call on it: calls that overlap on one GPU (two streams,
 // two host threads) race on it.  Each call overwrites the part it uses before reading it, so
@@ -70,7 +70,7 @@ int sk_fp_noalloc(sk_ctx* ctx, sk_geom* g, int batch, const float* d_img, float*
   SK_HIP(c, hipSetDevice(c->device));
   hipStream_t s = (hipStream_t)stream;
   const float* imgT = d_img;
-  if (G.n_steep < G.A) {
+  if (G.n_steep < G.A && !sk::fp_in_lds(c, &G, batch)) {
     int rc = sk::launch_transpose(c, d_img, ws, G.N, batch, s);
     if (rc) return rc;
     imgT = ws;

@@ -189,11 +189,12 @@ __device__ __forceinline__ float fpl_rows(const float* cells, int N, int h, int 
 
 // One image of a small geometry: a wave per 64 bins of a line, four to a workgroup, all bins of all
 // lines in turn; grid (workgroups, images).  The walk (row range, fractions, order of the sums) is
-// fp_item's, with the two pixels of a row from LDS: no transposed copy and no load latency per row.
-// What is left is launch, the copy and a serial walk of N rows at one wave per SIMD: 64^2 and 90
+// fp_item's, with the two pixels of a row from LDS: no load latency per row, and no transposed copy --
+// where one is at hand anyway (SIRT's update writes it; B^T reads it) the per-wave kernel needs
+// 2 us less (a SIRT iteration of 32^2, 22 angles 12.0 us against 13.5, of 64^2, 89 angles 23.9
+// against 25.7).  What is left is launch, the copy and a serial walk of N rows at one wave per SIMD: 64^2 and 90
 // angles, calls back to back, 7.9 us against 9.0 for the transposed copy and the per-wave kernel
 // (6.7 at 16^2, where only the launch is left).
-template <int MODE>
 __global__ __launch_bounds__(256) void k_fp_lds(FpParams P) {
   extern __shared__ float lds[];
   const int N = P.N, Q = fpl_pitch(N), h = N >> 1, origin = fpl_origin(N), end = origin + N * Q;
@@ -240,12 +241,7 @@ __global__ __launch_bounds__(256) void k_fp_lds(FpParams P) {
     s = nt ? fpl_rows<false, true>(cells, N, h, i0, i1, cs, rs, L.slope, icpt, rslope)
            : fpl_rows<false, false>(cells, N, h, i0, i1, cs, rs, L.slope, icpt, 0.0f);
   if (r >= P.R) return;
-  s = s * L.lbase;
-  const size_t o = (size_t)blockIdx.y * P.A * P.R + (size_t)L.orig * P.R + r;
-  if constexpr (MODE == FP_PLAIN)
-    P.out[o] = s;
-  else  // SIRT.fut:33-36: R * (b - A x)
-    P.out[o] = P.rowinv[(size_t)L.orig * P.R + r] * (P.b[o] - s);
+  P.out[(size_t)blockIdx.y * P.A * P.R + (size_t)L.orig * P.R + r] = s * L.lbase;
 }
 
 // ------------------------------------------------------------- staged A.x (fast mode)
@@ -399,24 +395,22 @@ static int fp_variant_default(const Geom* g, int batch) {
   return g->N < 128 && fp_workgroups(g, batch) < 512 ? 3 : 7;
 }
 
-// Whether a call takes k_fp_lds, the same way as the rule above: the image is small enough to be
-// copied by every workgroup (us with it and with the better of the other two and their transposed
-// copy: 64^2 and 90 angles 7.9, 9.0; 80^2 and 126 9.4, 10.2; 96^2 and 150 12.0, 11.1; 120^2 and 190
-// 13.4, 13.0), and no more than the three workgroups per CU or so that hide it (64^2 and 90 angles: 4
-// images 8.0, 9.4; 16 images, 720 workgroups, 10.9, 13.8; with half bins, 1440 workgroups, 15.4, 12.8).
-static bool fp_in_lds(const Ctx* c, const Geom* g, int batch) {
-  return !c->exact && g->fp_variant < 0 && !c->fp_variant && g->N <= FPL_MAX_N && fp_workgroups(g, batch) <= 768;
+// Whether A.x with no transposed copy at hand (FpArgs: imgT = img) takes k_fp_lds, and needs none, the
+// same way as the rule above: the image is small enough to be copied by every workgroup (us with it and
+// with the better of the other two and their transposed copy: 64^2 and 90 angles 7.9, 9.0; 80^2 and 126
+// 9.4, 10.2; 96^2 and 150 12.0, 11.1; 120^2 and 190 13.4, 13.0), and no more than the three workgroups
+// per CU or so that hide it (64^2 and 90 angles: 4 images 8.0, 9.4; 16 images, 720 workgroups, 10.9,
+// 13.8; with half bins, 1440 workgroups, 15.4, 12.8).  Without flat lines there is no copy to save.
+bool fp_in_lds(const Ctx* c, const Geom* g, int batch) {
+  return !c->exact && g->fp_variant < 0 && !c->fp_variant && g->N <= FPL_MAX_N && g->n_steep < g->A &&
+         fp_workgroups(g, batch) <= 768;
 }
 
 int launch_fp(Ctx* c, const Geom* g, FpMode mode, const FpArgs& a, hipStream_t s) {
   const bool ex = c->exact != 0;
-  if (mode != FP_ONES_INV && fp_in_lds(c, g, a.batch)) {
+  if (mode == FP_PLAIN && a.imgT == a.img && fp_in_lds(c, g, a.batch)) {
     const dim3 grid((unsigned)fp_workgroups(g, 1), a.batch);
-    const size_t lds = sizeof(float) * fpl_cells(g->N);
-    if (mode == FP_PLAIN)
-      hipLaunchKernelGGL((k_fp_lds<FP_PLAIN>), grid, dim3(256), lds, s, fp_params(g, a));
-    else
-      hipLaunchKernelGGL((k_fp_lds<FP_SIRT>), grid, dim3(256), lds, s, fp_params(g, a));
+    hipLaunchKernelGGL(k_fp_lds, grid, dim3(256), sizeof(float) * fpl_cells(g->N), s, fp_params(g, a));
     return launched(c, "forward projection kernel");
   }
   int v = g->fp_variant >= 0 ? g->fp_variant : (c->fp_variant ? c->fp_variant : fp_variant_default(g, a.batch));
