@@ -382,17 +382,31 @@ static long fp_workgroups(const Geom* g, int batch) {
   return ((long)g->A * ((g->R + 63) / 64) + FP_WAVES - 1) / FP_WAVES * batch;
 }
 
-// The kernel of a geometry that was not tuned, on a context whose option is 0: the grouped one (and
-// below it what a geometry without line groups, or exact mode, falls back to).  From 128^2 to
-// 2048^2, angle counts 0.35 N to 1.6 N and bins of 0.5 to 2 it is the fastest or within 0.3 us of
-// the fastest (one ray per lane, the default before, us against grouped: 128^2 and 89 angles 13.5,
-// 13.2; 256^2 and 179 30.6, 21.1; 512^2 and 358 91, 59; 2048^2 and 1433 3662, 1750).  Smaller
-// images take a few rows only and the short per-wave kernel is as fast (64^2, 100 angles: 9.0,
-// 9.5), with a tenth of the code to fetch on a first call, until a batch fills the chip: per-wave and
-// grouped, 96^2 and 150 angles 11.6, 11.1 (1 image), 32, 20 (16), 99, 40 (64); 64^2 and 90 angles 9.0,
-// 9.2; 16, 14; 43, 19.
+// The kernel of a geometry that was not tuned, on a context whose option is 0: the grouped one (7, and
+// below it what a geometry without line groups, or exact mode, falls back to), where it is not
+// slower than one ray per lane (0 bins fastest, 3 lines fastest).  us for 0, 3 and 7, one image
+// unless said, R = sqrt(2) N / drho:
+// - 256^2 and 179 angles 29.5, 22.7, 20.9; 512^2 and 358 90, 94, 60; 2048^2 and 1433 3662, -, 1750.
+// - Below 128^2 a ray takes a few rows only and the per-wave kernel is as fast (64^2, 100 angles: 9.0 and
+//   9.5 for 3 and 7), with a tenth of the code to fetch on a first call, until a batch fills the chip
+//   (3 and 7: 96^2 and 150 angles 11.6, 11.1; 16 images 32, 20; 64 images 99, 40).
+// - Bins below 1: neighbouring lanes share pixels and the per-wave gathers cost less.  One image per
+//   workgroup and one round of workgroups: bins of 0.75, 362^2 and 506 angles 50, 47.5, 62.4; 724^2 and 253
+//   90, 91, 119; of 0.5, 512^2 and 716 145, 133, 140; past 4096 workgroups 1024^2 and 1433 938, 894, 822.
+//   Several images share the staging again (256^2 and 179, bins of 0.5, 4 images: 7 at 0.71 of 0).
+// - A detector that ends several image widths from the axis: bins that see nothing, whose workgroups cost
+//   the most where lines run fastest (256^2 and 256 angles, bins of 1, R = 14481: 48, 70, 83; 512^2 and
+//   512, bins of 2, R = 14481, 4 images: 415, 1063, 1061), and line groups that spread more the farther
+//   off their bins lie, so with narrow bins from little more than the image's diagonal on (512^2 and 179,
+//   bins of 0.5, R = 5792, four times what is seen: 76, 64, 119; 256^2 and 128, bins of 1, the axis 2000 from
+//   the first one: 27, -, 41).
 static int fp_variant_default(const Geom* g, int batch) {
-  return g->N < 128 && fp_workgroups(g, batch) < 512 ? 3 : 7;
+  // the farthest bin from the axis, in image widths (0.71 sees the whole image)
+  const double reach = fmax(fabs((double)g->rho0), fabs(g->rho0 + (double)g->R * g->drho)) / g->N;
+  const bool narrow = g->drho < 1.0f && fpg_images(g, batch) == 1;
+  if (reach > (narrow ? 0.9 : 6.0)) return 0;
+  if (g->N < 128 && fp_workgroups(g, batch) < 512) return 3;
+  return narrow && fp_workgroups(g, batch) < 4096 ? 3 : 7;
 }
 
 // Whether A.x with no transposed copy at hand (FpArgs: imgT = img) takes k_fp_lds, and needs none, the
