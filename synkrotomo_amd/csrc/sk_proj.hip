@@ -69,8 +69,8 @@ __global__ __launch_bounds__(FP_BLOCK) void k_fp(FpParams P) {
 // B^T of the listed (degenerate) lines: every row of 64 bins with the backprojector's lengths.  Few
 // rays and two gathers a row, so latency bounds it: LISTED_WAVES waves of a workgroup take a run of
 // the rows each, four rows' loads in flight, and their sums are added in order.  B^T of 8 images of
-// 512^2, 360 angles, two of them such lines: 355 us with one wave walking all rows, 199 us like this
-// (A.x: 199).  Grid (bins / 64, listed lines, images).
+// 512^2, 360 angles, two of them such lines: 355 us with one wave walking all rows, 201 us like this
+// (A.x: 185).  Grid (bins / 64, listed lines, images).
 constexpr int LISTED_WAVES = 16;
 template <bool DR1>
 __global__ __launch_bounds__(64 * LISTED_WAVES) void k_fp_listed(FpParams P, const int* __restrict__ list) {
@@ -120,14 +120,16 @@ __global__ __launch_bounds__(64 * LISTED_WAVES) void k_fp_listed(FpParams P, con
 // line that is not degenerate, the row sums in order.  A.x forms a row as vb + f*(vo - vb):
 // - A ray that leaves most of a row's length outside gets its short part from 1 - f, 6e-8 off however
 //   short, and divided by a row sum of 1e-3 (the gradient of a SIRT step) that is 6e-5 of the
-//   result: rays that cross less than two pixels' length.  The outermost corners of a line are at
-//   (frame) x = -+h, y = -+h by the signs of cost and sint; a chord at distance d from one is
-//   d/|cost*sint| long.  d only picks the rays (FP32: on a nearly axis-parallel line its error can
-//   exceed the whole range of short chords); the rows come from the ray's own intercept, and a ray
-//   that crosses more of them than a short chord can is left as it is, A.x being right for it.
+//   result: rays that cross less than two pixels' length.  The outermost corners of a line lie at
+//   distance h*(|cost| + |sint|) from the axis, and a chord d nearer than that is d/|cost*sint|
+//   long.  d only picks the rays (FP32: on a nearly axis-parallel line its error can exceed the
+//   whole range of short chords); the rows come from the ray's own intercept, and a ray that
+//   crosses more of them than a short chord can is left as it is, A.x being right for it.
 // - A pixel that is not finite, or two whose difference overflows, reach every ray that passes beside
 //   them (0*inf), and A.x is then not finite, whatever follows: those rays are walked again.
-// Two divisions, a load and a store's mask per ray: 8 images of 512^2, 360 angles: 6 us of 199.
+// Nearly every ray costs its load and a handful of VALU, the few walked ones the latency of their
+// loads, four rows in flight.  8 images of 512^2, 360 angles: 8 us of 201.  Grid (bins / 256,
+// lines, images).
 constexpr int RIM_ROWS = 32;  // a short chord: 3 rows, one more at each end, and 2e-6*h/|slope| <= 17 for rounding
 template <bool DR1>
 __global__ __launch_bounds__(256) void k_bpt_rays(FpParams P) {
@@ -137,24 +139,36 @@ __global__ __launch_bounds__(256) void k_bpt_rays(FpParams P) {
   const int N = P.N, h = N >> 1;
   float* out = P.out + (size_t)blockIdx.z * P.A * P.R + (size_t)L.orig * P.R + r;
   const bool finite = (__builtin_bit_cast(unsigned, *out) & 0x7f800000u) != 0x7f800000u;
-  const float reach = (float)h * (fabsf(L.cost) + fabsf(L.sint));
-  const float low = (-reach - P.rho0) / P.drho, high = (reach - P.rho0) / P.drho;  // bins of the corners
-  const float d = fminf((float)r - low, high - (float)r) * P.drho;
+  const float rho = P.rho0 + (float)r * P.drho;
+  const float d = (float)h * (fabsf(L.cost) + fabsf(L.sint)) - fabsf(rho);
   if (finite && d > 2.0f * fabsf(L.cost * L.sint)) return;
-  const float icpt = (P.rho0 + (float)r * P.drho) / L.cost;  // forwardprojection.fut:33-34
+  const float icpt = rho / L.cost;  // forwardprojection.fut:33-34
   int i0, i1;
   row_span(L.slope, icpt, h, i0, i1);
   if (finite && (i0 >= i1 || i1 - i0 > RIM_ROWS)) return;
   const float* src = ((L.flags & LINE_FLAT) ? P.imgT : P.img) + (size_t)blockIdx.z * N * N;
   float sum = 0.0f;
-  for (int i = i0; i < i1; ++i) {
-    const float xbot = (float)i * L.slope + icpt, xtop = xbot + L.slope;
-    const int Xb = (int)floorf(xbot), Xt = (int)floorf(xtop);
-    auto part = [&](int X) {
-      const float len = bp_entry<false, DR1>(L, X, (float)i, xbot, xtop, r, P.ncand, P.rho0, P.drho);
-      return (unsigned)(X + h) < (unsigned)N ? len * src[(size_t)(i + h) * N + X + h] : 0.0f;
-    };
-    sum = sum + (part(Xb) + (Xb == Xt ? 0.0f : part(Xt)));
+  for (int i = i0; i < i1; i += 4) {
+    float xbot[4], vb[4], vt[4];
+    int Xb[4], Xt[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      xbot[q] = (float)(i + q) * L.slope + icpt;
+      Xb[q] = (int)floorf(xbot[q]);
+      Xt[q] = (int)floorf(xbot[q] + L.slope);
+      const float* row = src + (size_t)(i + q + h) * N + h;
+      vb[q] = i + q < i1 && (unsigned)(Xb[q] + h) < (unsigned)N ? row[Xb[q]] : 0.0f;
+      vt[q] = i + q < i1 && (unsigned)(Xt[q] + h) < (unsigned)N ? row[Xt[q]] : 0.0f;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if (i + q >= i1) break;
+      auto part = [&](int X, float v) {
+        const float len = bp_entry<false, DR1>(L, X, (float)(i + q), xbot[q], xbot[q] + L.slope, r, P.ncand, P.rho0, P.drho);
+        return (unsigned)(X + h) < (unsigned)N ? len * v : 0.0f;
+      };
+      sum = sum + (part(Xb[q], vb[q]) + (Xb[q] == Xt[q] ? 0.0f : part(Xt[q], vt[q])));
+    }
   }
   *out = sum;
 }
@@ -465,7 +479,7 @@ int launch_fp(Ctx* c, const Geom* g, FpMode mode, const FpArgs& a, hipStream_t s
 // short rays at the image's corners and those that are not finite (k_bpt_rays).  The degenerate lines (theta ~ 0, pi/2: a ray on
 // a pixel edge counts in A and not in B) are walked again with the backprojector's own lengths, one
 // launch over their table indices.  8 images of 512^2, 360 angles: 1249 us with every line on that
-// walk (60 VALU a row and two dependent global gathers), 199 us like this.  Small images take few
+// walk (60 VALU a row and two dependent global gathers), 201 us like this.  Small images take few
 // rows, and one launch of that walk is as fast as two or three (us, walk and this: with degenerate
 // lines 16^2 and 22 angles 8.2, 11.2; 24^2 and 33 angles 11.3, 12.5; 32^2 and 44 angles 14.8, 13.5;
 // without them 8.2, 8.9; 11.3, 9.9) until a batch fills the chip (16^2, 256 images: 23.7, 17.4).
