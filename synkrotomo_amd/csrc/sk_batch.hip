@@ -162,7 +162,11 @@ __global__ __launch_bounds__(FPS_RAYS, S == 1 ? 8 : (CPLMAX == 2 ? 5 : 4)) void 
   }
 }
 
-// Tiles of S images (S > 1: 16 x 32 tiles, the hoisted fast path).
+// Tiles of S images (S > 1: 16 x 32 tiles, the hoisted fast path).  NC = NC_ANY: the hoisted path with
+// each problem's own 1 to 4 candidates (a fourth candidate of a pixel that has fewer is 0 long, and
+// 0 times a value that is not finite reaches pixels its ray does not).
+constexpr int NC_ANY = -1;
+
 template <bool EXACT, int NC, bool DR1, int PPT, int S>
 __global__ __launch_bounds__(256) void k_bp_persist(const BatchArgs a, unsigned* __restrict__ ctr) {
   extern __shared__ float4 win[];
@@ -187,7 +191,20 @@ __global__ __launch_bounds__(256) void k_bp_persist(const BatchArgs a, unsigned*
       tx = (int)(t & 0xffffu);
       ty = (int)(t >> 16);
     }
-    bp_item<EXACT, BP_SIRT, W_REF, NC, DR1, PPT, S>(B.bp, u32(tx), u32(ty), u32(bz), (float2*)win, lsh);
+    auto run = [&](auto nc) {
+      bp_item<EXACT, BP_SIRT, W_REF, decltype(nc)::value, DR1, PPT, S>(B.bp, u32(tx), u32(ty), u32(bz), (float2*)win,
+                                                                       lsh);
+    };
+    if constexpr (NC == NC_ANY) {
+      switch (u32(B.bp.ncand)) {
+        case 1: run(std::integral_constant<int, 1>{}); break;
+        case 2: run(std::integral_constant<int, 2>{}); break;
+        case 3: run(std::integral_constant<int, 3>{}); break;
+        default: run(std::integral_constant<int, 4>{});
+      }
+    } else {
+      run(std::integral_constant<int, NC>{});
+    }
   }
 }
 
@@ -207,7 +224,7 @@ struct BatchPlan {
   unsigned* d_ctr = nullptr;
   int Wmax = 0;
   bool dr1 = true;
-  int nc = 0;         // candidates per pixel of the hoisted backprojector, 0: the general path
+  int nc = 0;         // hoisted backprojector: 2 candidates per pixel in every group, or NC_ANY; 0: the general path
   const void *kfp = nullptr, *kbp = nullptr;
   size_t fp_lds = 0, bp_lds = 0;
 };
@@ -252,7 +269,7 @@ static const void* bp_kernel(const BatchPlan& p, bool ex) {
   if (ex)
     return p.bp_ppt == 4 ? (const void*)k_bp_persist<true, 0, false, 4, 1> : (const void*)k_bp_persist<true, 0, false, 2, 1>;
   if (p.nc == 2) return bp_kernel_nc<2>(p);
-  if (p.nc > 0) return bp_kernel_nc<4>(p);
+  if (p.nc == NC_ANY) return bp_kernel_nc<NC_ANY>(p);
   return p.bp_ppt == 4 ? (const void*)k_bp_persist<false, 0, false, 4, 1> : (const void*)k_bp_persist<false, 0, false, 2, 1>;
 }
 
@@ -366,7 +383,7 @@ int sk_sirt_batched(sk_ctx* ctx, const sk_problem* problems, int count, int iter
     if (!G.bp_nc || !plan.nc)
       plan.nc = 0;
     else if (G.bp_nc != 2)
-      plan.nc = 4;  // serves 1 to 4: a further candidate's length is 0
+      plan.nc = NC_ANY;
   }
   if (!ex && plan.fp_mode == 5) {
     const int sizes[3] = {1, 2, 4};
@@ -404,7 +421,6 @@ int sk_sirt_batched(sk_ctx* ctx, const sk_problem* problems, int count, int iter
     B.bp_ty = (G.N + 16 * ppt - 1) / (16 * ppt);
     B.fp_begin = args.fp_total;
     B.bp_begin = args.bp_total;
-    if (!ex && plan.nc) B.bp.W = bp_window_bins(ppt, G.drho, plan.nc);
     args.fp_total += (long)((P.batch + plan.fp_images - 1) / plan.fp_images) * B.fp_units * B.fp_wb;
     args.bp_total += (long)((P.batch + plan.bp_images - 1) / plan.bp_images) * B.bp_tx * B.bp_ty;
     plan.Wmax = std::max(plan.Wmax, B.bp.W);

@@ -1,0 +1,34 @@
+"""sirt_batched with several images per work item, bit for bit against each slice alone."""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _group(ctx, N, A, drho, batch, gen):
+    R = math.ceil(math.sqrt(2) * N / drho)
+    geo = ctx.geometry((np.arange(A) * math.pi / A).astype(np.float32), -(R - 1) / 2 * drho + 0.3, drho, R, N)
+    return geo, torch.zeros(batch, N, N, device="cuda"), torch.rand(batch, A, R, device="cuda", generator=gen)
+
+
+# A measurement that is not finite reaches the pixels its ray is a candidate of, and no others: a group
+# whose pixels have fewer candidates than another group's takes only its own.
+@pytest.mark.parametrize("batch", [1, 12])
+def test_values_that_are_not_finite_stay_with_their_candidates(ctx, batch):
+    from synkrotomo_amd.projector import sirt_batched
+    gen = torch.Generator(device="cuda").manual_seed(2)
+    groups = [_group(ctx, *s, batch, gen) for s in ((256, 29, 0.4), (230, 31, 2.0), (200, 23, 0.5), (96, 17, 1.0))]
+    for geo, x, sino in groups:
+        sino[0, 3, geo.R // 2] = math.inf
+        sino[-1, 5, geo.R // 3] = math.nan
+    sirt_batched(groups, 1)
+    for geo, x, sino in groups:
+        for i in {0, batch - 1}:
+            one = torch.zeros(geo.N, geo.N, device="cuda")
+            geo.sirt_(one, sino[i].contiguous(), 1)
+            same = (x[i] == one) | (x[i].isnan() & one.isnan())
+            assert bool(same.all()), (geo.N, i, int((~same).sum()))
+            assert 0 < int((~x[i].isfinite()).sum()) < geo.N * geo.N // 4
