@@ -195,7 +195,9 @@ __global__ __launch_bounds__(256) void k_bp_persist(const BatchArgs a, unsigned*
       bp_item<EXACT, BP_SIRT, W_REF, decltype(nc)::value, DR1, PPT, S>(B.bp, u32(tx), u32(ty), u32(bz), (float2*)win,
                                                                        lsh);
     };
-    if constexpr (NC == NC_ANY) {
+    if constexpr (NC == NC_ANY && S == 8) {  // sets with 3 or 4 candidates stop at 4 images
+      B.bp.ncand == 1 ? run(std::integral_constant<int, 1>{}) : run(std::integral_constant<int, 2>{});
+    } else if constexpr (NC == NC_ANY) {
       switch (u32(B.bp.ncand)) {
         case 1: run(std::integral_constant<int, 1>{}); break;
         case 2: run(std::integral_constant<int, 2>{}); break;
@@ -377,8 +379,10 @@ int sk_sirt_batched(sk_ctx* ctx, const sk_problem* problems, int count, int iter
       plan.fp_mode = want & 3;
   }
   plan.nc = 2;
+  int max_cand = 0;
   for (int i = 0; i < count; i++) {
     const Geom& G = problems[i].geom->g;
+    max_cand = std::max(max_cand, G.ncand);
     plan.dr1 = plan.dr1 && G.bp_two_cand;
     if (!G.bp_nc || !plan.nc)
       plan.nc = 0;
@@ -395,7 +399,10 @@ int sk_sirt_batched(sk_ctx* ctx, const sk_problem* problems, int count, int iter
   if (!ex && plan.nc) {
     const int sizes[4] = {1, 2, 4, 8};
     const double cost[4] = {1.0, 1.39, 1.9, 3.4};
-    plan.bp_images = images_per_item(problems, count, sizes, cost, 4, [](const Geom& G) {
+    // Eight images of 3 or 4 candidates hold a window of 88 to 122 KB, one workgroup per CU: us an
+    // iteration for 1, 2, 4 and 8 images per item, 64 x 512^2, 358 angles: bins of 1 3557, 2821, 2221,
+    // 2173; of 2 2445, 2120, 1723, 1579; of 0.5 5879, 4796, 4255, 5329; of 0.36 9277, 7498, 6097, 7134.
+    plan.bp_images = images_per_item(problems, count, sizes, cost, max_cand <= 2 ? 4 : 3, [](const Geom& G) {
       return (long)((G.N + BP_TW - 1) / BP_TW) * ((G.N + 31) / 32);
     });
   }
