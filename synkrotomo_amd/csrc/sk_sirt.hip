@@ -6,6 +6,9 @@
 // epilogue), and k_bp in BP_SIRT mode writes x += C*B(q) together with the transposed
 // copy of x that the next k_fp reads for flat lines.  A block of iterations is captured
 // once into a hipGraph and replayed.
+#include <cstdio>
+#include <cstdlib>
+
 #include "sk_common.h"
 
 namespace sk {
@@ -105,8 +108,10 @@ int sk_sirt(sk_ctx* ctx, sk_geom* g, int batch, float* d_img, const float* d_sin
   if (rc) return rc;
 
   const int K = iters < 8 ? iters : 8;
-  const int fpv = G.fp_variant >= 0 ? G.fp_variant : c->fp_variant;
-  const int bpv = G.bp_variant >= 0 ? G.bp_variant : c->bp_variant;
+  // the kernels a graph holds: a variant of the geometry's or the context's, or -1, the rules by size
+  // (an option of 0 is a rule, a geometry's 0 a kernel)
+  const int fpv = G.fp_variant >= 0 ? G.fp_variant : (c->fp_variant ? c->fp_variant : -1);
+  const int bpv = G.bp_variant >= 0 ? G.bp_variant : (c->bp_variant ? c->bp_variant : -1);
   Geom::SirtGraph* slot = nullptr;
   for (auto& sg : G.sirt_graphs)
     if (sg.exec && sg.img == d_img && sg.b == d_sino && sg.ws == ws && sg.batch == batch &&
@@ -126,6 +131,8 @@ int sk_sirt(sk_ctx* ctx, sk_geom* g, int batch, float* d_img, const float* d_sin
     hipGraphExec_t ex = nullptr;
     rc = capture(c, &G, K, batch, d_img, imgT, d_sino, q, &ex);
     if (rc) return rc;
+    if (getenv("SYNKRO_VERBOSE"))
+      fprintf(stderr, "sk_sirt: captured %d iterations of %d images, fp variant %d, bp variant %d\n", K, batch, fpv, bpv);
     slot->exec = ex;
     slot->img = d_img;
     slot->b = d_sino;
