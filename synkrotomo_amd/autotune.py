@@ -3,9 +3,11 @@
 ``tuned(geom, batch)`` applies the cached choice for the geometry's shape (image size, angle
 count, bins, bin width, device architecture) and the calls' batch size (rounded up to a power
 of two, at most 64) or runs ``sk_autotune_batch`` on the GPU and stores the result: batches of
-small images fill the chip where one image does not, and favour other kernel shapes.  The cache is a JSON file at $SYNKRO_TUNE_CACHE, default
-~/.cache/synkrotomo_amd/tune.json.  Variants only change tile shapes and rays per lane --
-every variant computes identical results -- so a stale cache can only cost time.
+small images fill the chip where one image does not, and favour other kernel shapes (of the
+backprojector only until several images share a workgroup, where it has one shape).  The cache is
+a JSON file at $SYNKRO_TUNE_CACHE, default ~/.cache/synkrotomo_amd/tune.json.  Variants only change
+tile shapes and rays per lane -- every variant computes identical results -- so a stale cache can
+only cost time.
 """
 from __future__ import annotations
 
@@ -23,7 +25,7 @@ def cache_path() -> str:
 
 
 # Bumped whenever the meaning of the variant numbers changes, so old cache entries are ignored.
-VARIANT_TABLE = 6
+VARIANT_TABLE = 7
 
 
 def batch_bucket(batch: int) -> int:

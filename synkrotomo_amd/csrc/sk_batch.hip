@@ -30,6 +30,7 @@ int launched(Ctx* c, const char* what);
 int ensure_weights(Ctx* c, Geom* g, hipStream_t s);
 FpParams fp_params(const Geom* g, const FpArgs& a);
 BpParams bp_params(const Geom* g, const BpArgs& a, int ppt);
+int bp_images(const Geom* g, int batch);
 
 struct BatchProb {
   FpParams fp;
@@ -564,12 +565,16 @@ int sk_autotune_batch(sk_ctx* ctx, sk_geom* g, int batch, int* fp_variant, int* 
   int rc = (e == hipSuccess) ? SK_OK : hip_fail(c, e, "autotune setup");
   const int saved_fp = G.fp_variant, saved_bp = G.bp_variant;
   int best_fp = 0, best_bp = 0;
+  // Where several images share a workgroup the backprojector has one tile height and no variant: its
+  // variants are timed on the most images that do not.
+  int bp_batch = batch;
+  while (!c->exact && bp_batch > 1 && bp_images(&G, bp_batch) > 1) --bp_batch;
   auto time_it = [&](bool fp, int v, float* ms) -> int {
     if (fp) G.fp_variant = v; else G.bp_variant = v;
     const int reps = 3;
     for (int k = 0; k <= reps; k++) {
       if (k == 1) SK_HIP(c, hipEventRecord(e0, s));
-      int r = fp ? sk_fp(ctx, g, batch, img, sino, stream) : sk_bp(ctx, g, batch, sino, img, stream);
+      int r = fp ? sk_fp(ctx, g, batch, img, sino, stream) : sk_bp(ctx, g, bp_batch, sino, img, stream);
       if (r) return r;
     }
     SK_HIP(c, hipEventRecord(e1, s));
@@ -588,7 +593,7 @@ int sk_autotune_batch(sk_ctx* ctx, sk_geom* g, int batch, int* fp_variant, int* 
   for (int v = 0; v <= 2 && !rc; v++) {
     rc = time_it(false, v, &ms);
     if (!rc && ms < best) { best = ms; best_bp = v; }
-    if (!rc && verbose) fprintf(stderr, "sk_autotune: bp variant %d: %.3f ms / 3\n", v, ms);
+    if (!rc && verbose) fprintf(stderr, "sk_autotune: bp variant %d, %d images: %.3f ms / 3\n", v, bp_batch, ms);
   }
   if (e0) (void)hipEventDestroy(e0);
   if (e1) (void)hipEventDestroy(e1);
