@@ -162,9 +162,12 @@ int sk_sirt_batched(sk_ctx* ctx, const sk_problem* problems, int count, int iter
 int sk_autotune(sk_ctx* ctx, sk_geom* g, int* fp_variant, int* bp_variant, void* stream);
 /* No reference counterpart: sk_autotune timed on calls of `batch` images (1..1024) -- the
  * batch the caller will run, since batches of small images favour other shapes than one
- * image (sk_autotune is batch 1).  Keeps the fastest pair for the geometry. */
+ * image (sk_autotune is batch 1).  Keeps the fastest pair for the geometry; *fp_variant is -1 (no
+ * variant) where A.x from an image in LDS, the context default's kernel for images up to 80 x 80, is
+ * faster than all of them.  The bp variants of batches that run several images per workgroup are
+ * timed on the most images that do not. */
 int sk_autotune_batch(sk_ctx* ctx, sk_geom* g, int batch, int* fp_variant, int* bp_variant, void* stream);
-/* Apply previously tuned variants (-1 = the context default). */
+/* Apply previously tuned variants (-1 = the context's option, whose default is a rule on the sizes). */
 int sk_geom_set_variants(sk_geom* g, int fp_variant, int bp_variant);
 
 /* ---------------------------------------------------------------- learned correction */

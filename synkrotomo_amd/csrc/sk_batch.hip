@@ -584,7 +584,9 @@ int sk_autotune_batch(sk_ctx* ctx, sk_geom* g, int batch, int* fp_variant, int* 
   };
   const bool verbose = getenv("SYNKRO_VERBOSE") != nullptr;
   float best = 1e30f, ms = 0.0f;
-  for (int v = 0; v <= 7 && !rc; v++) {
+  for (int v = -1; v <= 7 && !rc; v++) {
+    G.fp_variant = v;
+    if (v < 0 && !fp_in_lds(c, &G, batch)) continue;  // no variant: a kernel of its own only for small images
     rc = time_it(true, v, &ms);
     if (!rc && ms < best) { best = ms; best_fp = v; }
     if (!rc && verbose) fprintf(stderr, "sk_autotune: fp variant %d: %.3f ms / 3\n", v, ms);
