@@ -4,7 +4,8 @@
 //               block owns a 16 x 16*PPT pixel tile and walks the lines in order, staging
 //               for each block of 32 lines the tile's rho-window of the sinogram in LDS
 //               together with the per-bin intercepts r/cost.
-//   k_bp_images B.r of 2, 4 or 8 images per workgroup on 16 x 32 tiles (unit bins, fast mode).
+//   k_bp_images B.r of 2, 4 or 8 images per workgroup on 16 x 32 tiles (fast mode, 1 to 4 candidates
+//               per pixel; 2 and 8 images with two candidates only).
 //
 // The work item itself lives in sk_kern.h (shared with the persistent kernels).
 #include "sk_kern.h"

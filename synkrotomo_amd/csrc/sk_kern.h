@@ -816,14 +816,15 @@ __device__ __forceinline__ void bp_item(const BpParams& P, int tile_x, int tile_
               for (int m = 0; m < S; ++m) acc[q][m] = fmaf(g, pack_at<S>(ev[q][k], m), acc[q][m]);
             }
         };
+        // One pixel per thread: nothing within a line to overlap its record and window reads with, and
+        // the launches that use it (below 1024 taller tiles) hold few waves, so four lines at a time
+        // (by hand: no unroll pragma takes a loop with a readfirstlane).  us before and after: 64^2,
+        // 100 angles 22 and 17.5; 256^2, 179 angles 37 and 31; 512^2, 804 angles 168 and 150.
+        // Setting a block's lines up, or staging its window, during the block before it gained
+        // nothing more.
         auto run = [&](auto kind, auto slots, int jb, int je) {
           int jj = jb;
-          // One pixel per thread: nothing within a line to overlap its record and window reads with, and
-      // the launches that use it (below 1024 taller tiles) hold few waves, so four lines at a time (by
-      // hand: no unroll pragma takes a loop with a readfirstlane).  us before and after: 64^2, 100
-      // angles 22 and 17.5; 256^2, 179 angles 37 and 31; 512^2, 804 angles 168 and 150.  Setting a
-      // block's lines up, or staging its window, during the block before it gained nothing more.
-      if constexpr (PPT * S == 1) {
+          if constexpr (PPT * S == 1) {
             for (; jj + 4 <= je; jj += 4) {
               line_body(kind, slots, jj);
               line_body(kind, slots, jj + 1);
