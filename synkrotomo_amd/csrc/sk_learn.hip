@@ -354,15 +354,19 @@ __global__ __launch_bounds__(256) void k_conv_out_dgrad(int H, int W, long npix,
 // each, 69 us = 4.7 TB/s (on VALU with one thread per pixel re-reading every neighbour's 32
 // channels: 851 us); 31 us for a gradient that needs no mask.
 template <int CIN, bool MASK>
-__global__ __launch_bounds__(256) void k_conv_in_dgrad(int H, int W, const __bf16* __restrict__ dh,
+__global__ __launch_bounds__(256) void k_conv_in_dgrad(int H, int W, long ntiles,
+                                                       const __bf16* __restrict__ dh,
                                                        const __bf16* __restrict__ hmask,
                                                        const __bf16* __restrict__ w,
                                                        float* __restrict__ dx) {
   __shared__ float U[CO_SLOTS * 9];
   const int tiles_x = (W + CT - 1) / CT, tiles_img = tiles_x * ((H + CT - 1) / CT);
-  const int tile = blockIdx.x % tiles_img;
+  const long block = (long)blockIdx.y * gridDim.x + blockIdx.x;
+  if (block >= ntiles) return;  // uniform
+  const long b = block / tiles_img;
+  const int tile = (int)(block - b * tiles_img);
   const int tx0 = (tile % tiles_x) * CT, ty0 = (tile / tiles_x) * CT;
-  const size_t img = (size_t)(blockIdx.x / tiles_img) * H * W;
+  const size_t img = (size_t)b * H * W;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int m = lane & 15, kq = lane >> 4;
   constexpr int NG = CO_SLOTS / 16, GPW = (NG + 3) / 4;
@@ -900,13 +904,15 @@ static int conv_in_dgrad_go(sk_ctx* ctx, int cin, int B, int H, int W, const voi
   if (rc) return rc;
   if (cin < 1 || cin > 2 || B < 1 || H < 1 || W < 1 || !dh || (MASK && !hmask) || !w || !dx)
     return fail(&ctx->c, SK_EINVAL, "conv_in_dgrad: bad arguments");
-  const dim3 grid((unsigned)((long)((W + CT - 1) / CT) * ((H + CT - 1) / CT) * B));
+  const long ntiles = (long)((W + CT - 1) / CT) * ((H + CT - 1) / CT) * B;
+  const long across = std::min(ntiles, 1L << 22);  // a dimension of a launch holds fewer than 2^32 threads
+  const dim3 grid((unsigned)across, (unsigned)((ntiles + across - 1) / across));
   if (cin == 1)
-    hipLaunchKernelGGL((k_conv_in_dgrad<1, MASK>), grid, dim3(256), 0, (hipStream_t)stream, H, W, (const __bf16*)dh,
-                       (const __bf16*)hmask, (const __bf16*)w, dx);
+    hipLaunchKernelGGL((k_conv_in_dgrad<1, MASK>), grid, dim3(256), 0, (hipStream_t)stream, H, W, ntiles,
+                       (const __bf16*)dh, (const __bf16*)hmask, (const __bf16*)w, dx);
   else
-    hipLaunchKernelGGL((k_conv_in_dgrad<2, MASK>), grid, dim3(256), 0, (hipStream_t)stream, H, W, (const __bf16*)dh,
-                       (const __bf16*)hmask, (const __bf16*)w, dx);
+    hipLaunchKernelGGL((k_conv_in_dgrad<2, MASK>), grid, dim3(256), 0, (hipStream_t)stream, H, W, ntiles,
+                       (const __bf16*)dh, (const __bf16*)hmask, (const __bf16*)w, dx);
   return launched(&ctx->c, "conv_in_dgrad kernel");
 }
 
