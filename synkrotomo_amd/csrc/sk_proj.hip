@@ -284,7 +284,11 @@ __global__ __launch_bounds__(FPS_RAYS) void k_fp_staged(FpParams P) {
 // position, address and fraction, so each adds 3 VALU and its 8 bytes of LDS reads per row and
 // ray; at S = 4 the LDS is busy 65% of the time.  64 images of 512^2, 512 angles: 3.01 ms
 // one image at a time, 2.24 ms for S = 2, 1.75 ms for S = 4.
-constexpr int fpg_waves_per_simd(int s, int cpl) { return s == 1 ? 8 : (s == 4 ? 4 : (cpl == 2 ? 8 : (cpl == 3 ? 6 : 5))); }
+// Waves per SIMD the registers are held to: one image, what its LDS (17, 26 and 35 KB at 2, 3 and 4 chunks)
+// lets run together; at 8 the residual's pointers spilled 16 to 19 scalar registers from 3 chunks on.
+constexpr int fpg_waves_per_simd(int s, int cpl) {
+  return s == 4 ? 4 : (cpl == 2 ? 8 : (cpl == 3 ? 6 : (s == 1 ? 4 : 5)));
+}
 
 template <int MODE, int S, int CPLMAX>
 __global__ __launch_bounds__(FPS_RAYS, fpg_waves_per_simd(S, CPLMAX)) void k_fp_grouped(FpParams P) {
