@@ -44,7 +44,8 @@ enum {
   /* 1: every division in the inner loops is an IEEE division, so results are bitwise
    *    those of the sequential FP32 restatement of the reference (slower).
    * 0 (default): the per-step quotients use the hardware reciprocal (<= 2 ulp per
-   *    length); pixel indices and candidate sets are unchanged. */
+   *    length); pixel indices and candidate sets are unchanged.  B and A^T scale a
+   *    measurement by up to 1.4e3 on the way: magnitudes beyond 1e35 can overflow. */
   SK_OPT_EXACT = 1,
   /* Kernel variant of the projector kernels for geometries that were not tuned (0 = chosen by a
    * rule on the sizes). */
