@@ -388,6 +388,14 @@ __device__ __forceinline__ void fp_item(const FpParams& P, int j, int wb, int bz
           const float bot = inb ? lb * vb : 0.0f;
           const float top = intop ? lt * vt : 0.0f;
           sum[k] = sum[k] + (bot + top);
+          if constexpr (WEIGHTS == W_ADJ) {
+            // At 45 degrees x_bot can lie an ulp below a pixel and x_top round up to its far edge: the
+            // pixel between the two ends' is the one that B gives the row's length to.
+            const int Xm = (Xb + Xt) / 2;
+            if (abs(Xt - Xb) == 2 && (unsigned)(Xm + h) < (unsigned)N)
+              sum[k] = sum[k] + bp_entry<EXACT, DR1>(L, Xm, (float)i, xbot, xtop, r[k], P.ncand, P.rho0, P.drho) *
+                                    row_load(row, Xm + h);
+          }
         }
       }
     }

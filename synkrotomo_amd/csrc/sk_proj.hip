@@ -168,6 +168,9 @@ __global__ __launch_bounds__(256) void k_bpt_rays(FpParams P) {
         return (unsigned)(X + h) < (unsigned)N ? len * v : 0.0f;
       };
       sum = sum + (part(Xb[q], vb[q]) + (Xb[q] == Xt[q] ? 0.0f : part(Xt[q], vt[q])));
+      const int Xm = (Xb[q] + Xt[q]) / 2;  // as fp_item: the pixel between two ends that rounded apart
+      if (abs(Xt[q] - Xb[q]) == 2 && (unsigned)(Xm + h) < (unsigned)N)
+        sum = sum + part(Xm, src[(size_t)(i + q + h) * N + h + Xm]);
     }
   }
   *out = sum;

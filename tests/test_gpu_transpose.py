@@ -107,3 +107,27 @@ def test_transpose_of_small_images(ctx, N, A, first, batch):
     B = sp.csr_matrix((vals.astype(np.float64), c, rp), shape=(N * N, A * R))
     for k in {0, batch // 2, batch - 1}:
         assert rel_l2(got[k].ravel(), B.T @ v[k].ravel().astype(np.float64)) <= 2e-6
+
+
+# Diagonal rays an ulp off the pixels' corners: x_bot just below a pixel, x_top rounded up to its far edge,
+# so the two ends' pixels are not the one the ray crosses.  By the walk of every ray (small images,
+# exact mode), by A.x and its single rays.  Tolerance as in test_gpu_adjoints.py, in exact mode too
+# (the sums' order is not the oracle's).
+@pytest.mark.parametrize("exact_mode", [False, True], ids=["fast", "exact"])
+@pytest.mark.parametrize("N,dr,rz,R", [(20, 0.70710677, -14.849242, 43), (22, 0.35355338, -16.617008, 94),
+                                       (22, 1.4142135, -16.970562, 24), (30, 0.70710677, -22.627417, 64),
+                                       (64, 0.35355338, -48.08326, 272), (64, 0.3, -11.7, 64)])
+def test_transpose_on_diagonal_rays(ctx, N, dr, rz, R, exact_mode):
+    ang = np.array([np.pi / 4, 3 * np.pi / 4, 5 * np.pi / 4, -np.pi / 4], np.float32)
+    v = np.random.default_rng(1).standard_normal((N, N)).astype(np.float32)
+    geo = ctx.geometry(ang, rz, dr, R, N)
+    ctx.exact = exact_mode
+    try:
+        got = geo.bp_transpose(torch.from_numpy(v).cuda()).cpu().numpy().ravel()
+        ones = geo.bp_transpose(torch.ones(N, N, device="cuda")).cpu().numpy().ravel()
+    finally:
+        ctx.exact = False
+    rp, c, vals = oracle.bp_csr(ang, rz, dr, R, N)
+    B = sp.csr_matrix((vals.astype(np.float64), c, rp), shape=(N * N, ang.size * R))
+    assert rel_l2(got, B.T @ v.ravel().astype(np.float64)) <= 2e-6
+    assert rel_l2(ones, B.T @ np.ones(N * N)) <= 2e-6
