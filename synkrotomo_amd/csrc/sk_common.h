@@ -22,9 +22,16 @@ enum : int {
   // step from 1/|slope| (newton_min_slope in sk_geom.hip); set only on geometry tables
   LINE_NEWTON = 8,
   LINE_KEY_BITS = 15,
-  // bits >= LINE_RUN_SHIFT: number of lines from this one to the end of its run of
-  // consecutive table entries with equal LINE_KEY_BITS (>= 1)
-  LINE_RUN_SHIFT = 8
+  // |slope| > 0.99: only so can the ends of a row, x_bot and x_top, round two pixels apart (x is exact
+  // to 0.008 below 2^17).  A then has the row's whole length in x_bot's pixel, B in the one between.
+  LINE_DIAG = 16,
+  // number of lines from this one to the end of its run of consecutive table entries with equal
+  // LINE_KEY_BITS, at least 1, at most LINE_RUN_MAX (more than any block's lines); eight bits
+  // higher the same for runs with equal LINE_DIAG as well: A^T, which weighs those lines apart,
+  // alone pays for the shorter runs (7% of 44 lines on 128^2)
+  LINE_RUN_SHIFT = 8,
+  LINE_DIAG_RUN_SHIFT = 16,
+  LINE_RUN_MAX = 255
 };
 
 // One line in its frame (futhark/sirtlib.fut:39-41): steep angles keep the image frame

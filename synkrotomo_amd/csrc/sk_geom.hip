@@ -187,7 +187,7 @@ static int build_lines(const float* ang, int A, std::vector<Line>& out, int N = 
     L.fs = fact * L.sint;
     L.orig = i;
     L.flags = (is_flat ? LINE_FLAT : 0) | (L.slope >= 0.0f ? LINE_SLOPE_POS : 0) |
-              (fabsf(L.slope) < 1e-3f ? LINE_DEGEN : 0);
+              (fabsf(L.slope) < 1e-3f ? LINE_DEGEN : 0) | (fabsf(L.slope) > 0.99f ? LINE_DIAG : 0);
     if (N > 0 && !(L.flags & LINE_DEGEN) && fabsf(L.slope) >= newton_min_slope(N)) L.flags |= LINE_NEWTON;
     (is_flat ? flat : steep).push_back(L);
   }
@@ -195,9 +195,12 @@ static int build_lines(const float* ang, int A, std::vector<Line>& out, int N = 
   out.insert(out.end(), flat.begin(), flat.end());
   // run lengths (consecutive lines with equal key bits), counted from the back
   for (int j = A - 1; j >= 0; j--) {
-    const bool same = j + 1 < A && (out[j + 1].flags & LINE_KEY_BITS) == (out[j].flags & LINE_KEY_BITS);
-    const int run = same ? (out[j + 1].flags >> LINE_RUN_SHIFT) + 1 : 1;
-    out[j].flags = (out[j].flags & LINE_KEY_BITS) | (run << LINE_RUN_SHIFT);
+    const int f = out[j].flags, next = j + 1 < A ? out[j + 1].flags : 0;
+    auto run = [&](int key, int shift) {
+      const bool same = j + 1 < A && (next & key) == (f & key);
+      return (same ? std::min((next >> shift & LINE_RUN_MAX) + 1, (int)LINE_RUN_MAX) : 1) << shift;
+    };
+    out[j].flags = f | run(LINE_KEY_BITS, LINE_RUN_SHIFT) | run(LINE_KEY_BITS | LINE_DIAG, LINE_DIAG_RUN_SHIFT);
   }
   return (int)steep.size();
 }

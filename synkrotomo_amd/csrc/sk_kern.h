@@ -402,9 +402,8 @@ __device__ __forceinline__ void fp_item(const FpParams& P, int j, int wb, int bz
         }
       }
     };
-    // Only near 45 degrees can a row's two ends round two pixels apart (x is exact to 0.008 below 2^17).
     // Other lines have a loop without that pixel: B^T of one 22^2 image, 7 angles: 10.7 us, 11.4 in one loop.
-    if (WEIGHTS == W_ADJ && fabsf(slope) > 0.99f)
+    if (WEIGHTS == W_ADJ && (L.flags & LINE_DIAG))
       walk(std::bool_constant<WEIGHTS == W_ADJ>{});
     else
       walk(std::false_type{});
@@ -455,7 +454,8 @@ __host__ __device__ inline int bp_window_bins(int ppt, float drho, int ncand) {
 // only: ci, si, cst give the candidate index t = ci*(xmin+0.5) + si*(ymin+0.5) + cst (the
 // reference's ((cost*x + sint*y) - rho0)/drho, x = xmin+0.5-fact*cost, y = ymin+0.5-fact*sint,
 // with the constant terms folded).  t does not depend on the tile, so every tile shape
-// selects the same candidates.
+// selects the same candidates.  W_ADJ on LINE_DIAG lines: cost, sint and, in cst and rs, fact*cost
+// and fact*sint (read from the line table, two such lines were 10% of a 64^2 image's A^T).
 struct alignas(16) BpLineLds {
   int w0;
   float ci, si, cst;
@@ -546,12 +546,13 @@ __device__ __forceinline__ void bp_item(const BpParams& P, int tile_x, int tile_
   constexpr int LB = BP_LB;  // the same for every kernel: a block's tie lines are summed at its end
   static_assert(LB <= 64, "one lane per line of a block");
   // Fast mode: slope sign hoisted per line, lbase folded into the staged value.  Hoisted (NC > 0),
-  // W_ADJ takes the same lengths: on a line that is not degenerate, intersect_fact of a candidate
-  // is the forward projector's length of that ray in that pixel (both are the part of the row's
-  // x-range inside the pixel over the range; neither counts a ray that only touches an edge), so
-  // only the degenerate lines, whose rays can lie on pixel edges, are weighed differently.  Where
-  // it does not run hoisted (NC = 0; DR1 with two candidates: the fast index is not safe) W_ADJ
-  // keeps the reference's index and the forward projector's own lengths.
+  // W_ADJ takes the same lengths: on a line that is neither degenerate nor near a diagonal,
+  // intersect_fact of a candidate is the forward projector's length of that ray in that pixel
+  // (both are the part of the row's x-range inside the pixel over the range; neither counts a ray
+  // that only touches an edge), so only the degenerate lines, whose rays can lie on pixel edges,
+  // and the diagonal ones (LINE_DIAG) are weighed differently.  Where it does not run hoisted (NC = 0; DR1
+  // with two candidates: the fast index is not safe) W_ADJ keeps the reference's index and the
+  // forward projector's own lengths.
   constexpr bool FASTREF = !EXACT && !(WEIGHTS == W_ADJ && (NC == 0 || DR1));
   // The hoisted fast path keeps each line's window in descending bin order, so that the
   // candidate address comes from floor(-t) (one conversion) instead of ceil(t).
@@ -633,8 +634,16 @@ __device__ __forceinline__ void bp_item(const BpParams& P, int tile_x, int tile_
       e.tab = 4u * ((unsigned)(l0 + (int)threadIdx.x) * (unsigned)P.R + (unsigned)e.w0);
       e.flags = L.flags;
       e.rs = (L.flags & LINE_NEWTON) ? 1.0f / fabsf(L.slope) : 0.0f;
+      if constexpr (REV && WEIGHTS == W_ADJ) {
+        if (L.flags & LINE_DIAG) {  // the reference's index
+          e.ci = L.cost;
+          e.si = L.sint;
+          e.cst = L.fc;
+          e.rs = L.fs;
+        }
+      }
       const int eb = ebin[fl ? 1 : 0];
-      const bool exd = REV && eb >= 0 && !(L.flags & LINE_DEGEN);
+      const bool exd = REV && eb >= 0 && !(L.flags & (WEIGHTS == W_ADJ ? LINE_DEGEN | LINE_DIAG : LINE_DEGEN));
       e.dx = exd ? binade_step(L.slope, eb) : 0.0f;
       e.tie = exd && e.dx == 0.0f;
       e.wscale = e.dx > 0.0f ? L.lbase / e.dx : L.lbase;
@@ -744,14 +753,15 @@ __device__ __forceinline__ void bp_item(const BpParams& P, int tile_x, int tile_
       }
       if constexpr (REV) {
         // The table keeps the lines of each part in angle order, so the lines of one slope
-        // sign (degenerate or not) form runs; Line::flags >> LINE_RUN_SHIFT is the number of
-        // lines from a line to the end of its run.  Each run is walked by a loop whose body
+        // sign (degenerate or not) form runs; Line::flags holds the number of lines
+        // from a line to the end of its run.  Each run is walked by a loop whose body
         // has the sign and the degenerate case resolved at compile time (no per-line branch).
         // Kinds: 0: slope >= 0, 1: slope < 0, 2: degenerate; 3, 4: as 0, 1 on LINE_NEWTON
         // lines; 5, 6: as 0, 1 in a tile with one binade (tile_binade), with the exact step.
         // SLOTS (kinds 0, 1, 3, 4 of a flat run whose band has a binade, bp_band_rule): bit q
         // set: slot q takes the exact step as kinds 5, 6 do; the other slots take the kind's
         // own step, times dx (the staged value is lbase/dx).  -1: the kind's step, unscaled.
+        // 7: W_ADJ on LINE_DIAG lines, the forward projector's lengths and the reference's index.
         auto line_body = [&](auto kind, auto slots, int jj) {
           constexpr int KIND = decltype(kind)::value;
           constexpr int SLOTS = decltype(slots)::value;
@@ -771,10 +781,11 @@ __device__ __forceinline__ void bp_item(const BpParams& P, int tile_x, int tile_
           bool ex[PPT];  // the slot takes the exact step (constant once the loops unroll)
 #pragma unroll
           for (int q = 0; q < PPT; ++q) {
-            ex[q] = KIND == 5 || KIND == 6 || (KIND != 2 && SLOTS >= 0 && ((SLOTS >> q) & 1));
+            ex[q] = KIND == 5 || KIND == 6 || (KIND != 2 && KIND != 7 && SLOTS >= 0 && ((SLOTS >> q) & 1));
             // t is within 0.4 bin of the reference's index (|rho0| + N < 2^20 bins for this
             // path), so its ceiling lies in [w0, w0 + W - NC]: no clamp.
-            const float t = part == 0 ? fmaf(lc.si, yh[q], tb) : fmaf(lc.ci, xh[q], tb);
+            float t = part == 0 ? fmaf(lc.si, yh[q], tb) : fmaf(lc.ci, xh[q], tb);
+            if constexpr (KIND == 7) t = (lc.ci * (xh[q] - lc.cst) + lc.si * (yh[q] - lc.rs) - P.rho0) / P.drho;
             const int at = neg_ceil_to_int(t);
             xbase[q] = ym[q] * slope;  // backprojection.fut:55
             // x_top - xmin = x_bot - (xmin - d), resp. xmin + 1 - x_top = (xmin + 1 + d) -
@@ -802,7 +813,7 @@ __device__ __forceinline__ void bp_item(const BpParams& P, int tile_x, int tile_
             for (int k = 0; k < NC; ++k) {
               const float xb = xbase[q] + ei[q][k];
               float g;  // the candidate's weight of its staged value
-              if constexpr (KIND == 2) {
+              if constexpr (KIND == 2 || KIND == 7) {
                 // degenerate line: general form with the m == 0 case, lbase already in e.y
                 g = cand_len<false, WEIGHTS>(xb, slope, 1.0f, xm[q], x1[q], true);
               } else if (ex[q]) {
@@ -875,7 +886,13 @@ __device__ __forceinline__ void bp_item(const BpParams& P, int tile_x, int tile_
         const bool all_slots = part == 0 || fslots == (1 << PPT) - 1;  // uniform
         for (int jr = j_begin; jr < j_end;) {  // uniform: scalar loop over the runs
           const int f = __builtin_amdgcn_readfirstlane(lsh[jr].flags);
-          const int je = min(jr + (f >> LINE_RUN_SHIFT), j_end);
+          constexpr int SHIFT = WEIGHTS == W_ADJ ? LINE_DIAG_RUN_SHIFT : LINE_RUN_SHIFT;
+          const int je = min(jr + (f >> SHIFT & LINE_RUN_MAX), j_end);
+          if (WEIGHTS == W_ADJ && (f & LINE_DIAG)) {
+            for (int jj = jr; jj < je; ++jj) line_body(std::integral_constant<int, WEIGHTS == W_ADJ ? 7 : 2>{}, none{}, jj);
+            jr = je;
+            continue;
+          }
           if (f & LINE_DEGEN)
             run(std::integral_constant<int, 2>{}, none{}, jr, je);
           else if (exact_step && all_slots && (f & LINE_SLOPE_POS))

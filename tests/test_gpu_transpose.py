@@ -131,3 +131,29 @@ def test_transpose_on_diagonal_rays(ctx, N, dr, rz, R, exact_mode):
     B = sp.csr_matrix((vals.astype(np.float64), c, rp), shape=(N * N, ang.size * R))
     assert rel_l2(got, B.T @ v.ravel().astype(np.float64)) <= 2e-6
     assert rel_l2(ones, B.T @ np.ones(N * N)) <= 2e-6
+
+
+# The same rays in A^T: A gives such a row's whole length to the pixel of x_bot, B to the one between, and
+# lines of each kind stand next to them in the table (other slopes, degenerate ones).  One image in
+# the three tile heights, and 2, 4 and 8 at once (66^2 and 80^2 of two candidates).  Tolerance as in
+# test_gpu_adjoints.py.
+@pytest.mark.parametrize("variant,batch", [(0, 1), (1, 1), (2, 1), (-1, 52), (-1, 80), (-1, 280)])
+@pytest.mark.parametrize("N,dr,rz,R", [(20, 1.4142135, -14.142135, 21), (80, 2.828427, -55.154327, 41),
+                                       (80, 0.70710677, -21.92031, 64), (80, 0.35355338, -10.960155, 64),
+                                       (66, 1.0, -30.292893, 63), (40, 0.4, -12.4, 64), (80, 1.25, -39.292893, 65)])
+def test_adjoint_on_diagonal_rays(ctx, N, dr, rz, R, variant, batch):
+    diag = [np.pi / 4, 3 * np.pi / 4, 5 * np.pi / 4, -np.pi / 4]
+    ang = np.array(sorted(diag + [d + e for d in diag for e in (-0.3, -0.005, -0.0005, 0.0005, 0.005, 0.3)] + [0.0, np.pi / 2]),
+                   np.float32)
+    A = ang.size
+    y = np.random.default_rng(2).standard_normal((batch, A, R)).astype(np.float32)
+    geo = ctx.geometry(ang, rz, dr, R, N)
+    geo.set_variants(-1, variant)
+    try:
+        got = geo.bp_adjoint(torch.from_numpy(y).cuda()).cpu().numpy().reshape(batch, -1)
+    finally:
+        geo.set_variants(-1, -1)
+    rp, c, vals = oracle.fp_csr(ang, rz, dr, R, N)
+    At = sp.csr_matrix((vals.astype(np.float64), c, rp), shape=(A * R, N * N)).T
+    for k in {0, batch // 2, batch - 1}:
+        assert rel_l2(got[k], At @ y[k].ravel().astype(np.float64)) <= 2e-6
