@@ -116,6 +116,16 @@ int bp_images(const Geom* g, int batch) {
   return 1;
 }
 
+// A^T by the general kernel: where the candidate index is not safe, and few lines of few pixels, which
+// the hoisted kernel's set-up of a block and its loop per kind of line outweigh.  us hoisted and
+// general, one image: 64^2, 8 lines HA and HB; 512^2, 4 lines 6.0 and 4.2, 12 lines HC and HD; bins of 0.4, 4 lines
+// of 512^2 HE and HF.  Up to 1.4x at 2^18 pixels, even at 2^19 and 8 lines, the other way from 2^20.
+static bool adj_general(const Geom* g, int batch) {
+  const long pixels = (long)batch * g->N * g->N;
+  const int few = g->ncand > 2 ? 5 : (pixels <= 1L << 18 ? 12 : 8);
+  return !g->index_safe || (pixels < 1L << 20 && g->A <= few);
+}
+
 template <bool EXACT, int MODE, int WEIGHTS, int PPT>
 static void bp_go_nc(const Geom* g, const BpArgs& a, hipStream_t s) {
   if constexpr (EXACT) {
@@ -125,7 +135,7 @@ static void bp_go_nc(const Geom* g, const BpArgs& a, hipStream_t s) {
       bp_go<true, MODE, WEIGHTS, 0, false, PPT>(g, a, s);
   } else {
     if constexpr (WEIGHTS == W_ADJ) {
-      if (!g->index_safe) {
+      if (adj_general(g, a.batch)) {
         if (g->bp_two_cand)
           bp_go<false, MODE, W_ADJ, 2, true, 1>(g, a, s);
         else
@@ -185,7 +195,7 @@ int launch_bp(Ctx* c, const Geom* g, BpMode mode, BpWeights w, const BpArgs& a, 
   if (sizeof(float2) * BP_LB * (size_t)bp_window_bins(1, g->drho, g->ncand) > 60 * 1024)
     return fail(c, SK_EINVAL, "backprojection window exceeds LDS (deltarho too small)");
   if (w == W_ADJ && mode != BP_PLAIN) return fail(c, SK_EINVAL, "adjoint weights support plain mode only");
-  const int images = ex || mode == BP_ONES_INV || (w == W_ADJ && !g->index_safe) ? 1 : bp_images(g, a.batch);
+  const int images = ex || mode == BP_ONES_INV || (w == W_ADJ && adj_general(g, a.batch)) ? 1 : bp_images(g, a.batch);
   if (images > 1) {
     if (w == W_ADJ)
       bp_go_images_s<BP_PLAIN, W_ADJ>(images, g, a, s);

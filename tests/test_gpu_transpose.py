@@ -157,3 +157,19 @@ def test_adjoint_on_diagonal_rays(ctx, N, dr, rz, R, variant, batch):
     At = sp.csr_matrix((vals.astype(np.float64), c, rp), shape=(A * R, N * N)).T
     for k in {0, batch // 2, batch - 1}:
         assert rel_l2(got[k], At @ y[k].ravel().astype(np.float64)) <= 2e-6
+
+
+# Few lines of few pixels run A^T's general kernel: both sides of each line of that rule (12 lines up to
+# 2^18 pixels, 8 up to 2^20, 5 of narrow bins).  Tolerance as in test_gpu_adjoints.py.
+@pytest.mark.parametrize("N,batch,A,dr", [(2, 1, 1, 1.0), (64, 64, 12, 1.0), (64, 65, 12, 1.0), (64, 64, 13, 2.0), (64, 65, 8, 2.0),
+                                          (64, 255, 8, 1.0), (64, 256, 8, 1.0), (66, 30, 5, 0.4), (66, 30, 6, 0.4), (64, 256, 5, 0.4)])
+def test_adjoint_of_few_lines(ctx, N, batch, A, dr):
+    ang = ((np.arange(A) + 0.2) * np.pi / A).astype(np.float32)
+    R = int(np.ceil(np.sqrt(2.0) * N / dr))
+    rz = -(R - 1) / 2 * dr + 0.1
+    y = np.random.default_rng(A).standard_normal((batch, A, R)).astype(np.float32)
+    got = ctx.geometry(ang, rz, dr, R, N).bp_adjoint(torch.from_numpy(y).cuda()).cpu().numpy().reshape(batch, -1)
+    rp, c, vals = oracle.fp_csr(ang, rz, dr, R, N)
+    At = sp.csr_matrix((vals.astype(np.float64), c, rp), shape=(A * R, N * N)).T
+    for k in {0, batch // 2, batch - 1}:
+        assert rel_l2(got[k], At @ y[k].ravel().astype(np.float64)) <= 2e-6
