@@ -118,8 +118,9 @@ int bp_images(const Geom* g, int batch) {
 
 // A^T by the general kernel: where the candidate index is not safe, and few lines of few pixels, which
 // the hoisted kernel's set-up of a block and its loop per kind of line outweigh.  us hoisted and
-// general, one image: 64^2, 8 lines HA and HB; 512^2, 4 lines 6.0 and 4.2, 12 lines HC and HD; bins of 0.4, 4 lines
-// of 512^2 HE and HF.  Up to 1.4x at 2^18 pixels, even at 2^19 and 8 lines, the other way from 2^20.
+// general: 256^2, 8 lines 6.1 and 5.3; 512^2, 4 lines 6.0 and 4.5, 12 lines 7.7 and 7.5; bins of
+// 0.4, 4 lines of 512^2 7.1 and 6.4.  From 2^20 pixels the hoisted kernel is the faster one
+// (four 512^2 images, 8 lines 9.7 and 13.5).
 static bool adj_general(const Geom* g, int batch) {
   const long pixels = (long)batch * g->N * g->N;
   const int few = g->ncand > 2 ? 5 : (pixels <= 1L << 18 ? 12 : 8);
