@@ -421,13 +421,24 @@ static long fp_workgroups(const Geom* g, int batch) {
 //   off their bins lie, so with narrow bins from little more than the image's diagonal on (512^2 and 179,
 //   bins of 0.5, R = 5792, four times what is seen: 76, 64, 119; 256^2 and 128, bins of 1, the axis 2000 from
 //   the first one: 27, -, 41).
+// - Few lines: those of a group lie far apart, so its rows are wide and each wave waits for more columns
+//   than its rays meet.  One line: 256^2 14.6 us, 17.6 grouped.  Up to ten lines, from 128 workgroups of
+//   the per-wave kernel: 256^2, 6 angles, 64 images, bins of 2 34, 48; 130^2, 4 angles, 64 images 18, 25.  Bins
+//   below 1, by the farthest bin's pixels per line (centred detectors: 8 pixels of width per line), times of 7
+//   over 0: 256^2, 12 angles, bins of 0.36, 64 images 1.5; 512^2, 16 images, 32 angles 1.2, 64 angles 0.6;
+//   4 images, 179 angles, a detector of six times what is seen 1.9.
+// - Bins below 1 of a geometry without line groups: one line at a time, staged (6), is no faster (1024^2, 48
+//   angles, bins of 0.5, 32 images: 1141 and 1947).
 static int fp_variant_default(const Geom* g, int batch) {
   // the farthest bin from the axis, in image widths (0.71 sees the whole image)
   const double reach = fmax(fabs((double)g->rho0), fabs(g->rho0 + (double)g->R * g->drho)) / g->N;
   const bool narrow = g->drho < 1.0f && fpg_images(g, batch) == 1;
   if (reach > (narrow ? 0.9 : 6.0)) return 0;
-  if (g->N < 128 && fp_workgroups(g, batch) < 512) return 3;
-  return narrow && fp_workgroups(g, batch) < 4096 ? 3 : 7;
+  const long workgroups = fp_workgroups(g, batch);
+  if (g->N < 128 && workgroups < 512) return 3;
+  if (narrow && workgroups < 4096) return 3;
+  if (g->A == 1 || (g->A <= 10 && workgroups >= 128) || (g->drho < 1.0f && (g->N * reach > 6.0 * g->A || !g->d_fpg))) return 0;
+  return 7;
 }
 
 // Whether A.x with no transposed copy at hand (FpArgs: imgT = img) takes k_fp_lds, and needs none, the
